@@ -512,7 +512,7 @@ int fides_stage_modup(fides_context* ctx, int32_t level, const uint64_t* x, uint
  * The library loads its measured table (pyfideslib_amd/tune_gfx950.txt, or
  * FIDES_TUNE_FILE; empty = fixed rules) when the first context is created.
  * kind: FIDES_TUNE_NTT_FWD / _NTT_INV (size = limbs per launch; cfg = column
- * tile width, log2 values per column thread, row tile height, grid cap) or
+ * tile width, log2 values per column thread, row tile height, unused) or
  * FIDES_TUNE_MODUP / _MODDOWN (size = conversions per launch; cfg[0] =
  * target groups; FIDES_TUNE_MODUP cfg[1] = 1 selects the int8 matrix-core
  * conversion, built when the digit has at most 16 limbs).  fides_tune_force pins a kind's configuration for every

@@ -288,7 +288,8 @@ void Context::build_tables(const std::vector<uint64_t>& roots) {
         const uint64_t p = q[i];
         int n = 0;
         while ((p >> n) != 0) ++n;
-        primes[i] = PrimeInfo{p, (uint64_t)(((u128)1 << (n + 63)) / p), (uint32_t)n, 0u, 2 * p};
+        primes[i] = PrimeInfo{p, (uint64_t)(((u128)1 << (n + 63)) / p), (uint32_t)n, n <= FP_BITS ? 1u : 0u,
+                              2 * p, (double)p, 1.0 / (double)p};
         const uint64_t psi = roots[i], psi_inv = h_invmod(psi, p);
         uint64_t pw = 1, pwi = 1;
         for (int k = 0; k < N; ++k) {
@@ -431,7 +432,9 @@ void Context::build_tables(const std::vector<uint64_t>& roots) {
     const size_t o_qli = place(qlinv.size() * sizeof(ShoupConst));
     const size_t o_qlm = place(qlmodq.size() * 8);
     const size_t o_mfu = place(modup_mfma.size() * 8);
-    std::vector<char> host(off, 0);
+    const size_t staged = off;  // what follows is filled on the device
+    const size_t o_dwf = place((size_t)np * N * 8), o_dwi = place((size_t)np * N * 8);
+    std::vector<char> host(staged, 0);
     auto put = [&](size_t o, const void* src, size_t bytes) { if (bytes) std::memcpy(host.data() + o, src, bytes); };
     put(o_primes, primes.data(), primes.size() * sizeof(PrimeInfo));
     put(o_twf, tw_fwd.data(), tw_fwd.size() * sizeof(ShoupConst));
@@ -447,12 +450,18 @@ void Context::build_tables(const std::vector<uint64_t>& roots) {
     put(o_qlm, qlmodq.data(), qlmodq.size() * 8);
     put(o_mfu, modup_mfma.data(), modup_mfma.size() * 8);
     hip_check(hipMalloc(&blob_, off), "hipMalloc(tables)");
-    hip_check(hipMemcpy(blob_, host.data(), off, hipMemcpyHostToDevice), "hipMemcpy(tables)");
+    hip_check(hipMemcpy(blob_, host.data(), staged, hipMemcpyHostToDevice), "hipMemcpy(tables)");
     char* b = (char*)blob_;
     T.logN = logN; T.N = N; T.L = L; T.K = K; T.dnum = dnum; T.alpha = alpha; T.np = np;
     T.primes = (const PrimeInfo*)(b + o_primes);
     T.tw_fwd = (const ShoupConst*)(b + o_twf);
     T.tw_inv = (const ShoupConst*)(b + o_twi);
+    T.fpmask[0] = T.fpmask[1] = 0;
+    for (int i = 0; i < np; ++i) T.fpmask[i >> 6] |= (uint64_t)primes[i].fp << (i & 63);
+    T.twd_fwd = (const double*)(b + o_dwf);
+    T.twd_inv = (const double*)(b + o_dwi);
+    hip_check(launch_fp_twiddles(T, T.tw_fwd, (double*)(b + o_dwf), stream), "FP64 twiddles");
+    hip_check(launch_fp_twiddles(T, T.tw_inv, (double*)(b + o_dwi), stream), "FP64 twiddles");
     T.iscale_plain = (const ShoupConst*)(b + o_isp);
     T.iscale_modup = (const ShoupConst*)(b + o_ism);
     T.iscale_moddown = (const ShoupConst*)(b + o_isd);

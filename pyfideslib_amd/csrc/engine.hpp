@@ -19,9 +19,12 @@ namespace fides {
 // every kernel by value.
 struct DevTables {
     int logN, N, L, K, dnum, alpha, np;
+    uint64_t fpmask[2];                // bit i: prime i is transformed in FP64 (PrimeInfo::fp); np <= 96
     const PrimeInfo* primes;           // [np]
     const ShoupConst* tw_fwd;          // [np][N]  psi^brev(k) with Shoup companion
     const ShoupConst* tw_inv;          // [np][N]  psi^-brev(k)
+    const double* twd_fwd;             // [np][N]  the same, centered in (-p/2, p/2), for the FP64 transforms
+    const double* twd_inv;             // [np][N]  (entries of the primes with fp set)
     const ShoupConst* iscale_plain;    // [np][2]  (N^-1, psi_inv_rev[1] N^-1)
     const ShoupConst* iscale_modup;    // [L+1 level][L+1 pos][2]  N^-1 * PartQlHatInvModq
     const ShoupConst* iscale_moddown;  // [K][2]   N^-1 * PHatInvModp
@@ -111,6 +114,21 @@ __device__ __forceinline__ J get_job(const JobList<J, CAP>& L, int i) {
 #pragma unroll
         for (int k = 0; k < NW; ++k) u.w[k] = p[i * NW + k];
     }
+    return u.j;
+}
+
+// Entry i of an inline list: scalar loads at an offset known at launch.
+template <class J, int CAP>
+__device__ __forceinline__ J get_inline(const JobList<J, CAP>& L, int i) {
+    constexpr int NW = sizeof(J) / 4;
+    union Words {
+        J j;
+        uint32_t w[NW];
+    } u;
+    const __attribute__((address_space(4))) uint32_t* p =
+        (const __attribute__((address_space(4))) uint32_t*)(&L.inl[0]) + i * NW;
+#pragma unroll
+    for (int k = 0; k < NW; ++k) u.w[k] = p[k];
     return u.j;
 }
 
@@ -287,7 +305,7 @@ struct LinCombJob {
 // on the device (pyfideslib_amd/tune.py writes it, tune.hip loads it once per
 // process), falling back to the launchers' fixed rules when no entry covers
 // the size.  NTT entries: {column tile width, log2 values per column thread,
-// row tile height, grid cap (0 = one block per tile)} by limb count;
+// row tile height, unused (once a grid cap)} by limb count;
 // conversion entries: {target groups} by conversions per launch.
 enum TuneKind { TUNE_NTT_FWD = 0, TUNE_NTT_INV = 1, TUNE_MODUP = 2, TUNE_MODDOWN = 3, TUNE_KINDS = 4 };
 constexpr int TUNE_NV = 4;
@@ -309,6 +327,8 @@ int conv_rule_tg(int base_blocks, int max_targets);
 hipError_t launch_ntt_fwd(const DevTables& T, const NttJobs& jobs, int total_limbs, int load_mode, int store_mode,
                           hipStream_t stream);
 hipError_t launch_ntt_inv(const DevTables& T, const NttJobs& jobs, int total_limbs, hipStream_t stream);
+// Fills out[np][N] (T.twd_fwd or T.twd_inv) from the integer table tw.
+hipError_t launch_fp_twiddles(const DevTables& T, const ShoupConst* tw, double* out, hipStream_t stream);
 hipError_t launch_tensor(const DevTables& T, const TensorJobs& jobs, int max_nl, hipStream_t stream);
 hipError_t launch_modup_conv(const DevTables& T, const ModUpJobs& jobs, int max_nd, hipStream_t stream);
 // shared: all jobs use the same ext / own / level (rotations of one hoisted set)

@@ -3,7 +3,10 @@
 // CDNA4 has no 64x64-bit integer multiply; the compiler lowers the pieces
 // below to v_mul_hi_u32 / v_mul_lo_u32 / v_mad_u64_u32.  Every routine returns
 // the exact residue (or an exact residue plus a stated multiple of p when
-// named *_lazy); no floating point enters the ring.
+// named *_lazy).  Moduli below 2^50 have a second, equally exact form on
+// the FP64 units (fp_mul): every value is an integer below 2^53 in magnitude,
+// every product the exact pair (rounded product, fma remainder), so rounding
+// only ever picks the multiple of p that is taken off, never a residue's digit.
 //
 // Reference counterparts: FIDESlib src/ModMult.cuh:46-74 (Barrett),
 // :96-102 (Shoup), :288-313 (128-bit reduce), src/AddSub.cuh:37-50.
@@ -18,9 +21,14 @@ struct PrimeInfo {
     uint64_t p;      // modulus, < 2^60
     uint64_t mu;     // floor(2^(n+63) / p), n = bit length of p
     uint32_t nbits;  // n
-    uint32_t pad;
+    uint32_t fp;     // 1: p < 2^FP_BITS, the transforms run in FP64 (FpArith)
     uint64_t p2;     // 2p
+    double pd, pinv; // p and 1/p, rounded to nearest
 };
+
+// Largest modulus of the exact FP64 transforms: every intermediate is an
+// integer of magnitude below 8p <= 2^53.
+constexpr int FP_BITS = 50;
 
 // Pair (w, floor(w * 2^64 / p)) for Shoup multiplication by the constant w.
 struct ShoupConst {
@@ -86,6 +94,38 @@ __device__ __forceinline__ uint64_t submod(uint64_t a, uint64_t b, uint64_t p) {
     return a >= b ? a - b : a + p - b;
 }
 
+// ---- exact FP64 residues (p < 2^50) ----
+// x w mod p as a signed integer: x w = h + l exactly, q is within 1/2 + 3 2^-53
+// |x w| / p of x w / p, and h - q p is an integer below 2^53, so the fma and
+// the sum are exact.  With |x| <= B p (B <= 8) and |w| <= p / 2 the result is at
+// most (1/2 + 3 B / 16) p in magnitude; |w| < p doubles the second term.  6
+// instructions at the rate of one 32-bit multiply each (a Shoup product: 10
+// multiplies and about 20 adds, carries and moves).
+__device__ __forceinline__ double fp_mul(double x, double w, double p, double pinv) {
+    const double h = x * w;
+    const double l = __builtin_fma(x, w, -h);
+    const double q = __builtin_rint(h * pinv);
+    return __builtin_fma(-q, p, h) + l;
+}
+// x mod p, centered: |result| <= p / 2 + 1 for |x| <= 8p
+__device__ __forceinline__ double fp_reduce(double x, double p, double pinv) {
+    return __builtin_fma(-__builtin_rint(x * pinv), p, x);
+}
+// an integer below 2^52 as a double, and a non-negative one back
+__device__ __forceinline__ double fp_from(uint64_t x) {
+    return __longlong_as_double((long long)(x | 0x4330000000000000ull)) - 0x1p52;
+}
+__device__ __forceinline__ uint64_t fp_to(double x) {
+    return (uint64_t)__double_as_longlong(x + 0x1p52) & 0x000fffffffffffffull;
+}
+// the residue in [0, p) of |x| <= 8p
+__device__ __forceinline__ uint64_t fp_canon(double x, double p, double pinv) {
+    const double r = fp_reduce(x, p, pinv);
+    return fp_to(r < 0 ? r + p : r);
+}
+
 __device__ __forceinline__ uint32_t brev_bits(uint32_t x, int bits) { return __brev(x) >> (32 - bits); }
+// the same for bits >= 0
+__device__ __forceinline__ uint32_t brev_low(uint32_t x, int bits) { return bits ? brev_bits(x, bits) : 0u; }
 
 }  // namespace fides

@@ -13,15 +13,17 @@
 // thread keeps 4 values in registers and runs two radix-2 stages on them
 // between LDS exchanges.  Short per-wave instruction streams and many waves
 // matter more than register blocking here: a pass is latency-bound (a tile's
-// load -> phases -> store chain), not VALU-bound.
+// load -> phases -> store chain), not VALU-bound.  A ring
+// of 2^14 would fit one block's LDS, but one CU alone needs 9 us for its
+// butterflies (29 us measured, against 10 us for two launches over many CUs).
 //
-// Twiddles psi^brev(k) come from the bit-reversed table with their Shoup
-// companions, so each butterfly costs one Shoup product.  Column-pass
+// Twiddles psi^brev(k) come from the bit-reversed tables: centered doubles for
+// the primes below 2^50, whose butterflies run on the FP64 units, 64-bit words
+// with their Shoup companions for the others (ntt_core.hpp).  Column-pass
 // twiddles (the first N1 table entries, shared by all columns) are staged in
 // LDS; row-pass twiddles (distinct per row) are prefetched into registers
-// before the data load so their latency overlaps it.  Butterflies are
-// Harvey-lazy: forward values live in [0, 4p) and inverse values in [0, 2p)
-// between stages, reduced once at the final store.
+// before the data load so their latency overlaps it.  Values
+// stay lazily reduced between stages and are reduced once at the final store.
 //
 // Fusions (FIDESlib src/NTTfusions.cuh:218-262):
 //   LOAD_SWITCH   (forward, pass 1): read the q_l coefficient limb and lift it
@@ -38,530 +40,240 @@
 //   inverse pass 2 folds N^-1 (times an optional per-limb base-conversion
 //   factor) into its last stage.
 #include <cstdlib>
-#include <type_traits>
 
-#include "engine.hpp"
+#include "ntt_core.hpp"
 
 namespace fides {
 
-// log2 of the values per thread: 2, or 3 when a 16-wide column tile of
-// 4-value threads would exceed 1024 threads (logN = 17).
-template <int LOGN>
-constexpr int ntt_lr() { return ((1 << ((LOGN + 1) / 2)) / 4) * 16 > 1024 ? 3 : 2; }
-
-// W: tile width (columns or rows per block); LRC: log2 of the values per thread
-// in the column pass (2, or 3 for radix-8 phases); the row pass always uses
-// ntt_lr (its twiddles are register-prefetched, which needs short phases).
-template <int LOGN, int W, int LRC = ntt_lr<LOGN>()>
-struct NttGeom {
+// Column pass: CC columns of N1 rows per block, TC threads per column, 2^LRC
+// values per thread (2, or 3 for radix-8 phases; logN = 17 only 3, as 16
+// columns of 4-value threads would exceed 1024 threads).
+template <int LOGN, int W, int LRC>
+struct ColGeom {
     static constexpr int K1 = (LOGN + 1) / 2, K2 = LOGN / 2;
     static constexpr int N1 = 1 << K1, N2 = 1 << K2, N = 1 << LOGN;
-    static constexpr int LR = ntt_lr<LOGN>(), R = 1 << LR;
-    static constexpr int LRC_ = LRC, RC = 1 << LRC;
-    // column pass: CC columns of N1 rows per block, TC threads per column
+    static constexpr int RC = 1 << LRC;
     static constexpr int TC = N1 / RC;
     static constexpr int CC = N2 < W ? N2 : W;
     static constexpr int NTC = TC * CC;
     static constexpr int SC = N1 + N1 / 16 + 1;
-    // row pass: RR rows of N2 elements per block, TR threads per row
-    static constexpr int TR = N2 / R;
-    static constexpr int RR = N1 < W ? N1 : W;
-    static constexpr int NTR = TR * RR;
-    static constexpr int SR = N2 + N2 / 16 + 1;
-    // twiddle slots per thread in the row pass: K2 stages x R/2 butterflies
-    static constexpr int NS = K2 * (R / 2);
+    static constexpr int TPL = N2 / CC;                  // tiles per limb
+    static constexpr int NTW = (N1 + NTC - 1) / NTC;     // column twiddles a thread stages
 };
+template <int LOGN>
+constexpr int min_lrc() { return ((1 << ((LOGN + 1) / 2)) / 4) * 16 > 1024 ? 3 : 2; }
+template <int LOGN, int W>
+using Rows = RowGeom<(LOGN + 1) / 2, LOGN / 2, 2, W>;
 
-__device__ __forceinline__ int find_ntt_job(const NttJobs& L, int limb) {
-    int j = 0;
+// The first N1 twiddles, shared by all columns: loaded with the tile, written
+// to LDS after it (so neither waits for the other).
+template <class G, class W>
+__device__ __forceinline__ void stage_load(const W* tab, W* r) {
 #pragma unroll
-    for (int i = 1; i < NTT_INLINE; ++i)
-        if (i < L.n && limb >= L.inl[i].first) j = i;
-    return j;
+    for (int i = 0; i < G::NTW; ++i) r[i] = tab[(threadIdx.x + i * G::NTC) & (G::N1 - 1)];
 }
-
-__device__ __forceinline__ NttJob load_ntt_job(const NttJobs& L, int limb, int& pos) {
-    limb = __builtin_amdgcn_readfirstlane(limb);
-    const int ji = L.dev ? ((const __attribute__((address_space(1))) int*)L.limbmap)[limb] : find_ntt_job(L, limb);
-    const NttJob J = get_job(L, ji);
-    const int a = limb - J.first;
-    pos = a < J.skip_lo ? a : a + (J.skip_hi - J.skip_lo);
-    return J;
-}
-
-__device__ __forceinline__ uint32_t lds_off(uint32_t e) { return e + (e >> 4); }
-
-// [0, 4p) -> [0, p)
-__device__ __forceinline__ uint64_t reduce4p(uint64_t x, uint64_t p) {
-    x = x >= 2 * p ? x - 2 * p : x;
-    return x >= p ? x - p : x;
-}
-// [0, 2p) -> [0, p)
-__device__ __forceinline__ uint64_t reduce2p(uint64_t x, uint64_t p) { return x >= p ? x - p : x; }
-
-// Element index (within a 2^K sub-transform) of register j of thread t in a
-// phase over bits [LO, LO+NB); the LR-NB spare register bits and the thread
-// bits fill the remaining positions from the bottom up.
-template <int LR, int LO, int NB>
-__device__ __forceinline__ uint32_t elem(uint32_t t, uint32_t j) {
-    constexpr uint32_t EX = LR - NB;
-    const uint32_t jlo = j & ((1u << NB) - 1);
-    const uint32_t other = (t << EX) | (j >> NB);
-    return (other & ((1u << LO) - 1)) | (jlo << LO) | ((other >> LO) << (LO + NB));
-}
-
-// Index of butterfly (j, j | 1<<bb) among the R/2 butterflies of a stage.
-__device__ __forceinline__ constexpr int bfly(int j, int bb) { return ((j >> (bb + 1)) << bb) | (j & ((1 << bb) - 1)); }
-
-// Twiddle slot of a butterfly: phases visit the K bits in a fixed order (top
-// down for the forward transform, bottom up for the inverse); `done` bits
-// precede the phase, s is the stage's rank inside the phase.
-template <int LR>
-__device__ __forceinline__ constexpr int slot(int done, int s, int j, int bb) {
-    return (done + s) * (1 << (LR - 1)) + bfly(j, bb);
-}
-
-// ---- LDS exchange between phases ----
-template <int LR, int LO, int NB>
-__device__ __forceinline__ void lds_get(const uint64_t* sub, uint32_t t, uint64_t* v) {
+template <class G, class W>
+__device__ __forceinline__ void stage_put(W* twl, const W* r) {
 #pragma unroll
-    for (int j = 0; j < (1 << LR); ++j) v[j] = sub[lds_off(elem<LR, LO, NB>(t, j))];
+    for (int i = 0; i < G::NTW; ++i) twl[(threadIdx.x + i * G::NTC) & (G::N1 - 1)] = r[i];
 }
-template <int LR, int LO, int NB>
-__device__ __forceinline__ void lds_put(uint64_t* sub, uint32_t t, const uint64_t* v) {
-#pragma unroll
-    for (int j = 0; j < (1 << LR); ++j) sub[lds_off(elem<LR, LO, NB>(t, j))] = v[j];
-}
-
-// Phase boundaries of a K-bit sub-transform with up to LR bits per phase.
-// Forward phases run from the top bit down: the first covers bits
-// [K - NB, K), the last [0, fwd_last_nb).  Inverse phases run from bit 0 up:
-// the first covers [0, NB), the last [inv_last_lo, K).
-template <int LR, int K>
-constexpr int first_nb() { return K < LR ? K : LR; }
-template <int LR, int K>
-constexpr int fwd_last_nb() { return K % LR == 0 ? LR : K % LR; }
-template <int LR, int K>
-constexpr int inv_last_lo() { return LR * ((K - 1) / LR); }
-
-// ---- forward (Cooley-Tukey), bits processed from the top down ----
-template <int LR, int K, int LO, int NB, class TW>
-__device__ __forceinline__ void fwd_bfly(uint64_t* v, uint32_t t, const TW& tw, uint64_t p) {
-    constexpr int R = 1 << LR;
-#pragma unroll
-    for (int bb = NB - 1; bb >= 0; --bb) {
-#pragma unroll
-        for (int j = 0; j < R; ++j) {
-            if (j & (1 << bb)) continue;
-            const int j2 = j | (1 << bb);
-            // Harvey: inputs in [0, 4p), outputs in [0, 4p)
-            const ShoupConst w = tw(slot<LR>(K - LO - NB, NB - 1 - bb, j, bb), LO + bb, elem<LR, LO, NB>(t, j));
-            uint64_t U = v[j];
-            U = U >= 2 * p ? U - 2 * p : U;
-            const uint64_t V = mul_shoup_lazy(v[j2], w.w, w.wp, p);
-            v[j] = U + V;
-            v[j2] = U - V + 2 * p;
-        }
-    }
-}
-
-// Forward phases from bit HI down to 0.  On entry v holds the elements of the
-// phase that starts at HI (the caller loads them straight from global memory
-// for the first phase); phases exchange through LDS; on exit v holds the
-// elements of the last phase (bits [0, fwd_last_nb)), which the caller stores
-// straight to global memory.  One barrier per exchange: a thread writes back
-// exactly the elements it read, so reads and writes of one phase never race.
-// hook(integral_constant<HI>) runs at the start of each phase (the row pass
-// issues later phases' twiddle loads there).
-struct NoHook {
-    template <class X>
-    __device__ __forceinline__ void operator()(X) const {}
-};
-template <int LR, int K, int HI, class TW, class HOOK = NoHook>
-__device__ __forceinline__ void fwd_run(uint64_t* sub, uint64_t* v, uint32_t t, const TW& tw, uint64_t p,
-                                        const HOOK& hook = HOOK{}) {
-    constexpr int NB = HI < LR ? HI : LR;
-    constexpr int LO = HI - NB;
-    hook(std::integral_constant<int, HI>{});
-    fwd_bfly<LR, K, LO, NB>(v, t, tw, p);
-    if constexpr (LO > 0) {
-        constexpr int NB2 = LO < LR ? LO : LR;
-        lds_put<LR, LO, NB>(sub, t, v);
-        __syncthreads();
-        lds_get<LR, LO - NB2, NB2>(sub, t, v);
-        fwd_run<LR, K, LO>(sub, v, t, tw, p, hook);
-    }
-}
-
-// Prefetch of the forward twiddles into twr[] in slot order; IDX(b, e) gives
-// the table index of the twiddle of stage bit b at lower element e.
-// The twiddles of the one phase that starts at bit HI (none when HI <= 0).
-template <int LR, int K, int HI, class IDX>
-__device__ __forceinline__ void fwd_prefetch(ShoupConst* twr, const ShoupConst* tab, uint32_t t, const IDX& idx) {
-    if constexpr (HI > 0) {
-        constexpr int NB = HI < LR ? HI : LR;
-        constexpr int LO = HI - NB;
-#pragma unroll
-        for (int bb = NB - 1; bb >= 0; --bb)
-#pragma unroll
-            for (int j = 0; j < (1 << LR); ++j)
-                if (!(j & (1 << bb))) twr[slot<LR>(K - HI, NB - 1 - bb, j, bb)] = tab[idx(LO + bb, elem<LR, LO, NB>(t, j))];
-    }
-}
-
-// ---- inverse (Gentleman-Sande), bits processed from the bottom up ----
-// When SCALE, the stage on bit K-1 multiplies both outputs by the limb scale s
-// (sum by s, difference by w*s).
-template <int LR, int K, int LO, int NB, bool SCALE, class TW>
-__device__ __forceinline__ void inv_bfly(uint64_t* v, uint32_t t, const TW& tw, uint64_t p, ShoupConst s,
-                                         ShoupConst ws) {
-    constexpr int R = 1 << LR;
-#pragma unroll
-    for (int bb = 0; bb < NB; ++bb) {
-#pragma unroll
-        for (int j = 0; j < R; ++j) {
-            if (j & (1 << bb)) continue;
-            const int j2 = j | (1 << bb);
-            // Harvey: inputs in [0, 2p), outputs in [0, 2p)
-            const uint64_t U = v[j], V = v[j2];
-            if (SCALE && LO + bb == K - 1) {
-                v[j] = mul_shoup_lazy(U + V, s.w, s.wp, p);
-                v[j2] = mul_shoup_lazy(U - V + 2 * p, ws.w, ws.wp, p);
-            } else {
-                const ShoupConst w = tw(slot<LR>(LO, bb, j, bb), LO + bb, elem<LR, LO, NB>(t, j));
-                const uint64_t X = U + V;
-                v[j] = X >= 2 * p ? X - 2 * p : X;
-                v[j2] = mul_shoup_lazy(U - V + 2 * p, w.w, w.wp, p);
-            }
-        }
-    }
-}
-
-// Inverse phases from bit LO up to K, register/LDS discipline as fwd_run: v
-// enters with the elements of the phase starting at LO and leaves with those
-// of the last phase (bits [inv_last_lo, K)).
-template <int LR, int K, int LO, bool SCALE, class TW, class HOOK = NoHook>
-__device__ __forceinline__ void inv_run(uint64_t* sub, uint64_t* v, uint32_t t, const TW& tw, uint64_t p,
-                                        ShoupConst s, ShoupConst ws, const HOOK& hook = HOOK{}) {
-    constexpr int NB = (K - LO) < LR ? (K - LO) : LR;
-    hook(std::integral_constant<int, LO>{});
-    inv_bfly<LR, K, LO, NB, SCALE>(v, t, tw, p, s, ws);
-    if constexpr (LO + NB < K) {
-        constexpr int LO2 = LO + NB;
-        constexpr int NB2 = (K - LO2) < LR ? (K - LO2) : LR;
-        lds_put<LR, LO, NB>(sub, t, v);
-        __syncthreads();
-        lds_get<LR, LO2, NB2>(sub, t, v);
-        inv_run<LR, K, LO2, SCALE>(sub, v, t, tw, p, s, ws, hook);
-    }
-}
-
-// The twiddles of the one phase that starts at bit LO (none when LO >= K).
-template <int LR, int K, int LO, class IDX>
-__device__ __forceinline__ void inv_prefetch(ShoupConst* twr, const ShoupConst* tab, uint32_t t, const IDX& idx) {
-    if constexpr (LO < K) {
-        constexpr int NB = (K - LO) < LR ? (K - LO) : LR;
-#pragma unroll
-        for (int bb = 0; bb < NB; ++bb)
-#pragma unroll
-            for (int j = 0; j < (1 << LR); ++j)
-                if (!(j & (1 << bb))) twr[slot<LR>(LO, bb, j, bb)] = tab[idx(LO + bb, elem<LR, LO, NB>(t, j))];
-    }
-}
-
-// ------------------------------------------------------------ kernels ----
-// Thread layout: in the column pass thread (cc, t) owns column c0 + cc and the
-// rows elem(t, j) of the current phase; in the row pass thread (rr, t) owns
-// row r0 + rr.  The first phase reads its elements straight from global
-// memory and the last phase writes straight back (no LDS staging at either
-// end): three LDS exchanges per 8-stage pass.
 
 // Forward pass 1: column sub-transforms (global stages 0..K1-1).
 template <int LOGN, int W, int LRC, int LOAD>
-__global__ void __launch_bounds__((NttGeom<LOGN, W, LRC>::NTC)) k_ntt_fwd_cols(DevTables T, NttJobs L, int limbs) {
-    using G = NttGeom<LOGN, W, LRC>;
+__global__ void __launch_bounds__((ColGeom<LOGN, W, LRC>::NTC)) k_ntt_fwd_cols(DevTables T, NttJobs L, NttGrid g) {
+    using G = ColGeom<LOGN, W, LRC>;
     constexpr int R = G::RC, NB1 = first_nb<LRC, G::K1>(), LO1 = G::K1 - NB1, NBL = fwd_last_nb<LRC, G::K1>();
     __shared__ uint64_t lds[G::CC * G::SC];
-    __shared__ ShoupConst twl[G::N1];
-    constexpr int TPL = G::N2 / G::CC;  // tiles per limb
-    // grid-stride loop over (limb, tile); a launch with one block per tile
-    // runs one iteration per block
-    for (int tile = blockIdx.x; tile < TPL * limbs; tile += gridDim.x) {
-        const int limb_ = tile / TPL, tx_ = tile % TPL;
-        if (tile != (int)blockIdx.x) __syncthreads();  // LDS reuse across tiles
-        int pos;
-        const NttJob J = load_ntt_job(L, limb_, pos);
-        const int pid = pos_pid(pos, J.nq, J.q0, T.L + 1);
-        const PrimeInfo P = cld(T.primes + pid);
-        const int c0 = tx_ * G::CC;
-        const int tid = threadIdx.x;
-        const int cc = tid % G::CC, t = tid / G::CC;
-
-        {
-            const ShoupConst* tw = T.tw_fwd + (size_t)pid * G::N;
-            for (int i = tid; i < G::N1; i += G::NTC) twl[i] = tw[i];
-        }
-        uint64_t v[R];
+    __shared__ ShoupConst twlds[G::N1];
+    const uint32_t item = xcd_item(g.chunk);
+    NttJob J;
+    int pos;
+    if (!block_job(L, g, item / G::TPL, J, pos)) return;
+    const int pid = pos_pid(pos, J.nq, J.q0, T.L + 1);
+    const int cc = threadIdx.x % G::CC, t = threadIdx.x / G::CC;
+    const uint32_t col = (item % G::TPL) * G::CC + cc;
+    uint64_t x[R];
+    {
+        const gu64* src = gp(J.src) + (LOAD == LOAD_SWITCH ? (size_t)0 : (size_t)pos * G::N);
+#pragma unroll
+        for (int j = 0; j < R; ++j) x[j] = src[col + elem<LRC, LO1, NB1>(t, j) * G::N2];
+    }
+    const PrimeInfo P = cld(T.primes + pid);
+    with_arith(T, pid, P, [&](const auto& ar) {
+        using A = std::decay_t<decltype(ar)>;
+        using V = typename A::V;
+        typename A::W tw[G::NTW];
+        auto* twl = reinterpret_cast<typename A::W*>(twlds);
+        stage_load<G>(A::fwd(T) + (size_t)pid * G::N, tw);
+        V v[R];
         if constexpr (LOAD == LOAD_SWITCH) {
-            const uint64_t ql = cld(T.primes + J.level).p, half = ql >> 1;
-            const uint64_t qlmod = cld(T.qlmodq + (size_t)J.level * (T.L + 1) + pid);
-            const gu64* src = gp(J.src) + c0 + cc;
+            const SwitchLift lift(T, J.level, pid);
 #pragma unroll
-            for (int j = 0; j < R; ++j) {
-                const uint64_t x = src[(size_t)elem<LRC, LO1, NB1>(t, j) * G::N2];
-                uint64_t m = reduce64(x, P);
-                if (x > half) m = submod(m, qlmod, P.p);
-                v[j] = m;
-            }
+            for (int j = 0; j < R; ++j) v[j] = ar.from(lift(x[j], P));
         } else {
-            const gu64* src = gp(J.src) + (size_t)pos * G::N + c0 + cc;
 #pragma unroll
-            for (int j = 0; j < R; ++j) v[j] = src[(size_t)elem<LRC, LO1, NB1>(t, j) * G::N2];
+            for (int j = 0; j < R; ++j) v[j] = ar.from(x[j]);
         }
+        stage_put<G>(twl, tw);
         __syncthreads();
         auto twf = [&](int, int b, uint32_t e) { return twl[(1u << (G::K1 - 1 - b)) + (e >> (b + 1))]; };
-        fwd_run<LRC, G::K1, G::K1>(lds + cc * G::SC, v, t, twf, P.p);
-        gu64* mid = gp(J.mid) + (size_t)pos * G::N + c0 + cc;
+        fwd_run<LRC, G::K1, G::K1, true>(ar, reinterpret_cast<V*>(lds) + cc * G::SC, v, t, twf);
+        gu64* mid = gp(J.mid) + (size_t)pos * G::N;
 #pragma unroll
-        for (int j = 0; j < R; ++j) mid[(size_t)elem<LRC, 0, NBL>(t, j) * G::N2] = v[j];
-    }
+        for (int j = 0; j < R; ++j) mid[col + elem<LRC, 0, NBL>(t, j) * G::N2] = A::pack(v[j]);
+    });
 }
 
 // Forward pass 2: row sub-transforms (global stages K1..logN-1) + epilogue.
 template <int LOGN, int W, int STORE>
-__global__ void __launch_bounds__((NttGeom<LOGN, W>::NTR)) k_ntt_fwd_rows(DevTables T, NttJobs L, int limbs) {
-    using G = NttGeom<LOGN, W>;
-    constexpr int R = G::R, NB1 = first_nb<G::LR, G::K2>(), LO1 = G::K2 - NB1, NBL = fwd_last_nb<G::LR, G::K2>();
+__global__ void __launch_bounds__((Rows<LOGN, W>::NTR)) k_ntt_fwd_rows(DevTables T, NttJobs L, NttGrid g) {
+    using G = Rows<LOGN, W>;
     __shared__ uint64_t lds[G::RR * G::SR];
     constexpr int TPL = G::N1 / G::RR;  // tiles per limb
-    // grid-stride loop over (limb, tile); a launch with one block per tile
-    // runs one iteration per block
-    for (int tile = blockIdx.x; tile < TPL * limbs; tile += gridDim.x) {
-        const int limb_ = tile / TPL, tx_ = tile % TPL;
-        if (tile != (int)blockIdx.x) __syncthreads();  // LDS reuse across tiles
-        int pos;
-        const NttJob J = load_ntt_job(L, limb_, pos);
-        const int pid = pos_pid(pos, J.nq, J.q0, T.L + 1);
-        const PrimeInfo P = cld(T.primes + pid);
-        const int r0 = tx_ * G::RR;
-        const int tid = threadIdx.x;
-        const int t = tid % G::TR, rr = tid / G::TR;
-        const size_t base = (size_t)pos * G::N + (size_t)(r0 + rr) * G::N2;
-
-        // Loads run ahead of use without holding every phase's operands in
-        // registers at once: each phase's twiddles are issued one phase
-        // early (the first phase's with the tile), the epilogue operands of
-        // the elements this thread stores two phases before the store.
-        ShoupConst twr[G::NS];
-        const uint32_t row = G::N1 + r0 + rr;
-        const ShoupConst* twtab = T.tw_fwd + (size_t)pid * G::N;
-        auto idx = [&](int b, uint32_t e) { return (row << (G::K2 - 1 - b)) + (e >> (b + 1)); };
-        fwd_prefetch<G::LR, G::K2, G::K2>(twr, twtab, t, idx);
-        uint64_t v[R];
-        {
-            const gu64* mid = gp(J.mid) + base;
+    const uint32_t item = xcd_item(g.chunk);
+    NttJob J;
+    int pos;
+    if (!block_job(L, g, item / TPL, J, pos)) return;
+    const int pid = pos_pid(pos, J.nq, J.q0, T.L + 1);
+    const int t = threadIdx.x % G::TR, rr = threadIdx.x / G::TR;
+    const uint32_t r = (item % TPL) * G::RR + rr;
+    const size_t limb = (size_t)pos * G::N;
+    const uint32_t row = r * G::N2;
+    uint64_t x[G::R];
+    {
+        const gu64* mid = gp(J.mid) + limb;
 #pragma unroll
-            for (int j = 0; j < R; ++j) v[j] = mid[elem<G::LR, LO1, NB1>(t, j)];
-        }
-        uint64_t e0[R], e1[R];
-        gu64* dst = gp(J.dst) + base;
-        auto epi_load = [&]() {
-            if constexpr (STORE == STORE_MODDOWN || STORE == STORE_MODDOWN_RESCALE || STORE == STORE_MODDOWN_AUTO) {
-                const gu64* aux = gp(J.aux) + base;
-                const gu64* add = J.add ? gp(J.add) + base : nullptr;
-#pragma unroll
-                for (int j = 0; j < R; ++j) {
-                    const uint32_t e = elem<G::LR, 0, NBL>(t, j);
-                    e0[j] = aux[e];
-                    e1[j] = add ? add[e] : 0;
-                }
-            } else if constexpr (STORE == STORE_RESCALE) {
-#pragma unroll
-                for (int j = 0; j < R; ++j) e0[j] = dst[elem<G::LR, 0, NBL>(t, j)];
-            }
-        };
-        // the epilogue loads are issued at the start of the phase before the
-        // last one (phases start at K2, K2 - LR, ..., fwd_last_nb)
-        constexpr int EPI_HI = fwd_last_nb<G::LR, G::K2>() + G::LR < G::K2 ? fwd_last_nb<G::LR, G::K2>() + G::LR : G::K2;
-        auto hook = [&](auto hi) {
-            constexpr int H = decltype(hi)::value;
-            fwd_prefetch<G::LR, G::K2, H - G::LR>(twr, twtab, t, idx);
-            if constexpr (H == EPI_HI) epi_load();
-        };
-        auto twf = [&](int s, int, uint32_t) { return twr[s]; };
-        fwd_run<G::LR, G::K2, G::K2>(lds + rr * G::SR, v, t, twf, P.p, hook);
-        if constexpr (STORE == STORE_PLAIN) {
-#pragma unroll
-            for (int j = 0; j < R; ++j) dst[elem<G::LR, 0, NBL>(t, j)] = reduce4p(v[j], P.p);
-        } else if constexpr (STORE == STORE_MODDOWN) {
-            const ShoupConst pinv = cld(T.pinv + pid);
-#pragma unroll
-            for (int j = 0; j < R; ++j) {
-                const uint64_t x = reduce4p(v[j], P.p);
-                // the addend is 0 when absent, so the add is a no-op then
-                dst[elem<G::LR, 0, NBL>(t, j)] = addmod(mul_shoup(submod(e0[j], x, P.p), pinv.w, pinv.wp, P.p), e1[j], P.p);
-            }
-        } else if constexpr (STORE == STORE_MODDOWN_AUTO) {
-            // Element jg = r N2 + e sits at exponent 2 brev(jg) + 1 =
-            // 2 N1 brev(e) + 2 brev(r) + 1; times k (mod 2N) it lands at
-            // row brev(((c mod 2N1) - 1) / 2), column brev((brev(e) k + (c >> (K1+1))) mod N2)
-            // with c = (2 brev(r) + 1) k mod 2N: one destination row per row.
-            const ShoupConst pinv = cld(T.pinv + pid);
-            const uint32_t k = J.autok;
-            const uint32_t cx = (uint32_t)(((2ull * brev_bits(r0 + rr, G::K1) + 1) * k) & (2ull * G::N - 1));
-            const uint32_t rdst = brev_bits((cx & (2u * G::N1 - 1)) >> 1, G::K1);
-            const uint32_t coff = cx >> (G::K1 + 1);
-            uint64_t* row = lds + rr * G::SR;
-            __syncthreads();  // the last phase's LDS reads are done
-#pragma unroll
-            for (int j = 0; j < R; ++j) {
-                const uint64_t x = reduce4p(v[j], P.p);
-                const uint32_t e = elem<G::LR, 0, NBL>(t, j);
-                const uint32_t e2 = brev_bits((brev_bits(e, G::K2) * k + coff) & (G::N2 - 1), G::K2);
-                row[lds_off(e2)] = addmod(mul_shoup(submod(e0[j], x, P.p), pinv.w, pinv.wp, P.p), e1[j], P.p);
-            }
-            __syncthreads();
-            gu64* out = gp(J.dst) + (size_t)pos * G::N + (size_t)rdst * G::N2;
-#pragma unroll
-            for (int j = 0; j < R; ++j) {
-                const uint32_t e = elem<G::LR, 0, NBL>(t, j);
-                out[e] = row[lds_off(e)];
-            }
-        } else if constexpr (STORE == STORE_MODDOWN_RESCALE) {
-            // r = (acc P^-1 + add - v) q_l^-1  (see k_moddown_conv)
-            const ShoupConst pinv = cld(T.pinv + pid);
-            const ShoupConst qi = cld(T.qlinv + (size_t)J.level * (T.L + 1) + pid);
-#pragma unroll
-            for (int j = 0; j < R; ++j) {
-                const uint64_t x = reduce4p(v[j], P.p);
-                const uint64_t y = addmod(mul_shoup(e0[j], pinv.w, pinv.wp, P.p), e1[j], P.p);
-                dst[elem<G::LR, 0, NBL>(t, j)] = mul_shoup(submod(y, x, P.p), qi.w, qi.wp, P.p);
-            }
-        } else {  // STORE_RESCALE
-            const ShoupConst qi = cld(T.qlinv + (size_t)J.level * (T.L + 1) + pid);
-#pragma unroll
-            for (int j = 0; j < R; ++j) {
-                const uint64_t x = reduce4p(v[j], P.p);
-                dst[elem<G::LR, 0, NBL>(t, j)] = mul_shoup(submod(e0[j], x, P.p), qi.w, qi.wp, P.p);
-            }
-        }
+        for (int j = 0; j < G::R; ++j) x[j] = mid[row + elem<G::LR, G::LO1, G::NB1>(t, j)];
     }
+    const PrimeInfo P = cld(T.primes + pid);
+    uint64_t* sub = lds + rr * G::SR;
+    with_arith(T, pid, P, [&](const auto& ar) {
+        using A = std::decay_t<decltype(ar)>;
+        using V = typename A::V;
+        V v[G::R];
+#pragma unroll
+        for (int j = 0; j < G::R; ++j) v[j] = A::unpack(x[j]);
+        Epilogue<G, STORE> epi;
+        // the epilogue's operands are issued at the start of the phase before the last
+        constexpr int EPI_HI = G::NBL + G::LR < G::K2 ? G::NBL + G::LR : G::K2;
+        fwd_row<G, false>(ar, reinterpret_cast<V*>(sub), v, t, G::N1 + r, A::fwd(T) + (size_t)pid * G::N,
+                          [&](auto hi) {
+                              if constexpr (decltype(hi)::value == EPI_HI) epi.load(J, limb, row, t);
+                          });
+        epi.store(T, J, pos, pid, ar, sub, t, r, v);
+    });
 }
 
 // Inverse pass 1: row sub-transforms (global stages on bits 0..K2-1).
 template <int LOGN, int W>
-__global__ void __launch_bounds__((NttGeom<LOGN, W>::NTR)) k_ntt_inv_rows(DevTables T, NttJobs L, int limbs) {
-    using G = NttGeom<LOGN, W>;
-    constexpr int R = G::R, NB1 = first_nb<G::LR, G::K2>(), LOL = inv_last_lo<G::LR, G::K2>(), NBL = G::K2 - LOL;
+__global__ void __launch_bounds__((Rows<LOGN, W>::NTR)) k_ntt_inv_rows(DevTables T, NttJobs L, NttGrid g) {
+    using G = Rows<LOGN, W>;
     __shared__ uint64_t lds[G::RR * G::SR];
     constexpr int TPL = G::N1 / G::RR;  // tiles per limb
-    // grid-stride loop over (limb, tile); a launch with one block per tile
-    // runs one iteration per block
-    for (int tile = blockIdx.x; tile < TPL * limbs; tile += gridDim.x) {
-        const int limb_ = tile / TPL, tx_ = tile % TPL;
-        if (tile != (int)blockIdx.x) __syncthreads();  // LDS reuse across tiles
-        int pos;
-        const NttJob J = load_ntt_job(L, limb_, pos);
-        const int pid = pos_pid(pos, J.nq, J.q0, T.L + 1);
-        const PrimeInfo P = cld(T.primes + pid);
-        const int r0 = tx_ * G::RR;
-        const int tid = threadIdx.x;
-        const int t = tid % G::TR, rr = tid / G::TR;
-        const size_t base = (size_t)pos * G::N + (size_t)(r0 + rr) * G::N2;
-
-        ShoupConst twr[G::NS];
-        const uint32_t row = G::N1 + r0 + rr;
-        const ShoupConst* twtab = T.tw_inv + (size_t)pid * G::N;
-        auto idx = [&](int b, uint32_t e) { return (row << (G::K2 - 1 - b)) + (e >> (b + 1)); };
-        // each phase's twiddles are issued one phase early (the first's with the tile)
-        inv_prefetch<G::LR, G::K2, 0>(twr, twtab, t, idx);
-        auto hook = [&](auto lo) { inv_prefetch<G::LR, G::K2, decltype(lo)::value + G::LR>(twr, twtab, t, idx); };
-        uint64_t v[R];
-        {
-            const gu64* src = gp(J.src) + base;
+    const uint32_t item = xcd_item(g.chunk);
+    NttJob J;
+    int pos;
+    if (!block_job(L, g, item / TPL, J, pos)) return;
+    const int pid = pos_pid(pos, J.nq, J.q0, T.L + 1);
+    const int t = threadIdx.x % G::TR, rr = threadIdx.x / G::TR;
+    const uint32_t r = (item % TPL) * G::RR + rr;
+    const size_t limb = (size_t)pos * G::N;
+    const uint32_t row = r * G::N2;
+    uint64_t x[G::R];
+    {
+        const gu64* src = gp(J.src) + limb;
 #pragma unroll
-            for (int j = 0; j < R; ++j) v[j] = src[elem<G::LR, 0, NB1>(t, j)];
-        }
-        auto twf = [&](int s, int, uint32_t) { return twr[s]; };
-        inv_run<G::LR, G::K2, 0, false>(lds + rr * G::SR, v, t, twf, P.p, ShoupConst{0, 0}, ShoupConst{0, 0}, hook);
-        gu64* mid = gp(J.mid) + base;
-#pragma unroll
-        for (int j = 0; j < R; ++j) mid[elem<G::LR, LOL, NBL>(t, j)] = v[j];
+        for (int j = 0; j < G::R; ++j) x[j] = src[row + G::mem(t, j)];
     }
+    const PrimeInfo P = cld(T.primes + pid);
+    with_arith(T, pid, P, [&](const auto& ar) {
+        using A = std::decay_t<decltype(ar)>;
+        using V = typename A::V;
+        V v[G::R];
+#pragma unroll
+        for (int j = 0; j < G::R; ++j) v[j] = ar.from(x[j]);
+        inv_row<G>(ar, reinterpret_cast<V*>(lds) + rr * G::SR, v, t, G::N1 + r,
+                          A::inv(T) + (size_t)pid * G::N);
+        gu64* mid = gp(J.mid) + limb;
+#pragma unroll
+        for (int j = 0; j < G::R; ++j) mid[row + elem<G::LR, G::LOL, G::NBI>(t, j)] = A::pack(v[j]);
+    });
 }
 
 // Inverse pass 2: column sub-transforms, last stage scaled by N^-1 (x factor).
 template <int LOGN, int W, int LRC>
-__global__ void __launch_bounds__((NttGeom<LOGN, W, LRC>::NTC)) k_ntt_inv_cols(DevTables T, NttJobs L, int limbs) {
-    using G = NttGeom<LOGN, W, LRC>;
+__global__ void __launch_bounds__((ColGeom<LOGN, W, LRC>::NTC)) k_ntt_inv_cols(DevTables T, NttJobs L, NttGrid g) {
+    using G = ColGeom<LOGN, W, LRC>;
     constexpr int R = G::RC, NB1 = first_nb<LRC, G::K1>(), LOL = inv_last_lo<LRC, G::K1>(), NBL = G::K1 - LOL;
     __shared__ uint64_t lds[G::CC * G::SC];
-    __shared__ ShoupConst twl[G::N1];
-    constexpr int TPL = G::N2 / G::CC;  // tiles per limb
-    // grid-stride loop over (limb, tile); a launch with one block per tile
-    // runs one iteration per block
-    for (int tile = blockIdx.x; tile < TPL * limbs; tile += gridDim.x) {
-        const int limb_ = tile / TPL, tx_ = tile % TPL;
-        if (tile != (int)blockIdx.x) __syncthreads();  // LDS reuse across tiles
-        int pos;
-        const NttJob J = load_ntt_job(L, limb_, pos);
-        const int pid = pos_pid(pos, J.nq, J.q0, T.L + 1);
-        const PrimeInfo P = cld(T.primes + pid);
-        const int c0 = tx_ * G::CC;
-        const int tid = threadIdx.x;
-        const int cc = tid % G::CC, t = tid / G::CC;
-
-        const ShoupConst* sc;
-        if (J.scale_sel == ISCALE_MODUP)
-            sc = T.iscale_modup + ((size_t)J.level * (T.L + 1) + pos) * 2;
-        else if (J.scale_sel == ISCALE_MODDOWN)
-            sc = T.iscale_moddown + (size_t)(pos - J.nq) * 2;
-        else
-            sc = T.iscale_plain + (size_t)pid * 2;
-        const ShoupConst s = cld(sc), ws = cld(sc + 1);
-
-        {
-            const ShoupConst* tw = T.tw_inv + (size_t)pid * G::N;
-            for (int i = tid; i < G::N1; i += G::NTC) twl[i] = tw[i];
-        }
-        uint64_t v[R];
-        {
-            const gu64* mid = gp(J.mid) + (size_t)pos * G::N + c0 + cc;
+    __shared__ ShoupConst twlds[G::N1];
+    const uint32_t item = xcd_item(g.chunk);
+    NttJob J;
+    int pos;
+    if (!block_job(L, g, item / G::TPL, J, pos)) return;
+    const int pid = pos_pid(pos, J.nq, J.q0, T.L + 1);
+    const int cc = threadIdx.x % G::CC, t = threadIdx.x / G::CC;
+    const uint32_t col = (item % G::TPL) * G::CC + cc;
+    uint64_t x[R];
+    {
+        const gu64* mid = gp(J.mid) + (size_t)pos * G::N;
 #pragma unroll
-            for (int j = 0; j < R; ++j) v[j] = mid[(size_t)elem<LRC, 0, NB1>(t, j) * G::N2];
-        }
+        for (int j = 0; j < R; ++j) x[j] = mid[col + elem<LRC, 0, NB1>(t, j) * G::N2];
+    }
+    const PrimeInfo P = cld(T.primes + pid);
+    const ShoupConst* sc = inv_scale(T, J, pos, pid);
+    const ShoupConst s = cld(sc), ws = cld(sc + 1);
+    with_arith(T, pid, P, [&](const auto& ar) {
+        using A = std::decay_t<decltype(ar)>;
+        using V = typename A::V;
+        typename A::W tw[G::NTW];
+        auto* twl = reinterpret_cast<typename A::W*>(twlds);
+        stage_load<G>(A::inv(T) + (size_t)pid * G::N, tw);
+        V v[R];
+#pragma unroll
+        for (int j = 0; j < R; ++j) v[j] = A::unpack(x[j]);
+        stage_put<G>(twl, tw);
         __syncthreads();
         auto twf = [&](int, int b, uint32_t e) { return twl[(1u << (G::K1 - 1 - b)) + (e >> (b + 1))]; };
-        inv_run<LRC, G::K1, 0, true>(lds + cc * G::SC, v, t, twf, P.p, s, ws);
-        gu64* dst = gp(J.dst) + (size_t)pos * G::N + c0 + cc;
+        inv_run<LRC, G::K1, 0, true>(ar, reinterpret_cast<V*>(lds) + cc * G::SC, v, t, twf, s, ws);
+        gu64* dst = gp(J.dst) + (size_t)pos * G::N;
 #pragma unroll
-        for (int j = 0; j < R; ++j) dst[(size_t)elem<LRC, LOL, NBL>(t, j) * G::N2] = reduce2p(v[j], P.p);
-    }
+        for (int j = 0; j < R; ++j) dst[col + elem<LRC, LOL, NBL>(t, j) * G::N2] = ar.canon_inv(v[j]);
+    });
+}
+
+// Centered FP64 twiddles of the primes that use them.
+__global__ void k_fp_twiddles(DevTables T, const ShoupConst* tw, double* out) {
+    const PrimeInfo P = cld(T.primes + blockIdx.y);
+    if (!P.fp) return;
+    const size_t i = (size_t)blockIdx.y * T.N + blockIdx.x * blockDim.x + threadIdx.x;
+    const uint64_t w = tw[i].w;
+    out[i] = w > (P.p >> 1) ? fp_from(w) - P.pd : fp_from(w);
 }
 
 // ---------------------------------------------------------- launchers ----
 
 // Launch configuration of a transform: column tile width, log2 values per
-// column thread, row tile height, grid cap (0 = one block per tile).
+// column thread, row tile height (the fourth entry of a tuning configuration
+// capped the grid of a looping form and has no effect).
 struct NttPick {
     int cc, lrc, rr, pb;
 };
-
 // Fixed rules (measured on MI355X at N=2^16 over 2..25 limbs): column tiles
 // are 16 wide (128-byte row segments; 4-wide tiles lose more to partial lines
 // than they gain in parallelism) except for launches of under 64 tiles; row
 // tiles are 4 rows (256 threads), which keeps register-prefetched twiddles at
 // full occupancy; 8 values per column thread (radix-8 phases, one LDS
 // exchange fewer) from 40 limbs up, where it measured 3-15% faster.
-// FIDES_NTT_COLS / FIDES_NTT_ROWS (4, 8 or 16), FIDES_NTT_LRC (2 or 3) and
-// FIDES_NTT_PB force a value.
+// FIDES_NTT_COLS / FIDES_NTT_ROWS (4, 8 or 16) and FIDES_NTT_LRC (2 or 3)
+// force a value.
 static int env_int(const char* name) {
     const char* e = std::getenv(name);
     return e ? std::atoi(e) : -1;
 }
 static NttPick rule_pick(int logN, int limbs) {
     static const int ov_c = env_int("FIDES_NTT_COLS"), ov_r = env_int("FIDES_NTT_ROWS");
-    static const int ov_l = env_int("FIDES_NTT_LRC"), ov_pb = env_int("FIDES_NTT_PB");
+    static const int ov_l = env_int("FIDES_NTT_LRC");
     auto width = [](int w) { return w == 4 || w == 8 ? w : 16; };
     const int n2 = 1 << (logN / 2);
     const int tiles16 = limbs * (n2 < 16 ? 1 : n2 / 16);
@@ -569,7 +281,7 @@ static NttPick rule_pick(int logN, int limbs) {
     p.cc = ov_c > 0 ? width(ov_c) : (tiles16 < 64 ? 4 : 16);
     p.rr = ov_r > 0 ? width(ov_r) : 4;
     p.lrc = ov_l > 0 ? (ov_l == 3 ? 3 : 2) : (limbs >= 40 ? 3 : 2);
-    p.pb = ov_pb > 0 ? ov_pb : 0;
+    p.pb = 0;
     return p;
 }
 
@@ -586,47 +298,46 @@ TuneCfg ntt_rule_cfg(bool, int logN, int limbs) {
     return TuneCfg{{p.cc, p.lrc, p.rr, p.pb}};
 }
 
-// Blocks of a pass: one per tile, or at most pb blocks looping over the tiles.
-static dim3 pass_grid(int tiles, int pb) { return dim3(pb > 0 && pb < tiles ? pb : tiles); }
-
 template <int LOGN, int W, int LRC>
-static void fwd_cols(const DevTables& T, const NttJobs& L, int limbs, int load, int pb, hipStream_t s) {
-    using G = NttGeom<LOGN, W, LRC>;
-    const dim3 g = pass_grid(G::N2 / G::CC * limbs, pb);
+static void fwd_cols(const DevTables& T, const NttJobs& L, int limbs, int load, hipStream_t s) {
+    using G = ColGeom<LOGN, W, LRC>;
+    const NttGrid n = ntt_grid(L, limbs, G::TPL);
+    const dim3 g = n.grid;
     if (load == LOAD_SWITCH)
-        hipLaunchKernelGGL((k_ntt_fwd_cols<LOGN, W, LRC, LOAD_SWITCH>), g, dim3(G::NTC), 0, s, T, L, limbs);
+        hipLaunchKernelGGL((k_ntt_fwd_cols<LOGN, W, LRC, LOAD_SWITCH>), g, dim3(G::NTC), 0, s, T, L, n);
     else
-        hipLaunchKernelGGL((k_ntt_fwd_cols<LOGN, W, LRC, LOAD_PLAIN>), g, dim3(G::NTC), 0, s, T, L, limbs);
+        hipLaunchKernelGGL((k_ntt_fwd_cols<LOGN, W, LRC, LOAD_PLAIN>), g, dim3(G::NTC), 0, s, T, L, n);
 }
 
 template <int LOGN, int W, int LRC>
-static void inv_cols(const DevTables& T, const NttJobs& L, int limbs, int pb, hipStream_t s) {
-    using G = NttGeom<LOGN, W, LRC>;
-    hipLaunchKernelGGL((k_ntt_inv_cols<LOGN, W, LRC>), pass_grid(G::N2 / G::CC * limbs, pb), dim3(G::NTC), 0, s, T,
-                       L, limbs);
+static void inv_cols(const DevTables& T, const NttJobs& L, int limbs, hipStream_t s) {
+    using G = ColGeom<LOGN, W, LRC>;
+    const NttGrid n = ntt_grid(L, limbs, G::TPL);
+    hipLaunchKernelGGL((k_ntt_inv_cols<LOGN, W, LRC>), n.grid, dim3(G::NTC), 0, s, T, L, n);
 }
 
 template <int LOGN, int W>
-static void fwd_rows(const DevTables& T, const NttJobs& L, int limbs, int store, int pb, hipStream_t s) {
-    using G = NttGeom<LOGN, W>;
-    const dim3 g = pass_grid(G::N1 / G::RR * limbs, pb);
+static void fwd_rows(const DevTables& T, const NttJobs& L, int limbs, int store, hipStream_t s) {
+    using G = Rows<LOGN, W>;
+    const NttGrid n = ntt_grid(L, limbs, G::N1 / G::RR);
+    const dim3 g = n.grid, b(G::NTR);
     if (store == STORE_MODDOWN)
-        hipLaunchKernelGGL((k_ntt_fwd_rows<LOGN, W, STORE_MODDOWN>), g, dim3(G::NTR), 0, s, T, L, limbs);
+        hipLaunchKernelGGL((k_ntt_fwd_rows<LOGN, W, STORE_MODDOWN>), g, b, 0, s, T, L, n);
     else if (store == STORE_MODDOWN_AUTO)
-        hipLaunchKernelGGL((k_ntt_fwd_rows<LOGN, W, STORE_MODDOWN_AUTO>), g, dim3(G::NTR), 0, s, T, L, limbs);
+        hipLaunchKernelGGL((k_ntt_fwd_rows<LOGN, W, STORE_MODDOWN_AUTO>), g, b, 0, s, T, L, n);
     else if (store == STORE_MODDOWN_RESCALE)
-        hipLaunchKernelGGL((k_ntt_fwd_rows<LOGN, W, STORE_MODDOWN_RESCALE>), g, dim3(G::NTR), 0, s, T, L, limbs);
+        hipLaunchKernelGGL((k_ntt_fwd_rows<LOGN, W, STORE_MODDOWN_RESCALE>), g, b, 0, s, T, L, n);
     else if (store == STORE_RESCALE)
-        hipLaunchKernelGGL((k_ntt_fwd_rows<LOGN, W, STORE_RESCALE>), g, dim3(G::NTR), 0, s, T, L, limbs);
+        hipLaunchKernelGGL((k_ntt_fwd_rows<LOGN, W, STORE_RESCALE>), g, b, 0, s, T, L, n);
     else
-        hipLaunchKernelGGL((k_ntt_fwd_rows<LOGN, W, STORE_PLAIN>), g, dim3(G::NTR), 0, s, T, L, limbs);
+        hipLaunchKernelGGL((k_ntt_fwd_rows<LOGN, W, STORE_PLAIN>), g, b, 0, s, T, L, n);
 }
 
 template <int LOGN, int W>
-static void inv_rows(const DevTables& T, const NttJobs& L, int limbs, int pb, hipStream_t s) {
-    using G = NttGeom<LOGN, W>;
-    hipLaunchKernelGGL((k_ntt_inv_rows<LOGN, W>), pass_grid(G::N1 / G::RR * limbs, pb), dim3(G::NTR), 0, s, T, L,
-                       limbs);
+static void inv_rows(const DevTables& T, const NttJobs& L, int limbs, hipStream_t s) {
+    using G = Rows<LOGN, W>;
+    const NttGrid n = ntt_grid(L, limbs, G::N1 / G::RR);
+    hipLaunchKernelGGL((k_ntt_inv_rows<LOGN, W>), n.grid, dim3(G::NTR), 0, s, T, L, n);
 }
 
 template <class F>
@@ -639,25 +350,23 @@ static void by_width(int w, F&& f) {
         f(std::integral_constant<int, 16>{});
 }
 
-// Column-pass dispatch over (tile width, values per thread).  logN = 17 has
-// only the 8-value form (a 16-wide tile of 4-value threads exceeds 1024).
+// Column-pass dispatch over (tile width, values per thread).
 template <int LOGN, bool FWD>
 static void cols_dispatch(const DevTables& T, const NttJobs& L, int limbs, int load, const NttPick& pk,
                           hipStream_t s) {
-    const int lrc = ntt_lr<LOGN>() == 3 ? 3 : pk.lrc;
     by_width(pk.cc, [&](auto wv) {
         constexpr int WW = decltype(wv)::value;
         auto go = [&](auto lv) {
             constexpr int LL = decltype(lv)::value;
             if constexpr (FWD)
-                fwd_cols<LOGN, WW, LL>(T, L, limbs, load, pk.pb, s);
+                fwd_cols<LOGN, WW, LL>(T, L, limbs, load, s);
             else
-                inv_cols<LOGN, WW, LL>(T, L, limbs, pk.pb, s);
+                inv_cols<LOGN, WW, LL>(T, L, limbs, s);
         };
-        if (lrc == 3)
+        if (pk.lrc == 3)
             go(std::integral_constant<int, 3>{});
         else
-            go(std::integral_constant<int, ntt_lr<LOGN>()>{});
+            go(std::integral_constant<int, min_lrc<LOGN>()>{});
     });
 }
 
@@ -667,17 +376,22 @@ static hipError_t fwd_impl(const DevTables& T, const NttJobs& L, int limbs, int 
     cols_dispatch<LOGN, true>(T, L, limbs, load, pk, s);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    by_width(pk.rr, [&](auto wr) { fwd_rows<LOGN, decltype(wr)::value>(T, L, limbs, store, pk.pb, s); });
+    by_width(pk.rr, [&](auto wr) { fwd_rows<LOGN, decltype(wr)::value>(T, L, limbs, store, s); });
     return hipGetLastError();
 }
 
 template <int LOGN>
 static hipError_t inv_impl(const DevTables& T, const NttJobs& L, int limbs, hipStream_t s) {
     const NttPick pk = ntt_pick(false, LOGN, limbs);
-    by_width(pk.rr, [&](auto wr) { inv_rows<LOGN, decltype(wr)::value>(T, L, limbs, pk.pb, s); });
+    by_width(pk.rr, [&](auto wr) { inv_rows<LOGN, decltype(wr)::value>(T, L, limbs, s); });
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     cols_dispatch<LOGN, false>(T, L, limbs, 0, pk, s);
+    return hipGetLastError();
+}
+
+hipError_t launch_fp_twiddles(const DevTables& T, const ShoupConst* tw, double* out, hipStream_t s) {
+    hipLaunchKernelGGL(k_fp_twiddles, dim3(T.N / 256, T.np), dim3(256), 0, s, T, tw, out);  // N >= 2^10
     return hipGetLastError();
 }
 

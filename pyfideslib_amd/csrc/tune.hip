@@ -5,7 +5,7 @@
 // File format, one entry per line ('#' starts a comment):
 //   <kind> <logN> <size_lo> <size_hi> <v0> <v1> <v2> <v3>
 // kind: ntt_fwd | ntt_inv (size = limbs per launch; v = column tile width,
-// log2 values per column thread, row tile height, grid cap) or modup |
+// log2 values per column thread, row tile height, unused) or modup |
 // moddown (size = conversions per launch; v0 = target groups; modup v1 = 1:
 // the matrix-core conversion, k_modup_mfma).
 #include <dlfcn.h>

@@ -6,8 +6,7 @@ context's stream:
   * the forward and inverse NTT at limb counts 1 .. 8 (L+1+K) (the launch
     shapes of single ops and of batched stages; fides_ntt_limbs) over every
     column tile width (4, 8, 16), values per column thread (4, 8), row tile
-    height (4, 8, 16) and grid cap (one block per tile, or 1-2 blocks per CU
-    looping over the tiles);
+    height (4, 8, 16);
   * the ModUp conversion's target groups at 1, 2 and 3 digit conversions per
     launch (fides_stage_modup at levels with that many digits), and the int8
     matrix-core form of the same conversion against them, and the ModDown
@@ -90,8 +89,7 @@ def tune_ntt(F, ctx, raw, reps: int, margin: float, log):
     cap = max(sizes)
     host = np.stack([rng.integers(0, mods[i % np_], N, dtype=np.uint64) for i in range(cap)])
     buf = ctx.device_array((cap, N), host)
-    n_cu = 256
-    cands = [c for c in itertools.product((4, 8, 16), (2, 3), (4, 8, 16), (0, n_cu, 2 * n_cu))
+    cands = [c for c in itertools.product((4, 8, 16), (2, 3), (4, 8, 16), (0,))
              if not (raw.logN == 17 and c[1] == 2)]
     rows = []
     for kind, inverse in ((F.TUNE_NTT_FWD, False), (F.TUNE_NTT_INV, True)):
