@@ -97,7 +97,7 @@ static int active(const NttJob& j) { return j.npos - (j.skip_hi - j.skip_lo); }
 
 // Launch NTT jobs, NTT_INLINE per launch.
 static void run_ntt(Context& c, std::vector<NttJob> jobs, bool inverse, int load = LOAD_PLAIN,
-                    int store = STORE_PLAIN) {
+                    int store = STORE_PLAIN, int passes = NTT_BOTH) {
     for (size_t b = 0; b < jobs.size(); b += NTT_INLINE) {
         NttJobs L = inline_list<NttJobs>();
         int total = 0;
@@ -106,14 +106,14 @@ static void run_ntt(Context& c, std::vector<NttJob> jobs, bool inverse, int load
             total += active(jobs[i]);
             L.inl[L.n++] = jobs[i];
         }
-        hipError_t e = inverse ? launch_ntt_inv(c.T, L, total, c.stream)
-                               : launch_ntt_fwd(c.T, L, total, load, store, c.stream);
+        hipError_t e = inverse ? launch_ntt_inv(c.T, L, total, c.stream, passes)
+                               : launch_ntt_fwd(c.T, L, total, load, store, c.stream, passes);
         ck(e, inverse ? "intt launch" : "ntt launch");
     }
 }
 
-void run_ntt_jobs(Context& c, std::vector<NttJob> jobs, bool inverse, int load, int store) {
-    run_ntt(c, std::move(jobs), inverse, load, store);
+void run_ntt_jobs(Context& c, std::vector<NttJob> jobs, bool inverse, int load, int store, int passes) {
+    run_ntt(c, std::move(jobs), inverse, load, store, passes);
 }
 
 // ------------------------------------------------------ key-switch core ----
@@ -127,7 +127,7 @@ struct KsScratch {
         ext = DevBuf(&c.pool, (size_t)c.num_digits(level) * npos * N);
         acc_a = DevBuf(&c.pool, npos * N);
         acc_b = DevBuf(&c.pool, npos * N);
-        tk = DevBuf(&c.pool, (size_t)2 * c.K * N);
+        tk = DevBuf(&c.pool, (size_t)2 * (c.K + 1) * N);  // per part: the limb a rescale drops, K special limbs
         y = DevBuf(&c.pool, 2 * nl * N);
         if (mult) {
             d2 = DevBuf(&c.pool, nl * N);
@@ -189,14 +189,34 @@ static void run_cached(Context& c, const std::vector<uint64_t>& sig_in, Body bod
     hip_check(hipGraphLaunch(g->exec, c.stream), "hipGraphLaunch");
 }
 
+// The inverse transform of a key-switch source x (evaluation form, level l)
+// with ModUp's scale folded in, or only its second pass (t holds the first's).
+static void modup_intt(Context& c, int level, const uint64_t* x, uint64_t* t, int passes = NTT_BOTH) {
+    NttJob ji = ntt_job(x, t, t, level + 1, level + 1, 0);
+    ji.level = level;
+    ji.scale_sel = ISCALE_MODUP;
+    run_ntt(c, {ji}, true, LOAD_PLAIN, STORE_PLAIN, passes);
+}
+
+// The digits of t converted and transformed up to the second pass (fused_ok).
+static void modup_cols(Context& c, int level, const uint64_t* t, uint64_t* ext) {
+    ModUpJobs mj = inline_list<ModUpJobs>();
+    mj.inl[0] = ModUpJob{t, ext, level};
+    mj.n = 1;
+    ck(launch_modup_cols(c.T, mj, c.num_digits(level), level + 1, c.stream), "modup conversion and columns");
+}
+
+// ModUp of x up to what the fused inner product takes.
+void modup_half(Context& c, int level, const uint64_t* x, uint64_t* t, uint64_t* ext) {
+    modup_intt(c, level, x, t);
+    modup_cols(c, level, t, ext);
+}
+
 // ModUp of x (evaluation form, level l) into ext (evaluation form; the digit's
 // own positions are left unwritten: consumers read them from x).
 static void modup(Context& c, int level, const uint64_t* x, uint64_t* t, uint64_t* ext) {
     const int nl = level + 1, npos = nl + c.K, nd = c.num_digits(level);
-    NttJob ji = ntt_job(x, t, t, nl, nl, 0);
-    ji.level = level;
-    ji.scale_sel = ISCALE_MODUP;
-    run_ntt(c, {ji}, true);
+    modup_intt(c, level, x, t);
     ModUpJobs mj = inline_list<ModUpJobs>();
     mj.inl[0] = ModUpJob{t, ext, level};
     mj.n = 1;
@@ -210,6 +230,43 @@ static void modup(Context& c, int level, const uint64_t* x, uint64_t* t, uint64_
         jobs.push_back(j);
     }
     run_ntt(c, jobs, false);
+}
+
+// The fused form of what follows ModUp: rows + inner product (+ the first pass
+// of what goes down), its second pass, ModDown's conversion + columns, and the
+// rows with the epilogue.  ext as modup_half leaves it.  rescale: add_a / add_b are the
+// tensor terms at level l, folded in as k_moddown_conv states; out_* get level l-1.
+static void fused_ksk_moddown(Context& c, int level, const uint64_t* ext, const uint64_t* own,
+                              const KeySwitchingKey& key, KsScratch& s, uint64_t* out_b, const uint64_t* add_b,
+                              uint64_t* out_a, const uint64_t* add_a, bool rescale, uint32_t autok = 0) {
+    const int nl = level + 1, npos = nl + c.K, nout = rescale ? level : nl;
+    const size_t N = c.N;
+    uint64_t* down[2] = {s.tk.ptr, s.tk.ptr + (size_t)(c.K + 1) * N};
+    KskJobs kj = inline_list<KskJobs>();
+    kj.inl[0] = KskJob{ext, own, key.a.ptr, key.b.ptr, s.acc_a.ptr, s.acc_b.ptr, level, 0, down[0], down[1],
+                       rescale ? add_a : nullptr, rescale ? add_b : nullptr};
+    kj.n = 1;
+    ck(launch_rows_ksk(c.T, kj, npos, c.stream), "rows and ksk inner product");
+    std::vector<NttJob> iv, fw;
+    ModDownJobs mj = inline_list<ModDownJobs>();
+    for (int h = 0; h < 2; ++h) {
+        uint64_t* y = s.y.ptr + (size_t)h * nl * N;
+        NttJob j = rescale ? ntt_job(down[h], down[h], down[h], c.K + 1, 1, level)
+                           : ntt_job(down[h] + N, down[h] + N, down[h] + N, c.K, 0, 0);
+        j.scale_sel = ISCALE_MODDOWN;
+        iv.push_back(j);
+        mj.inl[mj.n++] = ModDownJob{down[h] + N, y, rescale ? down[h] : nullptr, nullptr, level, 0};
+        NttJob f = ntt_job(y, y, h ? out_b : out_a, nout, nout, 0);
+        f.aux = h ? s.acc_b.ptr : s.acc_a.ptr;
+        f.add = h ? add_b : add_a;
+        f.level = level;
+        f.autok = autok;
+        fw.push_back(f);
+    }
+    run_ntt(c, iv, true, LOAD_PLAIN, STORE_PLAIN, NTT_PASS2);
+    ck(launch_moddown_cols(c.T, mj, nl, rescale, c.stream), "moddown conversion and columns");
+    run_ntt(c, fw, false, LOAD_PLAIN, rescale ? STORE_MODDOWN_RESCALE : autok ? STORE_MODDOWN_AUTO : STORE_MODDOWN,
+            NTT_PASS2);
 }
 
 // KSK inner product with `key`, then ModDown of both accumulators:
@@ -294,6 +351,19 @@ static void ksk_moddown_rescale(Context& c, int level, const uint64_t* ext, cons
     run_ntt(c, {fa, fb}, false, LOAD_PLAIN, STORE_MODDOWN_RESCALE);
 }
 
+// ModUp of x, inner product with `key` and ModDown: see ksk_moddown.
+static void key_switch(Context& c, int level, const uint64_t* x, const KeySwitchingKey& key, KsScratch& s,
+                       uint64_t* out_b, const uint64_t* add_b, uint64_t* out_a, const uint64_t* add_a,
+                       uint32_t autok = 0) {
+    if (fused_ok(c.T)) {
+        modup_half(c, level, x, s.t.ptr, s.ext.ptr);
+        fused_ksk_moddown(c, level, s.ext.ptr, x, key, s, out_b, add_b, out_a, add_a, false, autok);
+        return;
+    }
+    modup(c, level, x, s.t.ptr, s.ext.ptr);
+    ksk_moddown(c, level, s.ext.ptr, x, key, s, out_b, add_b, out_a, add_a, autok);
+}
+
 // ------------------------------------------------------------ metadata ----
 static void require_same_key_level(const Ciphertext& a, const Ciphertext& b) {
     if (a.level < 0 || b.level < 0) throw Error(E_STATE, "ciphertext not loaded");
@@ -340,8 +410,15 @@ static void mult_core(Context& c, const Ciphertext* a, const Ciphertext* b, Ciph
     uint64_t *o0 = out.c0(), *o1 = out.c1();
     auto body = [&](KsScratch& s) {
         TensorJobs tj = inline_list<TensorJobs>();
-        tj.inl[0] = TensorJob{a0, a1, b0, b1, o0, o1, s.d2.ptr, nl};
+        tj.inl[0] = TensorJob{a0, a1, b0, b1, o0, o1, s.d2.ptr, nl, 0, s.t.ptr};
         tj.n = 1;
+        if (fused_ok(c.T)) {
+            ck(launch_tensor_rows(c.T, tj, nl, c.stream), "tensor and rows");
+            modup_intt(c, level, s.d2.ptr, s.t.ptr, NTT_PASS2);
+            modup_cols(c, level, s.t.ptr, s.ext.ptr);
+            fused_ksk_moddown(c, level, s.ext.ptr, s.d2.ptr, key, s, o0, o0, o1, o1, do_rescale);
+            return;
+        }
         ck(launch_tensor(c.T, tj, nl, c.stream), "tensor");
         modup(c, level, s.d2.ptr, s.t.ptr, s.ext.ptr);
         if (do_rescale)
@@ -374,8 +451,7 @@ static void mult_core(Context& c, const Ciphertext* a, const Ciphertext* b, Ciph
 void relin_add(Context& c, int level, const uint64_t* d2, uint64_t* o0, uint64_t* o1) {
     if (!c.eval_key) throw Error(E_NOKEY, "no relinearization key loaded");
     KsScratch& s = workspace(c);
-    modup(c, level, d2, s.t.ptr, s.ext.ptr);
-    ksk_moddown(c, level, s.ext.ptr, d2, *c.eval_key, s, o0, o0, o1, o1);
+    key_switch(c, level, d2, *c.eval_key, s, o0, o0, o1, o1);
 }
 
 void eval_square(Context& c, const Ciphertext& a, Ciphertext& out, bool do_rescale) {
@@ -455,8 +531,7 @@ static const KeySwitchingKey& rot_key(Context& c, uint32_t k) {
     return *it->second;
 }
 
-static void finish_rotation(Context& c, const Ciphertext& a, int level, const uint64_t* ext, const uint64_t* own,
-                            uint32_t k, KsScratch& s, Ciphertext& out) {
+static void switch_and_rotate(Context& c, const Ciphertext& a, int level, uint32_t k, KsScratch& s, Ciphertext& out) {
     const size_t N = c.N;
     const int nl = level + 1;
     // ModDown, + c0 and the automorphism in one epilogue; the automorphism
@@ -464,7 +539,7 @@ static void finish_rotation(Context& c, const Ciphertext& a, int level, const ui
     const bool alias = out.c0() == a.c0() || out.c0() == a.c1() || out.c1() == a.c0() || out.c1() == a.c1();
     uint64_t* o0 = alias ? s.tmp.ptr : out.c0();
     uint64_t* o1 = alias ? s.tmp.ptr + (size_t)nl * N : out.c1();
-    ksk_moddown(c, level, ext, own, rot_key(c, k), s, o0, a.c0(), o1, nullptr, c.auto_inverse(k));
+    key_switch(c, level, a.c1(), rot_key(c, k), s, o0, a.c0(), o1, nullptr, c.auto_inverse(k));
     if (alias) {
         ck(hipMemcpyAsync(out.c0(), o0, (size_t)nl * N * 8, hipMemcpyDeviceToDevice, c.stream), "rotate copy c0");
         ck(hipMemcpyAsync(out.c1(), o1, (size_t)nl * N * 8, hipMemcpyDeviceToDevice, c.stream), "rotate copy c1");
@@ -493,10 +568,7 @@ void eval_automorph(Context& c, const Ciphertext& a, uint32_t k, Ciphertext& out
     }
     const int level = a.level;
     const KeySwitchingKey& key = rot_key(c, k);
-    auto body = [&](KsScratch& s) {
-        modup(c, level, a.c1(), s.t.ptr, s.ext.ptr);
-        finish_rotation(c, a, level, s.ext.ptr, a.c1(), k, s, out);
-    };
+    auto body = [&](KsScratch& s) { switch_and_rotate(c, a, level, k, s, out); };
     const std::vector<uint64_t> sig{2, (uint64_t)a.c0(), (uint64_t)out.c0(), (uint64_t)level, k,
                                     (uint64_t)key.a.ptr, (uint64_t)key.b.ptr, (uint64_t)a.c1(), (uint64_t)out.c1()};
     run_cached(c, sig, body);
@@ -513,8 +585,7 @@ void eval_key_switch(Context& c, const Ciphertext& a, int id, Ciphertext& out) {
     const KeySwitchingKey& key = *it->second;
     const int level = a.level;
     auto body = [&](KsScratch& s) {
-        modup(c, level, a.c1(), s.t.ptr, s.ext.ptr);
-        ksk_moddown(c, level, s.ext.ptr, a.c1(), key, s, out.c0(), a.c0(), out.c1(), nullptr, 0);
+        key_switch(c, level, a.c1(), key, s, out.c0(), a.c0(), out.c1(), nullptr);
     };
     const std::vector<uint64_t> sig{3, (uint64_t)a.c0(), (uint64_t)out.c0(), (uint64_t)level, (uint64_t)id,
                                     (uint64_t)key.a.ptr, (uint64_t)key.b.ptr, (uint64_t)a.c1(), (uint64_t)out.c1()};
@@ -612,8 +683,7 @@ void stage_keyswitch(Context& c, int level, const uint64_t* x, const KeySwitchin
                      uint64_t* ks_a) {
     if (level < 0 || level > c.L) throw Error(E_LEVEL, "level out of range");
     KsScratch s(c, level);
-    modup(c, level, x, s.t.ptr, s.ext.ptr);
-    ksk_moddown(c, level, s.ext.ptr, x, k, s, ks_b, nullptr, ks_a, nullptr);
+    key_switch(c, level, x, k, s, ks_b, nullptr, ks_a, nullptr);
 }
 
 void stage_moddown(Context& c, int level, const uint64_t* x_ext, uint64_t* y) {

@@ -398,7 +398,10 @@ void server_counts(const Server& s, int& active, int& queued, uint64_t& used_byt
 void rotate_hoisted_batch(Context& c, const Ciphertext& a, const std::vector<uint32_t>& ks,
                           const std::vector<Ciphertext*>& outs);
 // NTT jobs, NTT_INLINE per launch (ckks.hip).
-void run_ntt_jobs(Context& c, std::vector<NttJob> jobs, bool inverse, int load = LOAD_PLAIN, int store = STORE_PLAIN);
+void run_ntt_jobs(Context& c, std::vector<NttJob> jobs, bool inverse, int load = LOAD_PLAIN, int store = STORE_PLAIN,
+                  int passes = NTT_BOTH);
+// ModUp of x up to what launch_rows_ksk takes (fused_ok).
+void modup_half(Context& c, int level, const uint64_t* x, uint64_t* t, uint64_t* ext);
 // ModUp of x (level l, evaluation form) into ext via the scaled coefficient limbs t.
 void modup_to(Context& c, int level, const uint64_t* x, uint64_t* t, uint64_t* ext);
 

@@ -164,6 +164,8 @@ struct TensorJob {
     const uint64_t *c0, *c1, *d0, *d1;
     uint64_t *o0, *o1, *o2;
     int nl;
+    int pad;
+    uint64_t* t;  // launch_tensor_rows: o2 after the first pass of its inverse transform
 };
 constexpr int TENSOR_INLINE = 2;
 using TensorJobs = JobList<TensorJob, TENSOR_INLINE>;
@@ -177,7 +179,12 @@ struct ModUpJob {
 constexpr int MODUP_INLINE = 2;
 using ModUpJobs = JobList<ModUpJob, MODUP_INLINE>;
 
-// Key-switch inner product over the l+1+K positions of one polynomial.
+// Key-switch inner product over the l+1+K positions of one polynomial.  The
+// fused kernel (launch_rows_ksk) takes ext after the first pass of its
+// transform, and for a ModDown that follows runs the first pass of the inverse
+// on what goes down: special limb k to down_x + (1 + k) N, and with add_a set
+// (a rescale folded in) acc P^-1 + add of limb l to down_x.  Limbs taken down
+// are not written to acc.
 struct KskJob {
     const uint64_t* ext;  // [nd][l+1+K][N]
     const uint64_t* own;  // [l+1][N] evaluation-form source (own-digit positions)
@@ -186,6 +193,11 @@ struct KskJob {
     uint64_t* acc_a;      // [l+1+K][N]
     uint64_t* acc_b;
     int level;
+    int pad;
+    uint64_t* down_a;     // [1 + K][N], or nullptr: every limb stays in acc
+    uint64_t* down_b;
+    const uint64_t* add_a;  // [l+1][N] addends, or nullptr
+    const uint64_t* add_b;
 };
 constexpr int KSK_INLINE = 2;
 using KskJobs = JobList<KskJob, KSK_INLINE>;
@@ -198,8 +210,9 @@ struct ModDownJob {
     const uint64_t* t;        // [K][N] scaled coefficient limbs of the special primes
     uint64_t* y;              // [l+1][N] (or [l][N] z when rescaling)
     const uint64_t* top_acc;  // INTT of acc limb l, or nullptr
-    const uint64_t* top_add;  // INTT of addend limb l
+    const uint64_t* top_add;  // INTT of addend limb l; nullptr: top_acc is INTT(acc P^-1 + addend)
     int level;
+    int pad;
 };
 constexpr int MODDOWN_INLINE = 4;
 using ModDownJobs = JobList<ModDownJob, MODDOWN_INLINE>;
@@ -324,9 +337,13 @@ int conv_rule_tg(int base_blocks, int max_targets);
 
 // ------------------------------------------------------------ launchers ----
 // All launchers enqueue on `stream` and return hipError_t.
+// passes: NTT_PASS1 and / or NTT_PASS2 of the transform (the fused key-switch
+// kernels run the other one).
+enum NttPass { NTT_PASS1 = 1, NTT_PASS2 = 2, NTT_BOTH = 3 };
 hipError_t launch_ntt_fwd(const DevTables& T, const NttJobs& jobs, int total_limbs, int load_mode, int store_mode,
-                          hipStream_t stream);
-hipError_t launch_ntt_inv(const DevTables& T, const NttJobs& jobs, int total_limbs, hipStream_t stream);
+                          hipStream_t stream, int passes = NTT_BOTH);
+hipError_t launch_ntt_inv(const DevTables& T, const NttJobs& jobs, int total_limbs, hipStream_t stream,
+                          int passes = NTT_BOTH);
 // Fills out[np][N] (T.twd_fwd or T.twd_inv) from the integer table tw.
 hipError_t launch_fp_twiddles(const DevTables& T, const ShoupConst* tw, double* out, hipStream_t stream);
 hipError_t launch_tensor(const DevTables& T, const TensorJobs& jobs, int max_nl, hipStream_t stream);
@@ -345,6 +362,23 @@ bool ksk_keystat_on();  // FIDES_KSK_KEYSTAT=0 turns the key-stationary form off
 hipError_t launch_moddown_conv(const DevTables& T, const ModDownJobs& jobs, int max_nl, hipStream_t stream);
 // rescale = every job carries top_acc/top_add (fused ModDown + rescale)
 hipError_t launch_moddown_conv_mode(const DevTables& T, const ModDownJobs& jobs, bool rescale, hipStream_t stream);
+
+// ---- the fused key switch (fused.hip, fused_down.hip) ----
+// Whether these parameters take it: rings of 2^12 .. 2^16, at most 4 digits of
+// at most 10 primes, at most 10 special primes, sums within one reduction.
+bool fused_ok(const DevTables& T);
+// Tensor product, and the first pass of the inverse transform of its third part.
+hipError_t launch_tensor_rows(const DevTables& T, const TensorJobs& jobs, int max_nl, hipStream_t stream);
+// ModUp conversion and the first pass of the forward transform of its outputs.
+// max_nl: limbs of the list's top level.
+hipError_t launch_modup_cols(const DevTables& T, const ModUpJobs& jobs, int max_nd, int max_nl, hipStream_t stream);
+// Second pass of the digits' transforms and the key-switch inner product
+// (several jobs: sorted by key).  shared: all jobs use the same ext / own / level.
+hipError_t launch_rows_ksk(const DevTables& T, const KskJobs& jobs, int max_npos, hipStream_t stream,
+                           bool shared = false);
+// ModDown conversion (+ rescale) and the first pass of its outputs' transform.
+hipError_t launch_moddown_cols(const DevTables& T, const ModDownJobs& jobs, int max_nl, bool rescale,
+                               hipStream_t stream);
 hipError_t launch_elementwise(const DevTables& T, const EwJobs& jobs, int max_nl, int op, hipStream_t stream);
 hipError_t launch_tensor_sum(const DevTables& T, const TensorSumJob& J, hipStream_t s);
 hipError_t launch_lincomb(const DevTables& T, const LinCombJob& job, hipStream_t stream);

@@ -1,0 +1,147 @@
+// Geometry and grids of the fused key-switch kernels (fused.hip, fused_down.hip).
+#pragma once
+#include "conv.hpp"
+#include "ntt_core.hpp"
+
+namespace fides {
+
+constexpr int FUSED_LOGN_MIN = 12, FUSED_LOGN_MAX = 16;
+constexpr int FUSED_CONV_MAX = 10;  // source limbs of a conversion
+constexpr int FUSED_DIGITS = 4;
+
+// Unsigned division by a launch constant d of values up to most: one multiply
+// where it is exact (most d < 2^32), else the division itself.
+struct FastDiv {
+    uint32_t d, m;
+    FastDiv(size_t d_, size_t most)
+        : d((uint32_t)d_), m(most * d_ < 0x100000000ull && d_ > 1 ? (uint32_t)(0x100000000ull / d_ + 1) : 0u) {}
+    __device__ __forceinline__ uint32_t div(uint32_t n) const { return m ? __umulhi(n, m) : d == 1 ? n : n / d; }
+};
+
+// Tiles of the conversion kernels: 4 columns of N1 rows, 512 threads, TB
+// target limbs at a time (2048 outputs, 4 a thread).  The conversion and the
+// column pass use different thread layouts and meet in LDS:
+//   convert  a thread holds its CPT coefficients of every source limb in
+//            registers (30-bit halves, 2 A CPT of them) and computes 4 sums, CPT
+//            coefficients of TPT targets each;
+//   columns  a wave runs whole columns of one target (4 values per thread), so
+//            its LDS exchanges need no block barrier and the waves of 64-bit
+//            and FP64 limbs go their own ways;
+//   store    4 neighbouring columns a row.
+// Two barriers per TB targets, LDS double-buffered.  Holding 4 coefficients per
+// thread and running the column pass in the same layout took 176 registers (2
+// waves per SIMD) and measured 51.8 us against the 45.6 us of separate kernels.
+template <int LOGN>
+struct ConvCols {
+    static constexpr int K1 = (LOGN + 1) / 2, K2 = LOGN / 2;
+    static constexpr int N1 = 1 << K1, N2 = 1 << K2, N = 1 << LOGN;
+    static constexpr int NT = 512, CC = 4, COEF = CC * N1;
+    static constexpr int TPC = N1 / 4;                   // threads per column
+    static constexpr int TB = 2048 / COEF;               // targets at a time
+    static constexpr int CPT = COEF > NT ? COEF / NT : 1;  // coefficients and
+    static constexpr int TPT = 4 / CPT;                  // targets of a thread's sums
+    static constexpr int SC = N1 + N1 / 16 + 1;
+    static constexpr int TPL = N2 / CC;
+    static constexpr int LO1 = K1 - 2, NBL = fwd_last_nb<2, K1>();
+    static_assert(COEF * TB == 4 * NT && TB * N1 == NT && CPT <= 2, "four sums and one twiddle per thread");
+    // the coefficients of thread tid: row, first column (CPT neighbouring columns), first target
+    static __device__ __forceinline__ uint32_t c_row(uint32_t tid) { return (tid * CPT / CC) % N1; }
+    static __device__ __forceinline__ uint32_t c_col(uint32_t tid) { return tid * CPT % CC; }
+    static __device__ __forceinline__ uint32_t c_tgt(uint32_t tid) { return tid * CPT / COEF * TPT; }
+    // column pass: target (wave-uniform), column and thread within the column
+    static __device__ __forceinline__ uint32_t n_tgt(uint32_t tid) { return tid / (CC * TPC); }
+    static __device__ __forceinline__ uint32_t n_col(uint32_t tid) { return tid / TPC % CC; }
+    static __device__ __forceinline__ uint32_t n_t(uint32_t tid) { return tid % TPC; }
+};
+template <int LOGN>
+struct ConvLds {
+    using G = ConvCols<LOGN>;
+    uint64_t tile[2][G::TB][G::CC][G::SC];
+    ShoupConst tw[2][G::TB][G::N1];
+};
+
+// The column pass of a wave's target (prime pid) on the buffer's tile.
+template <int LOGN>
+__device__ __forceinline__ void conv_columns(const DevTables& T, int pid, ConvLds<LOGN>& S, int buf, int i) {
+    using G = ConvCols<LOGN>;
+    const uint32_t t = G::n_t(threadIdx.x), cc = G::n_col(threadIdx.x);
+    const PrimeInfo P = cld(T.primes + pid);
+    with_arith(T, pid, P, [&](const auto& ar) {
+        using A = std::decay_t<decltype(ar)>;
+        using V = typename A::V;
+        const auto* twl = reinterpret_cast<const typename A::W*>(S.tw[buf][i]);
+        V* sub = reinterpret_cast<V*>(S.tile[buf][i][cc]);
+        V v[4];
+        lds_get<2, G::LO1, 2>(sub, t, v);
+        auto twf = [&](int, int b, uint32_t e) { return twl[(1u << (G::K1 - 1 - b)) + (e >> (b + 1))]; };
+        fwd_run<2, G::K1, G::K1, false, true>(ar, sub, v, t, twf);
+        lds_put<2, 0, G::NBL>(sub, t, v);
+    });
+}
+// One twiddle of a target (row r of its table) per thread: read ahead of the
+// conversion, put in LDS after it.
+struct ConvTw {
+    bool fp;
+    ShoupConst w;
+    __device__ __forceinline__ void load(const DevTables& T, int pid, int r) {
+        fp = is_fp(T, pid);
+        if (fp)
+            w.w = (uint64_t)__double_as_longlong(T.twd_fwd[(size_t)pid * T.N + r]);
+        else
+            w = T.tw_fwd[(size_t)pid * T.N + r];
+    }
+    template <int LOGN>
+    __device__ __forceinline__ void put(ConvLds<LOGN>& S, int buf, int i, int r) const {
+        if (fp)
+            reinterpret_cast<uint64_t*>(S.tw[buf][i])[r] = w.w;
+        else
+            S.tw[buf][i][r] = w;
+    }
+};
+// The tile's rows to limb `out`: 2048 words of TB targets, 4 a thread.
+template <int LOGN, class F>
+__device__ __forceinline__ void conv_store(const ConvLds<LOGN>& S, int buf, uint32_t col0, const F& limb) {
+    using G = ConvCols<LOGN>;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        const uint32_t w = (threadIdx.x + q * G::NT) * 2;
+        const uint32_t i = w / G::COEF, row = w / G::CC % G::N1, cc = w % G::CC;
+        uint64_t* o = limb((int)i);
+        if (o) st2(o + row * G::N2 + col0 + cc, S.tile[buf][i][cc][lds_off(row)], S.tile[buf][i][cc + 1][lds_off(row)]);
+    }
+}
+// A wave-uniform conversion sum in the arithmetic of its prime, as tile word.
+__device__ __forceinline__ uint64_t conv_word(const DevTables& T, int pid, const PrimeInfo& P, uint64_t lo,
+                                              uint64_t hi) {
+    const uint64_t r = reduce128_lazy(lo, hi, P);  // [0, 3p)
+    return is_fp(T, pid) ? FpArith::pack(fp_from(r)) : IntArith(P).from_lazy(r);
+}
+
+// Grid of a conversion kernel: items (job, [digit,] target group, tile), a
+// chunk of half a limb's tiles to an XCD at a time.
+struct ConvGrid {
+    uint32_t items, chunk;
+    FastDiv tg, nd;
+};
+// Target groups, of whole rounds of tb targets: about 1024 blocks in all, two
+// rounds of what is resident (512 or 1600 took 5 to 10% longer at N = 2^16, level 24).
+inline int fused_groups(size_t base_blocks, int targets, int tb) {
+    const int rounds = (targets + tb - 1) / tb;
+    size_t g = (size_t)1024 / (base_blocks ? base_blocks : 1);
+    if (g < 1) g = 1;
+    if (g > (size_t)rounds) g = rounds;
+    const size_t each = (rounds + g - 1) / g;  // rounds per group, evened out
+    return (int)((rounds + each - 1) / each);
+}
+
+// The exact sum over the A sources of x_i m_i (m: one matrix row, scalar
+// loads), before its reduction.
+template <int A>
+__device__ __forceinline__ void conv_acc(const Half2* x, const MatRow<A>& row, uint64_t& lo, uint64_t& hi) {
+    Acc4 acc;
+#pragma unroll
+    for (int i = 0; i < A; ++i) mac_split(acc, x[i], split30(row.v[i]));
+    combine(acc, lo, hi);
+}
+
+}  // namespace fides

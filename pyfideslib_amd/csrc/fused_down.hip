@@ -1,0 +1,155 @@
+// ModDown's conversion from the special primes (with the rescale that follows
+// folded in, see k_moddown_conv) and the column pass of its outputs'
+// transform in one kernel; layout and reasons as in fused.hip.
+#include "fused.hpp"
+
+namespace fides {
+
+template <int LOGN, int KK, bool RESCALE>
+__global__ void __launch_bounds__(512, 4) k_moddown_cols(DevTables T, ModDownJobs L, ConvGrid g) {
+    using G = ConvCols<LOGN>;
+    __shared__ ConvLds<LOGN> S;
+    const uint32_t item = xcd_item(g.chunk);
+    if (item >= g.items) return;
+    const uint32_t u = item / G::TPL, z = g.tg.div(u);
+    const int tg = (int)(u - z * g.tg.d);
+    const ModDownJob J = L.dev ? get_job(L, (int)z) : get_inline(L, (int)z);
+    const int nl = __builtin_amdgcn_readfirstlane(J.level) + 1, l = nl - 1;
+    const int ntarget = RESCALE ? l : nl;
+    // targets tg, tg + TG, ..: the 64-bit ones come last and are dealt out evenly
+    const int TG = (int)g.tg.d, k1 = (ntarget - tg + TG - 1) / TG;
+    if (k1 <= 0) return;
+    const uint32_t tid = threadIdx.x;
+    const uint32_t col0 = (item % G::TPL) * G::CC;
+    const uint32_t c_at = G::c_row(tid) * G::N2 + col0 + G::c_col(tid);
+    const int c_tgt = __builtin_amdgcn_readfirstlane(G::c_tgt(tid));
+    const int n_tgt = __builtin_amdgcn_readfirstlane(G::n_tgt(tid));
+    Half2 x[G::CPT][KK];
+    uint64_t top[G::CPT];
+    {
+        uint64_t v[KK][G::CPT];
+#pragma unroll
+        for (int i = 0; i < KK; ++i) {
+            const uint64_t* src = J.t + (size_t)i * G::N + c_at;
+            if constexpr (G::CPT == 2) {
+                const u64x2 w = ld2(src);
+                v[i][0] = w.x, v[i][1] = w.y;
+            } else {
+                v[i][0] = gp(src)[0];
+            }
+        }
+        if constexpr (RESCALE) {
+#pragma unroll
+            for (int c = 0; c < G::CPT; ++c) top[c] = gp(J.top_acc)[c_at + c];
+        }
+#pragma unroll
+        for (int i = 0; i < KK; ++i)
+#pragma unroll
+            for (int c = 0; c < G::CPT; ++c) x[c][i] = split30(v[i][c]);
+    }
+    const uint64_t* M = T.moddown_mat;
+    uint64_t half = 0;
+    if constexpr (RESCALE) {
+        const PrimeInfo Pl = cld(T.primes + l);
+        const ShoupConst pl = cld(T.pinv + l);
+        const MatRow<KK> row = cld(reinterpret_cast<const MatRow<KK>*>(M + (size_t)l * KK));
+        half = Pl.p >> 1;
+#pragma unroll
+        for (int c = 0; c < G::CPT; ++c) {
+            uint64_t lo, hi;
+            conv_acc<KK>(x[c], row, lo, hi);
+            top[c] = submod(top[c], mul_shoup(reduce128(lo, hi, Pl), pl.w, pl.wp, Pl.p), Pl.p);
+        }
+    }
+    int buf = 0;
+    const int s_tgt = __builtin_amdgcn_readfirstlane((int)(tid / G::N1)), s_row = (int)(tid % G::N1);
+    auto s_pid = [&](int k) { const int i = k + s_tgt < k1 ? k + s_tgt : k1 - 1; return i * TG + tg; };
+    ConvTw tw;
+    tw.load(T, s_pid(0), s_row);
+    for (int k = 0; k < k1; k += G::TB, buf ^= 1) {
+#pragma unroll
+        for (int q = 0; q < G::TPT; ++q) {
+            const int i = c_tgt + q, pid = (k + i) * TG + tg;
+            if (k + i >= k1) continue;
+            const PrimeInfo P = cld(T.primes + pid);
+            const MatRow<KK> row = cld(reinterpret_cast<const MatRow<KK>*>(M + (size_t)pid * KK));
+#pragma unroll
+            for (int c = 0; c < G::CPT; ++c) {
+                uint64_t lo, hi;
+                conv_acc<KK>(x[c], row, lo, hi);
+                uint64_t word;
+                if constexpr (RESCALE) {
+                    const ShoupConst pi = cld(T.pinv + pid);
+                    uint64_t sw = reduce64(top[c], P);  // centered lift of top into q_i
+                    if (top[c] > half) sw = submod(sw, cld(T.qlmodq + (size_t)l * (T.L + 1) + pid), P.p);
+                    const uint64_t y = reduce128_lazy(lo, hi, P);
+                    if (is_fp(T, pid)) {
+                        const FpArith ar(P);
+                        word = FpArith::pack(ar.scale_add(ar.from_lazy(y), pi, sw));
+                    } else {
+                        const IntArith ar(P);
+                        word = ar.scale_add(ar.from_lazy(y), pi, sw);
+                    }
+                } else {
+                    word = conv_word(T, pid, P, lo, hi);
+                }
+                S.tile[buf][i][G::c_col(tid) + c][lds_off(G::c_row(tid))] = word;
+            }
+        }
+        tw.put(S, buf, s_tgt, s_row);
+        if (k + G::TB < k1) tw.load(T, s_pid(k + G::TB), s_row);
+        __syncthreads();
+        if (k + n_tgt < k1) conv_columns(T, (k + n_tgt) * TG + tg, S, buf, n_tgt);
+        __syncthreads();
+        conv_store(S, buf, col0, [&](int i) -> uint64_t* {
+            return k + i < k1 ? J.y + (size_t)((k + i) * TG + tg) * G::N : nullptr;
+        });
+    }
+}
+
+template <int LOGN, int KK>
+static void moddown_cols(const DevTables& T, const ModDownJobs& L, int targets, bool rescale, hipStream_t s) {
+    using G = ConvCols<LOGN>;
+    const int tg = fused_groups((size_t)G::TPL * L.n, targets, G::TB);
+    const size_t items = (size_t)L.n * tg * G::TPL;
+    const XcdGrid x = xcd_grid(items, G::TPL);
+    const ConvGrid g{(uint32_t)items, x.chunk, FastDiv(tg, items), FastDiv(1, items)};
+    if (rescale)
+        hipLaunchKernelGGL((k_moddown_cols<LOGN, KK, true>), x.grid, dim3(G::NT), 0, s, T, L, g);
+    else
+        hipLaunchKernelGGL((k_moddown_cols<LOGN, KK, false>), x.grid, dim3(G::NT), 0, s, T, L, g);
+}
+
+template <int LOGN>
+static hipError_t moddown_cols_k(const DevTables& T, const ModDownJobs& L, int targets, bool rescale, hipStream_t s) {
+    switch (T.K) {  // the template bound the matrix rows are padded to
+        case 1: moddown_cols<LOGN, 1>(T, L, targets, rescale, s); break;
+        case 2: moddown_cols<LOGN, 2>(T, L, targets, rescale, s); break;
+        case 3: moddown_cols<LOGN, 3>(T, L, targets, rescale, s); break;
+        case 4: moddown_cols<LOGN, 4>(T, L, targets, rescale, s); break;
+        case 5: moddown_cols<LOGN, 5>(T, L, targets, rescale, s); break;
+        case 6: moddown_cols<LOGN, 6>(T, L, targets, rescale, s); break;
+        case 7: moddown_cols<LOGN, 7>(T, L, targets, rescale, s); break;
+        case 8: moddown_cols<LOGN, 8>(T, L, targets, rescale, s); break;
+        case 9: moddown_cols<LOGN, 9>(T, L, targets, rescale, s); break;
+        default: moddown_cols<LOGN, 10>(T, L, targets, rescale, s); break;
+    }
+    return hipGetLastError();
+}
+
+hipError_t launch_moddown_cols(const DevTables& T, const ModDownJobs& L, int max_nl, bool rescale, hipStream_t s) {
+    if (L.n <= 0) return hipSuccess;
+    if (!fused_ok(T)) return hipErrorInvalidValue;
+    const int targets = rescale ? max_nl - 1 : max_nl;
+    if (targets <= 0) return hipErrorInvalidValue;
+    switch (T.logN) {
+        case 12: return moddown_cols_k<12>(T, L, targets, rescale, s);
+        case 13: return moddown_cols_k<13>(T, L, targets, rescale, s);
+        case 14: return moddown_cols_k<14>(T, L, targets, rescale, s);
+        case 15: return moddown_cols_k<15>(T, L, targets, rescale, s);
+        case 16: return moddown_cols_k<16>(T, L, targets, rescale, s);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+}  // namespace fides

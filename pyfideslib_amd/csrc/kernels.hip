@@ -8,28 +8,11 @@
 // than 8 products are reduced in chunks of 8).
 #include <cstdlib>
 
-#include "engine.hpp"
+#include "conv.hpp"
 
 namespace fides {
 
 constexpr int EW_BLOCK = 256;
-
-__device__ __forceinline__ int num_digits(const DevTables& T, int nl) {
-    const int n = (nl + T.alpha - 1) / T.alpha;
-    return n < T.dnum ? n : T.dnum;
-}
-
-// Two adjacent coefficients per thread through 16-byte accesses.
-struct u64x2 {
-    uint64_t x, y;
-};
-typedef uint64_t v2u64 __attribute__((ext_vector_type(2)));
-typedef __attribute__((address_space(1))) v2u64 gv2u64;
-__device__ __forceinline__ u64x2 ld2(const uint64_t* p) {
-    const v2u64 v = *(const gv2u64*)p;
-    return u64x2{v.x, v.y};
-}
-__device__ __forceinline__ void st2(uint64_t* p, uint64_t a, uint64_t b) { *(gv2u64*)p = v2u64{a, b}; }
 
 // (c0,c1) x (d0,d1) -> (c0d0, c0d1 + c1d0, c1d1)
 // FIDESlib ElemenwiseBatchKernels.cu:1398-1438 binomialMult_.
@@ -73,48 +56,11 @@ constexpr int CV_B = 256;
 constexpr int CV_MAXT = 96;  // positions per polynomial (L+1+K <= 96, checked at context creation)
 constexpr int CV_MIN_BLOCKS = 2048;
 
-// Carry-free sum of products: residues (< 2^60) are split into 30-bit halves,
-// so every partial product is below 2^60 and up to 16 terms accumulate in four
-// 64-bit registers with one v_mad_u64_u32 each and no carry handling;
-// combine() forms the exact 128-bit sum once.
-struct Acc4 {
-    uint64_t s00 = 0, s01 = 0, s10 = 0, s11 = 0;
-};
-struct Half2 {
-    uint32_t lo, hi;  // x = hi * 2^30 + lo
-};
-__device__ __forceinline__ Half2 split30(uint64_t x) { return Half2{(uint32_t)(x & 0x3fffffffu), (uint32_t)(x >> 30)}; }
-__device__ __forceinline__ void mac_split(Acc4& a, Half2 x, Half2 y) {
-    a.s00 = (uint64_t)x.lo * y.lo + a.s00;
-    a.s01 = (uint64_t)x.lo * y.hi + a.s01;
-    a.s10 = (uint64_t)x.hi * y.lo + a.s10;
-    a.s11 = (uint64_t)x.hi * y.hi + a.s11;
-}
-// X = s11 2^60 + (s01 + s10) 2^30 + s00 as (lo, hi)
-__device__ __forceinline__ void combine(const Acc4& a, uint64_t& lo, uint64_t& hi) {
-    lo = a.s00;
-    hi = 0;
-    uint64_t t = a.s01 << 30;
-    lo += t;
-    hi += (a.s01 >> 34) + (lo < t);
-    t = a.s10 << 30;
-    lo += t;
-    hi += (a.s10 >> 34) + (lo < t);
-    t = a.s11 << 60;
-    lo += t;
-    hi += (a.s11 >> 4) + (lo < t);
-}
-
 // Sum over i < n (n <= A, wave-uniform) of x_i * m[i * stride], reduced mod
 // P.  The matrix column is read with scalar loads (uniform addresses).  ONE:
 // the host proved the exact sum fits one Barrett reduction, so split 30-bit
 // products accumulate carry-free; otherwise 128-bit MACs are reduced every 8
 // terms.
-
-template <int A>
-struct MatRow {
-    uint64_t v[A];
-};
 
 // Exact 128-bit MACs of terms [C0, A) in chunks of at most 8 (16 scalar
 // registers of matrix at a time), reduced between chunks: 8 products of a

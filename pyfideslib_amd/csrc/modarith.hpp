@@ -67,6 +67,13 @@ __device__ __forceinline__ uint64_t reduce128(uint64_t lo, uint64_t hi, const Pr
     return r >= P.p ? r - P.p : r;
 }
 
+// The same before its last subtractions: in [0, 3p).
+__device__ __forceinline__ uint64_t reduce128_lazy(uint64_t lo, uint64_t hi, const PrimeInfo& P) {
+    const uint32_t s = P.nbits - 1;
+    const uint64_t xs = (lo >> s) | (hi << (64 - s));
+    return lo - mulhi64(xs, P.mu) * P.p;
+}
+
 // Reduce a single 64-bit value (< 2^64) modulo p.
 __device__ __forceinline__ uint64_t reduce64(uint64_t x, const PrimeInfo& P) { return reduce128(x, 0, P); }
 
@@ -78,13 +85,21 @@ __device__ __forceinline__ uint64_t mulmod(uint64_t a, uint64_t b, const PrimeIn
 
 // Shoup: x * w mod p with x < 2^64, w < p; lazy result in [0, 2p).
 __device__ __forceinline__ uint64_t mul_shoup_lazy(uint64_t x, uint64_t w, uint64_t wp, uint64_t p) {
-    const uint64_t q = mulhi64(x, wp);
-    return x * w - q * p;
+    // x w + q (-p): both low products accumulate into one pair of registers
+    const uint64_t q = mulhi64(x, wp), n = 0 - p;
+    const uint32_t x0 = (uint32_t)x, x1 = (uint32_t)(x >> 32), w0 = (uint32_t)w, w1 = (uint32_t)(w >> 32);
+    const uint32_t q0 = (uint32_t)q, q1 = (uint32_t)(q >> 32), n0 = (uint32_t)n, n1 = (uint32_t)(n >> 32);
+    const uint64_t t = (uint64_t)q0 * n0 + (uint64_t)x0 * w0;
+    const uint32_t h = (uint32_t)(t >> 32) + x0 * w1 + x1 * w0 + q0 * n1 + q1 * n0;
+    return ((uint64_t)h << 32) | (uint32_t)t;
 }
 __device__ __forceinline__ uint64_t mul_shoup(uint64_t x, uint64_t w, uint64_t wp, uint64_t p) {
     const uint64_t r = mul_shoup_lazy(x, w, wp, p);
     return r >= p ? r - p : r;
 }
+
+// x or x - m, whichever is in [0, m) for x < 2m
+__device__ __forceinline__ uint64_t csub(uint64_t x, uint64_t m) { return x >= m ? x - m : x; }
 
 __device__ __forceinline__ uint64_t addmod(uint64_t a, uint64_t b, uint64_t p) {
     const uint64_t s = a + b;

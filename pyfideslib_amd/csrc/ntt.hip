@@ -371,21 +371,23 @@ static void cols_dispatch(const DevTables& T, const NttJobs& L, int limbs, int l
 }
 
 template <int LOGN>
-static hipError_t fwd_impl(const DevTables& T, const NttJobs& L, int limbs, int load, int store, hipStream_t s) {
+static hipError_t fwd_impl(const DevTables& T, const NttJobs& L, int limbs, int load, int store, hipStream_t s,
+                           int passes) {
     const NttPick pk = ntt_pick(true, LOGN, limbs);
-    cols_dispatch<LOGN, true>(T, L, limbs, load, pk, s);
+    if (passes & NTT_PASS1) cols_dispatch<LOGN, true>(T, L, limbs, load, pk, s);
     hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
+    if (e != hipSuccess || !(passes & NTT_PASS2)) return e;
     by_width(pk.rr, [&](auto wr) { fwd_rows<LOGN, decltype(wr)::value>(T, L, limbs, store, s); });
     return hipGetLastError();
 }
 
 template <int LOGN>
-static hipError_t inv_impl(const DevTables& T, const NttJobs& L, int limbs, hipStream_t s) {
+static hipError_t inv_impl(const DevTables& T, const NttJobs& L, int limbs, hipStream_t s, int passes) {
     const NttPick pk = ntt_pick(false, LOGN, limbs);
-    by_width(pk.rr, [&](auto wr) { inv_rows<LOGN, decltype(wr)::value>(T, L, limbs, s); });
+    if (passes & NTT_PASS1)
+        by_width(pk.rr, [&](auto wr) { inv_rows<LOGN, decltype(wr)::value>(T, L, limbs, s); });
     hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
+    if (e != hipSuccess || !(passes & NTT_PASS2)) return e;
     cols_dispatch<LOGN, false>(T, L, limbs, 0, pk, s);
     return hipGetLastError();
 }
@@ -395,32 +397,33 @@ hipError_t launch_fp_twiddles(const DevTables& T, const ShoupConst* tw, double* 
     return hipGetLastError();
 }
 
-hipError_t launch_ntt_fwd(const DevTables& T, const NttJobs& L, int limbs, int load, int store, hipStream_t s) {
+hipError_t launch_ntt_fwd(const DevTables& T, const NttJobs& L, int limbs, int load, int store, hipStream_t s,
+                          int passes) {
     if (limbs <= 0) return hipSuccess;
     switch (T.logN) {
-        case 10: return fwd_impl<10>(T, L, limbs, load, store, s);
-        case 11: return fwd_impl<11>(T, L, limbs, load, store, s);
-        case 12: return fwd_impl<12>(T, L, limbs, load, store, s);
-        case 13: return fwd_impl<13>(T, L, limbs, load, store, s);
-        case 14: return fwd_impl<14>(T, L, limbs, load, store, s);
-        case 15: return fwd_impl<15>(T, L, limbs, load, store, s);
-        case 16: return fwd_impl<16>(T, L, limbs, load, store, s);
-        case 17: return fwd_impl<17>(T, L, limbs, load, store, s);
+        case 10: return fwd_impl<10>(T, L, limbs, load, store, s, passes);
+        case 11: return fwd_impl<11>(T, L, limbs, load, store, s, passes);
+        case 12: return fwd_impl<12>(T, L, limbs, load, store, s, passes);
+        case 13: return fwd_impl<13>(T, L, limbs, load, store, s, passes);
+        case 14: return fwd_impl<14>(T, L, limbs, load, store, s, passes);
+        case 15: return fwd_impl<15>(T, L, limbs, load, store, s, passes);
+        case 16: return fwd_impl<16>(T, L, limbs, load, store, s, passes);
+        case 17: return fwd_impl<17>(T, L, limbs, load, store, s, passes);
         default: return hipErrorInvalidValue;
     }
 }
 
-hipError_t launch_ntt_inv(const DevTables& T, const NttJobs& L, int limbs, hipStream_t s) {
+hipError_t launch_ntt_inv(const DevTables& T, const NttJobs& L, int limbs, hipStream_t s, int passes) {
     if (limbs <= 0) return hipSuccess;
     switch (T.logN) {
-        case 10: return inv_impl<10>(T, L, limbs, s);
-        case 11: return inv_impl<11>(T, L, limbs, s);
-        case 12: return inv_impl<12>(T, L, limbs, s);
-        case 13: return inv_impl<13>(T, L, limbs, s);
-        case 14: return inv_impl<14>(T, L, limbs, s);
-        case 15: return inv_impl<15>(T, L, limbs, s);
-        case 16: return inv_impl<16>(T, L, limbs, s);
-        case 17: return inv_impl<17>(T, L, limbs, s);
+        case 10: return inv_impl<10>(T, L, limbs, s, passes);
+        case 11: return inv_impl<11>(T, L, limbs, s, passes);
+        case 12: return inv_impl<12>(T, L, limbs, s, passes);
+        case 13: return inv_impl<13>(T, L, limbs, s, passes);
+        case 14: return inv_impl<14>(T, L, limbs, s, passes);
+        case 15: return inv_impl<15>(T, L, limbs, s, passes);
+        case 16: return inv_impl<16>(T, L, limbs, s, passes);
+        case 17: return inv_impl<17>(T, L, limbs, s, passes);
         default: return hipErrorInvalidValue;
     }
 }

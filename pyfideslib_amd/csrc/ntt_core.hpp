@@ -34,10 +34,11 @@ struct IntArith {
     __device__ __forceinline__ V from(uint64_t x) const { return x; }
     static __device__ __forceinline__ V unpack(uint64_t m) { return m; }
     static __device__ __forceinline__ uint64_t pack(V v) { return v; }
-    // inputs in [0, 4p), outputs in [0, 4p)
+    // every stage adds 2p to the bound; U is brought below 8p where FpArith
+    // reduces, so four stages stay below 16p < 2^64 (any 64-bit b will do)
     template <bool RED>
     __device__ __forceinline__ void fwd_bf(V& a, V& b, const W& w) const {
-        const uint64_t U = a >= 2 * p ? a - 2 * p : a;
+        const uint64_t U = RED ? csub(a, 8 * p) : a;
         const uint64_t X = mul_shoup_lazy(b, w.w, w.wp, p);
         a = U + X;
         b = U - X + 2 * p;
@@ -54,22 +55,50 @@ struct IntArith {
         a = mul_shoup_lazy(U + X, s.w, s.wp, p);
         b = mul_shoup_lazy(U - X + 2 * p, ws.w, ws.wp, p);
     }
-    // the residue of a forward output in [0, 4p), of an inverse one in [0, 2p)
-    __device__ __forceinline__ uint64_t canon_fwd(V x) const {
-        x = x >= 2 * p ? x - 2 * p : x;
-        return x >= p ? x - p : x;
+    // the residue of a forward output in [0, 16p), of an inverse one in [0, 2p)
+    __device__ __forceinline__ uint64_t canon_fwd(V x) const { return csub(term_fwd(x), p); }
+    __device__ __forceinline__ uint64_t canon_inv(V x) const { return csub(x, p); }
+    // a b, a b + c d as residues; a value below 3p from reduce128_lazy
+    __device__ __forceinline__ uint64_t mul(uint64_t a, uint64_t b, const PrimeInfo& P) const { return mulmod(a, b, P); }
+    __device__ __forceinline__ uint64_t mul2(uint64_t a, uint64_t b, uint64_t c, uint64_t d,
+                                             const PrimeInfo& P) const {
+        uint64_t lo, hi;
+        mul128(a, b, lo, hi);
+        mac128(lo, hi, c, d);
+        return reduce128(lo, hi, P);
     }
-    __device__ __forceinline__ uint64_t canon_inv(V x) const { return x >= p ? x - p : x; }
+    __device__ __forceinline__ V from_lazy(uint64_t x) const {
+        return csub(csub(x, 2 * p), p);
+    }
+    // a forward output as an inner product's term, in [0, 2p)
+    __device__ __forceinline__ V term_fwd(V x) const { return csub(csub(csub(x, 8 * p), 4 * p), 2 * p); }
+    // sum of at most 4 products x k with x < 2p, k < p (below 8p^2 < 2^(bits(p) +
+    // 63), one reduction), as an inverse transform's input
+    struct Sum {
+        uint64_t lo = 0, hi = 0;
+    };
+    __device__ __forceinline__ void mac(Sum& s, V x, uint64_t k) const { mac128(s.lo, s.hi, x, k); }
+    __device__ __forceinline__ V sum(const Sum& s, const PrimeInfo& P) const { return reduce128(s.lo, s.hi, P); }
+    // the residue of an inverse transform's input
+    __device__ __forceinline__ uint64_t canon_in(V x) const { return x; }
+    // e c + f as an inverse transform's input
+    __device__ __forceinline__ V mul_add(V e, const ShoupConst& c, uint64_t f) const {
+        return addmod(mul_shoup(e, c.w, c.wp, p), f, p);
+    }
+    // y c + s for a conversion's sum y (from_lazy) and a residue s, as a forward input
+    __device__ __forceinline__ V scale_add(V y, const ShoupConst& c, uint64_t s) const {
+        return addmod(mul_shoup(y, c.w, c.wp, p), s, p);
+    }
     // (e - v) c,  (e - v) c + f,  (e c + f - v) d  for residues e, f, c, d
     __device__ __forceinline__ uint64_t sub_mul(uint64_t e, V v, const ShoupConst& c) const {
-        return mul_shoup(submod(e, canon_fwd(v), p), c.w, c.wp, p);
+        return mul_shoup(e + 8 * p - csub(v, 8 * p), c.w, c.wp, p);
     }
     __device__ __forceinline__ uint64_t sub_mul_add(uint64_t e, V v, const ShoupConst& c, uint64_t f) const {
         return addmod(sub_mul(e, v, c), f, p);
     }
     __device__ __forceinline__ uint64_t mul_add_sub_mul(uint64_t e, const ShoupConst& c, uint64_t f, V v,
                                                         const ShoupConst& d) const {
-        return mul_shoup(submod(addmod(mul_shoup(e, c.w, c.wp, p), f, p), canon_fwd(v), p), d.w, d.wp, p);
+        return mul_shoup(mul_shoup_lazy(e, c.w, c.wp, p) + f + 8 * p - csub(v, 8 * p), d.w, d.wp, p);
     }
 };
 struct FpArith {
@@ -103,6 +132,26 @@ struct FpArith {
     }
     __device__ __forceinline__ uint64_t canon_fwd(V x) const { return fp_canon(x, p, pinv); }
     __device__ __forceinline__ uint64_t canon_inv(V x) const { return fp_canon(x, p, pinv); }
+    __device__ __forceinline__ uint64_t mul(uint64_t a, uint64_t b, const PrimeInfo&) const {
+        return fp_canon(fp_mul(fp_from(a), fp_from(b), p, pinv), p, pinv);
+    }
+    __device__ __forceinline__ uint64_t mul2(uint64_t a, uint64_t b, uint64_t c, uint64_t d, const PrimeInfo&) const {
+        return fp_canon(fp_mul(fp_from(a), fp_from(b), p, pinv) + fp_mul(fp_from(c), fp_from(d), p, pinv), p, pinv);
+    }
+    __device__ __forceinline__ V from_lazy(uint64_t x) const { return fp_from(x); }  // 3p < 2^52
+    __device__ __forceinline__ V term_fwd(V x) const { return fp_reduce(x, p, pinv); }
+    // |x| <= p, k < p: each product at most (1/2 + 3/8) p, four of them below 4p
+    using Sum = double;
+    __device__ __forceinline__ void mac(Sum& s, V x, uint64_t k) const { s += fp_mul(x, fp_from(k), p, pinv); }
+    __device__ __forceinline__ V sum(Sum s, const PrimeInfo&) const { return fp_reduce(s, p, pinv); }
+    __device__ __forceinline__ uint64_t canon_in(V x) const { return fp_to(x < 0 ? x + p : x); }  // reduced before
+    __device__ __forceinline__ V mul_add(V e, const ShoupConst& c, uint64_t f) const {
+        return fp_reduce(fp_mul(e, fp_from(c.w), p, pinv) + fp_from(f), p, pinv);
+    }
+    // at most (1/2 + 9/8 + 1) p, a first phase's bound
+    __device__ __forceinline__ V scale_add(V y, const ShoupConst& c, uint64_t s) const {
+        return fp_mul(y, fp_from(c.w), p, pinv) + fp_from(s);
+    }
     // uncentered constants: fp_mul of a value B returns at most 1/2 + 3B/8; no sum below exceeds 7.1
     __device__ __forceinline__ uint64_t sub_mul(uint64_t e, V v, const ShoupConst& c) const {
         return fp_canon(fp_mul(fp_from(e) - v, fp_from(c.w), p, pinv), p, pinv);
@@ -436,7 +485,7 @@ struct Epilogue {
 // The limb scale of an inverse transform: N^-1, times a base-conversion factor.
 __device__ __forceinline__ const ShoupConst* inv_scale(const DevTables& T, const NttJob& J, int pos, int pid) {
     if (J.scale_sel == ISCALE_MODUP) return T.iscale_modup + ((size_t)J.level * (T.L + 1) + pos) * 2;
-    if (J.scale_sel == ISCALE_MODDOWN) return T.iscale_moddown + (size_t)(pos - J.nq) * 2;
+    if (J.scale_sel == ISCALE_MODDOWN && pos >= J.nq) return T.iscale_moddown + (size_t)(pos - J.nq) * 2;
     return T.iscale_plain + (size_t)pid * 2;
 }
 
