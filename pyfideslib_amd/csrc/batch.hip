@@ -38,6 +38,7 @@ struct BatchPlan {
     int n_mult = 0, max_nl = 0, max_nd = 0, max_npos = 0;
     int n = 0;
     NttStage intt_up, ntt_ext, intt_sp;
+    NttStage intt_rot;  // fused: the sources whose first pass no tensor kernel runs
     NttStage md_rescale, md_plain, md_auto;  // ModDown NTTs by epilogue
     const ModUpJob* modup = nullptr;
     const KskJob* ksk = nullptr;
@@ -48,6 +49,7 @@ struct BatchPlan {
     const int* ksk_chunks = nullptr;
     int n_ksk_chunks = 0;
     bool keystat = false;  // at least two jobs per key on average
+    bool fused = false;    // fused.hip's kernels (fused_ok)
 };
 
 // Key-stationary KSK for single-key batches (FIDES_KSK_KEYSTAT=0 turns it off).
@@ -91,13 +93,14 @@ static std::shared_ptr<BatchPlan> build_plan(Context& c, const std::vector<KsIte
     P->n = (int)items.size();
     const size_t N = c.N;
     const int K = c.K;
-    // scratch layout per item: [d2 (mult)], t, ext, acc_a, acc_b, tk(2K), y(2nl), [top(4) (rescale)]
+    P->fused = fused_ok(c.T);
+    // scratch layout per item: [d2 (mult)], t, ext, acc_a, acc_b, tk(2K + 2), y(2nl), [top(4) (rescale)]
     std::vector<size_t> off(P->n + 1, 0);
     for (int i = 0; i < P->n; ++i) {
         const KsItem& it = items[i];
         const int l = item_level(it);
         const size_t nl = l + 1, npos = nl + K, nd = c.num_digits(l);
-        const size_t words = (it.mult ? nl : 0) + nl + nd * npos + 2 * npos + 2 * K + 2 * nl + (it.rescale ? 4 : 0);
+        const size_t words = (it.mult ? nl : 0) + nl + nd * npos + 2 * npos + 2 * K + 2 + 2 * nl + (it.rescale ? 4 : 0);
         off[i + 1] = off[i] + words * N;
         P->max_nl = std::max(P->max_nl, (int)nl);
         P->max_nd = std::max(P->max_nd, (int)nd);
@@ -106,7 +109,7 @@ static std::shared_ptr<BatchPlan> build_plan(Context& c, const std::vector<KsIte
     uint64_t* base = c.batch_arena(off[P->n]);
 
     std::vector<TensorJob> tj;
-    std::vector<NttJob> iu, ne, isp, nmd_r, nmd_p, nmd_a;
+    std::vector<NttJob> iu, ir, ne, isp, nmd_r, nmd_p, nmd_a;
     std::vector<ModUpJob> mu;
     std::vector<KskJob> kj;
     std::vector<ModDownJob> md_r, md_p;
@@ -120,17 +123,18 @@ static std::shared_ptr<BatchPlan> build_plan(Context& c, const std::vector<KsIte
         uint64_t* acc_a = ext + (size_t)nd * npos * N;
         uint64_t* acc_b = acc_a + npos * N;
         uint64_t* tk = acc_b + npos * N;
-        uint64_t* y = tk + 2 * K * N;
+        uint64_t* y = tk + (2 * K + 2) * N;
         uint64_t* top = y + 2 * nl * N;
         Ciphertext& O = *it.out;
         // the key-switch input: c1 d1 (mult, from the tensor) or c1 (rotation)
         const uint64_t* x = it.mult ? d2 : it.a->c1();
         if (it.mult)
-            tj.push_back(TensorJob{it.a->c0(), it.a->c1(), it.b->c0(), it.b->c1(), O.c0(), O.c1(), d2, nl});
+            tj.push_back(TensorJob{it.a->c0(), it.a->c1(), it.b->c0(), it.b->c1(), O.c0(), O.c1(), d2, nl, 0, t});
         NttJob j{};
         j.src = x; j.mid = t; j.dst = t; j.npos = nl; j.nq = nl; j.q0 = 0;
         j.level = l; j.scale_sel = ISCALE_MODUP;
         iu.push_back(j);
+        if (!it.mult) ir.push_back(j);
         mu.push_back(ModUpJob{t, ext, l});
         for (int d = 0; d < nd; ++d) {
             NttJob e{};
@@ -140,41 +144,57 @@ static std::shared_ptr<BatchPlan> build_plan(Context& c, const std::vector<KsIte
             e.skip_hi = d * c.alpha + c.digit_size(d, l);
             ne.push_back(e);
         }
-        kj.push_back(KskJob{ext, x, it.key->a.ptr, it.key->b.ptr, acc_a, acc_b, l});
+        // fused: per part [dropped limb][K special limbs], as KskJob states
+        uint64_t* down[2] = {tk, tk + (size_t)(K + 1) * N};
+        const bool rs = it.mult && it.rescale;
+        if (P->fused)
+            kj.push_back(KskJob{ext, x, it.key->a.ptr, it.key->b.ptr, acc_a, acc_b, l, 0, down[0], down[1],
+                                rs ? O.c1() : nullptr, rs ? O.c0() : nullptr});
+        else
+            kj.push_back(KskJob{ext, x, it.key->a.ptr, it.key->b.ptr, acc_a, acc_b, l, 0, nullptr, nullptr, nullptr,
+                                nullptr});
         // h = 0: a-part -> c1, h = 1: b-part -> c0 (ckks.hip ksk_moddown / ksk_moddown_rescale)
         for (int h = 0; h < 2; ++h) {
             uint64_t* acc = h ? acc_b : acc_a;
-            uint64_t* tkh = tk + (size_t)h * K * N;
+            uint64_t* tkh = P->fused ? down[h] + N : tk + (size_t)h * K * N;
             uint64_t* yh = y + (size_t)h * nl * N;
             uint64_t* out = h ? O.c0() : O.c1();
             NttJob a{};
             a.src = acc + nl * N; a.mid = tkh; a.dst = tkh; a.npos = K; a.nq = 0; a.q0 = 0;
             a.scale_sel = ISCALE_MODDOWN;
+            if (P->fused) {  // second pass only, in place
+                a.src = a.mid = a.dst = tkh;
+                if (rs) {
+                    a.src = a.mid = a.dst = down[h];
+                    a.npos = K + 1; a.nq = 1; a.q0 = l;
+                }
+            }
             isp.push_back(a);
             NttJob f{};
             f.src = yh; f.mid = yh; f.dst = out; f.aux = acc; f.q0 = 0;
             if (it.mult && it.rescale) {
                 f.add = out;  // the tensor terms (c0 d0, c0 d1 + c1 d0), in place
-                for (int w = 0; w < 2; ++w) {  // top limbs of the accumulator and of the addend
+                for (int w = 0; w < 2 && !P->fused; ++w) {  // top limbs of the accumulator and of the addend
                     NttJob t1{};
                     t1.src = (w ? out : acc) + (size_t)l * N;
                     t1.mid = t1.dst = top + (size_t)(h + 2 * w) * N;
                     t1.npos = 1; t1.nq = 1; t1.q0 = l;
                     isp.push_back(t1);
                 }
-                md_r.push_back(ModDownJob{tkh, yh, top + (size_t)h * N, top + (size_t)(h + 2) * N, l});
+                md_r.push_back(P->fused ? ModDownJob{tkh, yh, down[h], nullptr, l, 0}
+                                        : ModDownJob{tkh, yh, top + (size_t)h * N, top + (size_t)(h + 2) * N, l, 0});
                 f.npos = l; f.nq = l; f.level = l;
                 nmd_r.push_back(f);
             } else if (it.mult) {
                 f.add = out;
-                md_p.push_back(ModDownJob{tkh, yh, nullptr, nullptr, l});
+                md_p.push_back(ModDownJob{tkh, yh, nullptr, nullptr, l, 0});
                 f.npos = nl; f.nq = nl;
                 nmd_p.push_back(f);
             } else {
                 // rotation: ModDown, + c0 (b part), then the automorphism on the way out
                 f.add = h ? it.a->c0() : nullptr;
                 f.autok = it.kinv;
-                md_p.push_back(ModDownJob{tkh, yh, nullptr, nullptr, l});
+                md_p.push_back(ModDownJob{tkh, yh, nullptr, nullptr, l, 0});
                 f.npos = nl; f.nq = nl;
                 nmd_a.push_back(f);
             }
@@ -196,6 +216,7 @@ static std::shared_ptr<BatchPlan> build_plan(Context& c, const std::vector<KsIte
     P->keystat = !kj.empty() && 2 * nkeys <= (int)kj.size();
     int tot;
     std::vector<int> m_iu = limbmap_of(iu, tot); P->intt_up.limbs = tot;
+    std::vector<int> m_ir = limbmap_of(ir, tot); P->intt_rot.limbs = tot;
     std::vector<int> m_ne = limbmap_of(ne, tot); P->ntt_ext.limbs = tot;
     std::vector<int> m_isp = limbmap_of(isp, tot); P->intt_sp.limbs = tot;
     std::vector<int> m_r = limbmap_of(nmd_r, tot); P->md_rescale.limbs = tot;
@@ -212,6 +233,7 @@ static std::shared_ptr<BatchPlan> build_plan(Context& c, const std::vector<KsIte
     };
     const size_t o_tj = append(tj.data(), tj.size() * sizeof(TensorJob));
     const size_t o_iu = append(iu.data(), iu.size() * sizeof(NttJob)), o_miu = append(m_iu.data(), m_iu.size() * 4);
+    const size_t o_ir = append(ir.data(), ir.size() * sizeof(NttJob)), o_mir = append(m_ir.data(), m_ir.size() * 4);
     const size_t o_mu = append(mu.data(), mu.size() * sizeof(ModUpJob));
     const size_t o_ne = append(ne.data(), ne.size() * sizeof(NttJob)), o_mne = append(m_ne.data(), m_ne.size() * 4);
     const size_t o_kj = append(kj.data(), kj.size() * sizeof(KskJob));
@@ -228,6 +250,7 @@ static std::shared_ptr<BatchPlan> build_plan(Context& c, const std::vector<KsIte
     char* d = (char*)P->table.ptr;
     P->tensor = (const TensorJob*)(d + o_tj);
     P->intt_up = {(const NttJob*)(d + o_iu), (const int*)(d + o_miu), (int)iu.size(), P->intt_up.limbs};
+    P->intt_rot = {(const NttJob*)(d + o_ir), (const int*)(d + o_mir), (int)ir.size(), P->intt_rot.limbs};
     P->modup = (const ModUpJob*)(d + o_mu);
     P->ntt_ext = {(const NttJob*)(d + o_ne), (const int*)(d + o_mne), (int)ne.size(), P->ntt_ext.limbs};
     P->ksk = (const KskJob*)(d + o_kj);
@@ -255,7 +278,36 @@ static JL dev_list(const J* jobs, int n, const int* map = nullptr) {
 
 static NttJobs ntt_list(const NttStage& st) { return dev_list<NttJobs>(st.jobs, st.njobs, st.map); }
 
+static void run_plan_fused(Context& c, const BatchPlan& P) {
+    const DevTables& T = c.T;
+    hipStream_t s = c.stream;
+    if (P.n_mult)
+        ckb(launch_tensor_rows(T, dev_list<TensorJobs>(P.tensor, P.n_mult), P.max_nl, s), "batch tensor and rows");
+    if (P.intt_rot.njobs)
+        ckb(launch_ntt_inv(T, ntt_list(P.intt_rot), P.intt_rot.limbs, s, NTT_PASS1), "batch intt rows");
+    ckb(launch_ntt_inv(T, ntt_list(P.intt_up), P.intt_up.limbs, s, NTT_PASS2), "batch intt columns");
+    ckb(launch_modup_cols(T, dev_list<ModUpJobs>(P.modup, P.n), P.max_nd, P.max_nl, s), "batch modup and columns");
+    ckb(launch_rows_ksk(T, dev_list<KskJobs>(P.ksk, P.n), P.max_npos, s), "batch rows and ksk");
+    ckb(launch_ntt_inv(T, ntt_list(P.intt_sp), P.intt_sp.limbs, s, NTT_PASS2), "batch intt sp columns");
+    if (P.n_conv_rescale)
+        ckb(launch_moddown_cols(T, dev_list<ModDownJobs>(P.conv_rescale, P.n_conv_rescale), P.max_nl, true, s),
+            "batch moddown+rescale and columns");
+    if (P.n_conv_plain)
+        ckb(launch_moddown_cols(T, dev_list<ModDownJobs>(P.conv_plain, P.n_conv_plain), P.max_nl, false, s),
+            "batch moddown and columns");
+    const NttStage* md[3] = {&P.md_rescale, &P.md_plain, &P.md_auto};
+    const int store[3] = {STORE_MODDOWN_RESCALE, STORE_MODDOWN, STORE_MODDOWN_AUTO};
+    for (int i = 0; i < 3; ++i)
+        if (md[i]->njobs)
+            ckb(launch_ntt_fwd(T, ntt_list(*md[i]), md[i]->limbs, LOAD_PLAIN, store[i], s, NTT_PASS2),
+                "batch moddown rows");
+}
+
 static void run_plan(Context& c, const BatchPlan& P) {
+    if (P.fused) {
+        run_plan_fused(c, P);
+        return;
+    }
     const DevTables& T = c.T;
     hipStream_t s = c.stream;
     if (P.n_mult) ckb(launch_tensor(T, dev_list<TensorJobs>(P.tensor, P.n_mult), P.max_nl, s), "batch tensor");
@@ -410,6 +462,7 @@ struct HoistPlan {
     }
     DevBuf scratch, table;
     int level = 0, nk = 0, npos = 0;
+    bool fused = false;  // fused.hip's kernels (fused_ok)
     const uint64_t *c0 = nullptr, *c1 = nullptr;
     uint64_t *t = nullptr, *ext = nullptr;
     const KskJob* ksk = nullptr;
@@ -431,8 +484,9 @@ static std::shared_ptr<HoistPlan> build_hoist_plan(Context& c, const Ciphertext&
     int nk = 0;
     for (uint32_t k : ks) nk += (k != 1);
     P->nk = nk;
-    // scratch: t, ext, then per key-switched rotation acc_a, acc_b, tk(2K), y(2nl)
-    const size_t per = 2 * npos + 2 * K + 2 * nl;
+    P->fused = fused_ok(c.T);
+    // scratch: t, ext, then per key-switched rotation acc_a, acc_b, tk(2K + 2), y(2nl)
+    const size_t per = 2 * npos + 2 * K + 2 + 2 * nl;
     P->scratch = DevBuf(&c.pool, (nl + (size_t)nd * npos + per * nk) * N);
     P->t = P->scratch.ptr;
     P->ext = P->t + nl * N;
@@ -453,20 +507,21 @@ static std::shared_ptr<HoistPlan> build_hoist_plan(Context& c, const Ciphertext&
         uint64_t* s = base + per * r * N;
         uint64_t* acc_a = s;
         uint64_t* acc_b = acc_a + npos * N;
-        uint64_t* tka = acc_b + npos * N;
-        uint64_t* tkb = tka + (size_t)K * N;
+        uint64_t* tka = acc_b + npos * N + N;  // one limb before each part: KskJob's layout
+        uint64_t* tkb = tka + (size_t)(K + 1) * N;
         uint64_t* ya = tkb + (size_t)K * N;
         uint64_t* yb = ya + nl * N;
         const uint32_t kinv = c.auto_inverse(ks[i]);
-        kj.push_back(KskJob{P->ext, P->c1, key.a.ptr, key.b.ptr, acc_a, acc_b, l});
+        kj.push_back(KskJob{P->ext, P->c1, key.a.ptr, key.b.ptr, acc_a, acc_b, l, 0, P->fused ? tka - N : nullptr,
+                            P->fused ? tkb - N : nullptr, nullptr, nullptr});
         for (int h = 0; h < 2; ++h) {
             NttJob j{};
-            j.src = (h ? acc_b : acc_a) + nl * N;
             j.mid = j.dst = h ? tkb : tka;
+            j.src = P->fused ? j.dst : (h ? acc_b : acc_a) + nl * N;  // fused: second pass only
             j.npos = K; j.nq = 0; j.q0 = 0;
             j.scale_sel = ISCALE_MODDOWN;
             isp.push_back(j);
-            mdj.push_back(ModDownJob{h ? tkb : tka, h ? yb : ya, nullptr, nullptr, l});
+            mdj.push_back(ModDownJob{h ? tkb : tka, h ? yb : ya, nullptr, nullptr, l, 0});
             NttJob f{};
             f.src = f.mid = h ? yb : ya;
             // ModDown, + c0 (b part) and the automorphism, into the output
@@ -513,7 +568,15 @@ static void run_hoist_plan(Context& c, const HoistPlan& P) {
     const DevTables& T = c.T;
     hipStream_t s = c.stream;
     const int nl = P.level + 1;
-    if (P.nk > 0) {
+    if (P.nk > 0 && P.fused) {
+        modup_half(c, P.level, P.c1, P.t, P.ext);
+        if (P.nk > 1) modup_rows(c, P.level, P.ext);
+        ckb(launch_rows_ksk(T, dev_list<KskJobs>(P.ksk, P.nk), P.npos, s, P.nk > 1), "hoist rows and ksk");
+        ckb(launch_ntt_inv(T, ntt_list(P.intt_sp), P.intt_sp.limbs, s, NTT_PASS2), "hoist intt sp columns");
+        ckb(launch_moddown_cols(T, dev_list<ModDownJobs>(P.moddown, 2 * P.nk), nl, false, s), "hoist moddown columns");
+        ckb(launch_ntt_fwd(T, ntt_list(P.ntt_md), P.ntt_md.limbs, LOAD_PLAIN, STORE_MODDOWN_AUTO, s, NTT_PASS2),
+            "hoist moddown automorph rows");
+    } else if (P.nk > 0) {
         modup_to(c, P.level, P.c1, P.t, P.ext);
         ckb(launch_ksk_inner(T, dev_list<KskJobs>(P.ksk, P.nk), P.npos, s, true), "hoist ksk");
         ckb(launch_ntt_inv(T, ntt_list(P.intt_sp), P.intt_sp.limbs, s), "hoist intt sp");

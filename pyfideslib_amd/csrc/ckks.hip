@@ -212,24 +212,32 @@ void modup_half(Context& c, int level, const uint64_t* x, uint64_t* t, uint64_t*
     modup_cols(c, level, t, ext);
 }
 
-// ModUp of x (evaluation form, level l) into ext (evaluation form; the digit's
-// own positions are left unwritten: consumers read them from x).
-static void modup(Context& c, int level, const uint64_t* x, uint64_t* t, uint64_t* ext) {
-    const int nl = level + 1, npos = nl + c.K, nd = c.num_digits(level);
-    modup_intt(c, level, x, t);
-    ModUpJobs mj = inline_list<ModUpJobs>();
-    mj.inl[0] = ModUpJob{t, ext, level};
-    mj.n = 1;
-    ck(launch_modup_conv(c.T, mj, nd, c.stream), "modup conv");
+// The digits' transforms (the digits' own positions are skipped).
+static void digit_ntts(Context& c, int level, uint64_t* ext, int passes) {
+    const int nl = level + 1, npos = nl + c.K;
     std::vector<NttJob> jobs;
-    for (int d = 0; d < nd; ++d) {
+    for (int d = 0; d < c.num_digits(level); ++d) {
         uint64_t* e = ext + (size_t)d * npos * c.N;
         NttJob j = ntt_job(e, e, e, npos, nl, 0);
         j.skip_lo = d * c.alpha;
         j.skip_hi = d * c.alpha + c.digit_size(d, level);
         jobs.push_back(j);
     }
-    run_ntt(c, jobs, false);
+    run_ntt(c, jobs, false, LOAD_PLAIN, STORE_PLAIN, passes);
+}
+
+void modup_rows(Context& c, int level, uint64_t* ext) { digit_ntts(c, level, ext, NTT_PASS2); }
+
+// ModUp of x (evaluation form, level l) into ext (evaluation form; the digit's
+// own positions are left unwritten: consumers read them from x).
+static void modup(Context& c, int level, const uint64_t* x, uint64_t* t, uint64_t* ext) {
+    const int nd = c.num_digits(level);
+    modup_intt(c, level, x, t);
+    ModUpJobs mj = inline_list<ModUpJobs>();
+    mj.inl[0] = ModUpJob{t, ext, level};
+    mj.n = 1;
+    ck(launch_modup_conv(c.T, mj, nd, c.stream), "modup conv");
+    digit_ntts(c, level, ext, NTT_BOTH);
 }
 
 // The fused form of what follows ModUp: rows + inner product (+ the first pass

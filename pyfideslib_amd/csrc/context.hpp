@@ -402,6 +402,8 @@ void run_ntt_jobs(Context& c, std::vector<NttJob> jobs, bool inverse, int load =
                   int passes = NTT_BOTH);
 // ModUp of x up to what launch_rows_ksk takes (fused_ok).
 void modup_half(Context& c, int level, const uint64_t* x, uint64_t* t, uint64_t* ext);
+// The rest of its transforms, for several keys: ext in evaluation form.
+void modup_rows(Context& c, int level, uint64_t* ext);
 // ModUp of x (level l, evaluation form) into ext via the scaled coefficient limbs t.
 void modup_to(Context& c, int level, const uint64_t* x, uint64_t* t, uint64_t* ext);
 

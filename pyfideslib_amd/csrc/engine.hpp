@@ -373,9 +373,9 @@ hipError_t launch_tensor_rows(const DevTables& T, const TensorJobs& jobs, int ma
 // max_nl: limbs of the list's top level.
 hipError_t launch_modup_cols(const DevTables& T, const ModUpJobs& jobs, int max_nd, int max_nl, hipStream_t stream);
 // Second pass of the digits' transforms and the key-switch inner product
-// (several jobs: sorted by key).  shared: all jobs use the same ext / own / level.
+// (several jobs: sorted by key).  eval: the digits' second pass has been run.
 hipError_t launch_rows_ksk(const DevTables& T, const KskJobs& jobs, int max_npos, hipStream_t stream,
-                           bool shared = false);
+                           bool eval = false);
 // ModDown conversion (+ rescale) and the first pass of its outputs' transform.
 hipError_t launch_moddown_cols(const DevTables& T, const ModDownJobs& jobs, int max_nl, bool rescale,
                                hipStream_t stream);

@@ -150,33 +150,32 @@ __global__ void __launch_bounds__(512, 4) k_modup_cols(DevTables T, ModUpJobs L,
 // positions come from the evaluation-form source), the inner product with both
 // key parts, and the inverse transform's row pass where the limb goes down.
 // Items (job, prime, tile); with several jobs the job runs fastest, so that
-// the jobs of one key (they are sorted by key) read its rows from the XCD's L2.
-// SHARED: one source (job 0's), every job's key against it (a hoisted set),
-// g.per jobs per item.
+// the jobs of one key (they are sorted by key), or of one source, read its rows
+// from the XCD's L2.  EVAL: the digits are in evaluation form already (a hoisted
+// set runs their row pass once for all its keys; doing it per key, or keeping
+// three digits in registers through a loop over the keys, spilled at 128
+// registers and took 348 us for 9 keys at level 17).
 struct KskGrid {
     uint32_t items, chunk;
-    FastDiv np, n;
-    int per, q_primes;  // primes below q_primes are the Q primes of the list's top level
+    FastDiv n;
+    int q_primes;  // primes below q_primes are the Q primes of the list's top level
 };
 
-template <int LOGN, int D, bool SHARED>
+template <int LOGN, bool EVAL>
 __global__ void __launch_bounds__(FRows<LOGN>::NTR, 4) k_rows_ksk(DevTables T, KskJobs L, KskGrid g) {
     using G = FRows<LOGN>;
     constexpr int TPL = G::N1 / G::RR;
     __shared__ uint64_t lds[G::RR * G::SR];
     const uint32_t item = xcd_item(g.chunk);
     if (item >= g.items) return;
-    const uint32_t u = g.n.div(item), z = item - u * g.n.d;  // z: job, or run of jobs (SHARED)
-    const uint32_t w = u / TPL;
-    const int py = (int)w < g.q_primes ? (int)w : T.L + 1 + ((int)w - g.q_primes);  // prime id
+    const uint32_t u = g.n.div(item), z = item - u * g.n.d;
+    const int py = (int)(u / TPL);
+    const int pid = py < g.q_primes ? py : T.L + 1 + (py - g.q_primes);
     const int t = threadIdx.x % G::TR, rr = threadIdx.x / G::TR;
     const uint32_t r = (u % TPL) * G::RR + rr;
     const uint32_t in0 = r * G::N2, x0 = r * G::N2 + G::mem(t, 0);
-    const int j0 = SHARED ? (int)z * g.per : (int)z;
-    const int j1 = SHARED ? (j0 + g.per < L.n ? j0 + g.per : L.n) : j0 + 1;
-    KskJob J = L.dev ? get_job(L, j0) : get_inline(L, j0);
+    const KskJob J = L.dev ? get_job(L, (int)z) : get_inline(L, (int)z);
     const int nl = __builtin_amdgcn_readfirstlane(J.level) + 1;
-    const int pid = py;
     if (pid <= T.L && pid >= nl) return;  // a Q prime above this job's level
     const int pos = pid <= T.L ? pid : nl + (pid - (T.L + 1));
     const PrimeInfo P = cld(T.primes + pid);
@@ -193,6 +192,12 @@ __global__ void __launch_bounds__(FRows<LOGN>::NTR, 4) k_rows_ksk(DevTables T, K
         auto digit = [&](int d, V* v) {
             if (d == own_d) {
                 const u64x2 a = ld2(J.own + limb + x0), b = ld2(J.own + limb + x0 + 2);
+                v[0] = ar.from(a.x), v[1] = ar.from(a.y), v[2] = ar.from(b.x), v[3] = ar.from(b.y);
+                return;
+            }
+            if constexpr (EVAL) {
+                const uint64_t* e = J.ext + ((size_t)d * npos + pos) * G::N;
+                const u64x2 a = ld2(e + x0), b = ld2(e + x0 + 2);
                 v[0] = ar.from(a.x), v[1] = ar.from(a.y), v[2] = ar.from(b.x), v[3] = ar.from(b.y);
                 return;
             }
@@ -234,31 +239,15 @@ __global__ void __launch_bounds__(FRows<LOGN>::NTR, 4) k_rows_ksk(DevTables T, K
 #pragma unroll
             for (int k = 0; k < 4; ++k) o[in0 + elem<2, G::LOL, G::NBI>(t, k)] = A::pack(a[k]);
         };
-        if constexpr (!SHARED) {
-            typename A::Sum sa[4] = {}, sb[4] = {};
+        typename A::Sum sa[4] = {}, sb[4] = {};
 #pragma unroll 1
-            for (int d = 0; d < nd; ++d) {
-                V v[4];
-                digit(d, v);
-                mac(sa, sb, d, v);
-            }
-            finish(sa, J.acc_a, J.down_a, J.add_a);
-            finish(sb, J.acc_b, J.down_b, J.add_b);
-        } else {
-            V v[D][4];
-#pragma unroll
-            for (int d = 0; d < D; ++d)
-                if (d < nd) digit(d, v[d]);
-            for (int j = j0; j < j1; ++j) {
-                if (j != j0) J = L.dev ? get_job(L, j) : get_inline(L, j);
-                typename A::Sum sa[4] = {}, sb[4] = {};
-#pragma unroll
-                for (int d = 0; d < D; ++d)
-                    if (d < nd) mac(sa, sb, d, v[d]);
-                finish(sa, J.acc_a, J.down_a, J.add_a);
-                finish(sb, J.acc_b, J.down_b, J.add_b);
-            }
+        for (int d = 0; d < nd; ++d) {
+            V v[4];
+            digit(d, v);
+            mac(sa, sb, d, v);
         }
+        finish(sa, J.acc_a, J.down_a, J.add_a);
+        finish(sb, J.acc_b, J.down_b, J.add_b);
     });
 }
 
@@ -328,31 +317,20 @@ hipError_t launch_modup_cols(const DevTables& T, const ModUpJobs& L, int max_nd,
     return by_logn(T.logN, [&](auto ln) { modup_cols_a<decltype(ln)::value>(T, L, max_nd, targets, s); });
 }
 
-template <int LOGN, bool SHARED>
-static void rows_ksk(const DevTables& T, const KskJobs& L, int nq, hipStream_t s) {
-    using G = FRows<LOGN>;
-    constexpr int TPL = G::N1 / G::RR;
-    const int np = nq + T.K, nz = SHARED ? 1 : L.n;
-    const size_t items = (size_t)nz * np * TPL;
-    const XcdGrid x = xcd_grid(items, TPL * nz);
-    const KskGrid g{(uint32_t)items, x.chunk, FastDiv(np, items), FastDiv(nz, items), SHARED ? L.n : 1, nq};
-    const dim3 b(G::NTR);
-    if (!SHARED || T.dnum <= 2)
-        hipLaunchKernelGGL((k_rows_ksk<LOGN, 2, SHARED>), x.grid, b, 0, s, T, L, g);
-    else if (T.dnum == 3)
-        hipLaunchKernelGGL((k_rows_ksk<LOGN, SHARED ? 3 : 2, SHARED>), x.grid, b, 0, s, T, L, g);
-    else
-        hipLaunchKernelGGL((k_rows_ksk<LOGN, SHARED ? 4 : 2, SHARED>), x.grid, b, 0, s, T, L, g);
-}
-
-hipError_t launch_rows_ksk(const DevTables& T, const KskJobs& L, int max_npos, hipStream_t s, bool shared) {
+hipError_t launch_rows_ksk(const DevTables& T, const KskJobs& L, int max_npos, hipStream_t s, bool eval) {
     if (L.n <= 0 || max_npos <= 0) return hipSuccess;
     if (!fused_ok(T)) return hipErrorInvalidValue;
     return by_logn(T.logN, [&](auto ln) {
-        if (shared && L.n > 1)
-            rows_ksk<decltype(ln)::value, true>(T, L, max_npos - T.K, s);
+        constexpr int LN = decltype(ln)::value;
+        using G = FRows<LN>;
+        constexpr int TPL = G::N1 / G::RR;
+        const size_t items = (size_t)L.n * max_npos * TPL;
+        const XcdGrid x = xcd_grid(items, TPL * L.n);
+        const KskGrid g{(uint32_t)items, x.chunk, FastDiv(L.n, items), max_npos - T.K};
+        if (eval)
+            hipLaunchKernelGGL((k_rows_ksk<LN, true>), x.grid, dim3(G::NTR), 0, s, T, L, g);
         else
-            rows_ksk<decltype(ln)::value, false>(T, L, max_npos - T.K, s);
+            hipLaunchKernelGGL((k_rows_ksk<LN, false>), x.grid, dim3(G::NTR), 0, s, T, L, g);
     });
 }
 

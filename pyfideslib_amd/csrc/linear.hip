@@ -154,15 +154,45 @@ void ext_keyswitch(Context& c, int level, const std::vector<KsReq>& reqs, std::v
     std::vector<const uint64_t*> xs;
     for (const KsReq& r : reqs)
         if (std::find(xs.begin(), xs.end(), r.x) == xs.end()) xs.push_back(r.x);
-    keep.emplace_back(&c.pool, (size_t)nl * N);
+    const bool fused = fused_ok(c.T);
+    keep.emplace_back(&c.pool, (fused ? xs.size() : 1) * nl * N);
     uint64_t* t = keep.back().ptr;
     keep.emplace_back(&c.pool, xs.size() * nd * npos * N);
     uint64_t* ext = keep.back().ptr;
-    for (size_t i = 0; i < xs.size(); ++i) modup_to(c, level, xs[i], t, ext + i * nd * npos * N);
+    if (fused) {
+        std::vector<NttJob> iv;
+        std::vector<ModUpJob> mu;
+        for (size_t i = 0; i < xs.size(); ++i) {
+            NttJob j;
+            std::memset(&j, 0, sizeof(j));
+            j.src = xs[i];
+            j.mid = j.dst = t + i * nl * N;
+            j.npos = j.nq = nl;
+            j.level = level;
+            j.scale_sel = ISCALE_MODUP;
+            iv.push_back(j);
+            mu.push_back(ModUpJob{t + i * nl * N, ext + i * nd * npos * N, level});
+        }
+        run_ntt_jobs(c, iv, true);
+        ck(launch_modup_cols(c.T, job_list<ModUpJobs>(c, keep, mu), nd, nl, c.stream), "ext modup and columns");
+    } else {
+        for (size_t i = 0; i < xs.size(); ++i) modup_to(c, level, xs[i], t, ext + i * nd * npos * N);
+    }
     std::vector<KskJob> kj;
     for (const KsReq& r : reqs) {
         const size_t i = std::find(xs.begin(), xs.end(), r.x) - xs.begin();
-        kj.push_back(KskJob{ext + i * nd * npos * N, r.x, r.key->a.ptr, r.key->b.ptr, r.acc_a, r.acc_b, level});
+        kj.push_back(KskJob{ext + i * nd * npos * N, r.x, r.key->a.ptr, r.key->b.ptr, r.acc_a, r.acc_b, level, 0,
+                            nullptr, nullptr, nullptr, nullptr});
+    }
+    if (fused) {
+        // several sources: sorted by key, so that the jobs of one key run side by side
+        if (xs.size() > 1)
+            std::stable_sort(kj.begin(), kj.end(), [](const KskJob& x, const KskJob& y) { return x.ka < y.ka; });
+        const bool eval = kj.size() > 1 && xs.size() == 1;  // several keys: the digits' rows once for all
+        if (eval) modup_rows(c, level, ext);
+        ck(launch_rows_ksk(c.T, job_list<KskJobs>(c, keep, kj), (int)npos, c.stream, eval),
+           "ext rows and key switch");
+        return;
     }
     // several sources switched by the same keys (the baby steps of a batch of
     // ciphertexts, a giant step of each): the jobs grouped by key and run
@@ -210,7 +240,7 @@ void ext_moddown(Context& c, int level, const std::vector<std::pair<const uint64
         j.npos = K;
         j.scale_sel = ISCALE_MODDOWN;
         isp.push_back(j);
-        md.push_back(ModDownJob{ti, yi, nullptr, nullptr, level});
+        md.push_back(ModDownJob{ti, yi, nullptr, nullptr, level, 0});
         NttJob f;
         std::memset(&f, 0, sizeof(f));
         f.src = f.mid = yi;
@@ -221,6 +251,11 @@ void ext_moddown(Context& c, int level, const std::vector<std::pair<const uint64
         fwd.push_back(f);
     }
     run_ntt_jobs(c, isp, true);
+    if (fused_ok(c.T)) {
+        ck(launch_moddown_cols(c.T, job_list<ModDownJobs>(c, keep, md), nl, false, c.stream), "ext moddown and columns");
+        run_ntt_jobs(c, fwd, false, LOAD_PLAIN, STORE_MODDOWN, NTT_PASS2);
+        return;
+    }
     ck(launch_moddown_conv(c.T, job_list<ModDownJobs>(c, keep, md), nl, c.stream),
        "ext moddown conv");
     run_ntt_jobs(c, fwd, false, LOAD_PLAIN, STORE_MODDOWN);
