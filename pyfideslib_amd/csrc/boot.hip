@@ -25,10 +25,12 @@
 // pre / (K N) (Bootstrap.cu:219-231); here that factor sits in the
 // CoeffsToSlots diagonals.
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <complex>
 #include <map>
 #include <set>
+#include <thread>
 
 #include "context.hpp"
 
@@ -68,25 +70,73 @@ int bitrev(int x, int bits) {
     return r;
 }
 
-// w = U0^-1 z in place: the inverse stages from B_n down, then P
-void special_fft_inverse(std::vector<cd>& v) {
-    const int n = (int)v.size();
-    const std::vector<Stage> st = stages(n);
-    for (auto it = st.rbegin(); it != st.rend(); ++it) {
-        const int h = it->h;
-        for (int blk = 0; blk < n; blk += 2 * h)
-            for (int j = 0; j < h; ++j) {
-                const cd a = v[blk + j], b = v[blk + j + h];
-                v[blk + j] = (a + b) * 0.5;
-                v[blk + j + h] = (a - b) * 0.5 / it->tw[j];
-            }
+// f(0) .. f(parts - 1), each on its own thread (part 0, and any the system
+// has no thread for, on the caller's).  f must not throw.
+template <class F>
+void in_parallel(int parts, const F& f) {
+    std::vector<std::thread> th;
+    int p = 1;
+    try {
+        th.reserve(parts);
+        for (; p < parts; ++p) th.emplace_back([&f, p] { f(p); });
+    } catch (const std::exception&) {  // no more threads: the parts from p on run here
     }
+    f(0);
+    for (int q = p; q < parts; ++q) f(q);
+    for (std::thread& t : th) t.join();
+}
+
+// round(scale [Re w, Im w]), w = U0^-1 z, into m[0 .. 2n): the inverse stages from
+// B_n down, then P.  The top three stages combine indices that agree mod n / 8
+// and the rest stays inside eighths of the vector, so both halves of the work
+// split over 8 threads; every butterfly is the same arithmetic in any order of
+// the others.  False: a coefficient is at or beyond 2^62 (or not a number).
+constexpr int FFT_PARTS = 8;
+bool rounded_coefficients(std::vector<cd>& v, const std::vector<Stage>& st, double scale, int64_t* m) {
+    const int n = (int)v.size(), ns = (int)st.size();  // st[s].h = 2^s
+    auto butterfly = [&](const Stage& s, int i) {  // elements i and i + h, i's bit h clear
+        const int h = s.h;
+        const cd a = v[i], b = v[i + h];
+        v[i] = (a + b) * 0.5;
+        v[i + h] = (a - b) * 0.5 / s.tw[i & (h - 1)];
+    };
+    auto range = [&](int s_hi, int s_lo, int from, int to) {  // stages s_hi-1 .. s_lo on [from, to)
+        for (int s = s_hi - 1; s >= s_lo; --s)
+            for (int blk = from; blk < to; blk += 2 * st[s].h)
+                for (int j = 0; j < st[s].h; ++j) butterfly(st[s], blk + j);
+    };
     int bits = 0;
     while ((1 << bits) < n) ++bits;
-    for (int i = 0; i < n; ++i) {
-        const int r = bitrev(i, bits);
-        if (r > i) std::swap(v[i], v[r]);
+    std::atomic<bool> ok{true};
+    auto store = [&](int from, int to) {
+        for (int i = from; i < to; ++i) {
+            const int r = bitrev(i, bits);
+            const double re = v[i].real() * scale, im = v[i].imag() * scale;
+            if (!(std::fabs(re) < 0x1p62) || !(std::fabs(im) < 0x1p62)) {
+                ok = false;
+                return;
+            }
+            m[r] = std::llround(re);
+            m[n + r] = std::llround(im);
+        }
+    };
+    if (n < 4096) {  // a thread's start costs more than an eighth of the work
+        range(ns, 0, 0, n);
+        store(0, n);
+        return ok;
     }
+    const int e = n / FFT_PARTS;
+    in_parallel(FFT_PARTS, [&](int p) {
+        for (int j = p * (e / FFT_PARTS); j < (p + 1) * (e / FFT_PARTS); ++j)
+            for (int s = ns - 1; s >= ns - 3; --s)
+                for (int k = 0; k < FFT_PARTS; ++k)
+                    if (!((j + k * e) & st[s].h)) butterfly(st[s], j + k * e);
+    });
+    in_parallel(FFT_PARTS, [&](int p) {
+        range(ns - 3, 0, p * e, (p + 1) * e);
+        store(p * e, (p + 1) * e);
+    });
+    return ok;
 }
 
 // one stage as {offset d: diag}, out[p] = sum_d diag[p] in[(p + d) mod n]
@@ -182,36 +232,34 @@ int64_t mod_n(int64_t x, int64_t n) { return ((x % n) + n) % n; }
 }  // namespace
 
 // MakeCKKSPackedPlaintext (api/CryptoContext.cpp:475-514): coefficients
-// round(scale [Re w, Im w]), w = U0^-1 z, reduced mod q_0..q_level on the
-// host, then the engine's forward NTT in place.  With ext the coefficients
-// are also reduced mod the K special primes (a P*Q plaintext, as OpenFHE
-// encodes the linear-transform diagonals in the extended basis for
-// EvalFastRotationExt).
+// round(scale [Re w, Im w]), w = U0^-1 z, on the host (FP64, the stages' twiddles
+// kept with the context), their residues mod q_0..q_level and the forward NTT
+// on the device.  With ext the coefficients are also reduced mod the K special
+// primes (a P*Q plaintext, as OpenFHE encodes the linear-transform diagonals
+// in the extended basis for EvalFastRotationExt).
+//
+// At N = 2^16, level 23 this was 9.3 ms of one host thread (4 ms of FFT, 1 ms of
+// twiddles, 3.5 ms of residues, a pageable upload of 13 MB).
 std::unique_ptr<Plaintext> encode_slots(Context& c, const std::vector<cd>& z, int level, double scale, bool ext) {
     const int n = c.N / 2;
     if ((int)z.size() != n) throw Error(E_ARG, "encode needs N/2 slot values");
     if (level < 0 || level > c.L) throw Error(E_LEVEL, "level out of range");
+    if (!c.fft_stages) c.fft_stages = std::make_shared<std::vector<Stage>>(stages(n));
+    const auto& st = *static_cast<const std::vector<Stage>*>(c.fft_stages.get());
     std::vector<cd> w(z);
-    special_fft_inverse(w);
+    std::vector<int64_t> m((size_t)c.N);
+    if (!rounded_coefficients(w, st, scale, m.data())) throw Error(E_ARG, "encoded coefficient exceeds 62 bits");
     const int nl = level + 1, nr = nl + (ext ? c.K : 0);
-    std::vector<uint64_t> res((size_t)nr * c.N);
-    for (int k = 0; k < (int)c.N; ++k) {
-        const double m = (k < n ? w[k].real() : w[k - n].imag()) * scale;
-        if (!(std::fabs(m) < 0x1p62)) throw Error(E_ARG, "encoded coefficient exceeds 62 bits");
-        const int64_t v = std::llround(m);
-        for (int i = 0; i < nr; ++i) {
-            const int64_t q = (int64_t)c.q[i < nl ? i : c.L + 1 + (i - nl)];
-            res[(size_t)i * c.N + k] = (uint64_t)(((v % q) + q) % q);
-        }
-    }
     std::unique_ptr<Plaintext> pt = pt_create(c);
-    if (ext) {
-        pt_load_ext(c, *pt, res.data(), nl, scale, 1, n, false);
-        poly_ntt(c, pt->c0() + (size_t)nl * c.N, c.K, c.L + 1, false);
-    } else {
-        pt_load(c, *pt, res.data(), nl, scale, 1, n, false);
-    }
-    poly_ntt(c, pt->c0(), nl, 0, false);
+    pt_set(c, *pt, nl, ext, scale, 1, n);
+    DevBuf coef(&c.pool, (size_t)c.N);
+    c.upload(coef.ptr, m.data(), (size_t)c.N * 8);
+    hip_check(launch_residues(c.T, (const int64_t*)coef.ptr, pt->c0(), nl, nr, c.stream), "encode residues");
+    NttJob j{};
+    j.src = j.mid = j.dst = pt->c0();
+    j.npos = nr;
+    j.nq = nl;
+    run_ntt_jobs(c, {j}, false);
     return pt;
 }
 

@@ -160,6 +160,7 @@ class Context {
     // key; each entry owns the scratch its graph was captured with.
     std::map<std::vector<uint64_t>, std::shared_ptr<void>> graph_cache;
     std::set<std::vector<uint64_t>> graph_seen;  // signatures run once (eagerly)
+    std::shared_ptr<void> fft_stages;  // twiddles of the encoder's special FFT (boot.hip)
     std::shared_ptr<void> ks_workspace;          // key-switch buffers shared by all ops
     bool use_graphs = true;  // FIDES_GRAPHS=0 disables capture
     // Per-op launch sequences captured and replayed (run_cached): off by
@@ -261,6 +262,7 @@ std::unique_ptr<Plaintext> pt_create(Context& c);
 // P*Q plaintext: limbs [num_res + K][N], the Q limbs 0 .. num_res-1 then the K special limbs.
 void pt_load_ext(Context& c, Plaintext& pt, const uint64_t* limbs, int num_res, double noise, int noise_level,
                  int slots, bool device_src);
+void pt_set(Context& c, Plaintext& pt, int num_res, bool ext, double noise, int noise_level, int slots);
 void pt_load(Context& c, Plaintext& pt, const uint64_t* limbs, int num_res, double noise, int noise_level, int slots,
              bool device_src);
 void eval_mult_plain(Context& c, const Ciphertext& a, const Plaintext& pt, Ciphertext& out, bool rescale);

@@ -385,6 +385,8 @@ hipError_t launch_lincomb(const DevTables& T, const LinCombJob& job, hipStream_t
 // max_gc: the largest gc of the list (selects the accumulator count)
 hipError_t launch_dot_bsgs(const DevTables& T, const DotJobs& jobs, int max_nl, int max_gc, hipStream_t stream);
 hipError_t launch_ext_rot(const DevTables& T, const ExtRotJobs& jobs, int max_nl, hipStream_t stream);
+// Residues of N signed coefficients on `limbs` limbs: nl Q limbs, then special ones.
+hipError_t launch_residues(const DevTables& T, const int64_t* v, uint64_t* o, int nl, int limbs, hipStream_t stream);
 // o = a * X^m (evaluation form) on each limb; b unused.
 hipError_t launch_monomial(const DevTables& T, const EwJobs& jobs, int max_nl, uint32_t m, hipStream_t stream);
 // o = a * c[i] (EW_MUL_SCALAR) or a + c[i] (EW_ADD_SCALAR) on limb i; b unused.

@@ -571,6 +571,17 @@ __global__ void __launch_bounds__(EW_BLOCK) k_scalar(DevTables T, EwJobs L, Limb
         st2(J.o + x, addmod(a.x, w.w, p), addmod(a.y, w.w, p));
 }
 
+// Residues of signed coefficients (|v| < 2^63) mod the primes of nl Q limbs and
+// then of the special primes (an encoded plaintext before its transform).
+__global__ void __launch_bounds__(EW_BLOCK) k_residues(DevTables T, const int64_t* v, uint64_t* o, int nl) {
+    const int i = blockIdx.y;
+    const PrimeInfo P = cld(T.primes + pos_pid(i, nl, 0, T.L + 1));
+    const uint32_t x = blockIdx.x * EW_BLOCK + threadIdx.x;
+    const int64_t s = (int64_t)gp((const uint64_t*)v)[x];
+    const uint64_t r = reduce64(s < 0 ? (uint64_t)0 - (uint64_t)s : (uint64_t)s, P);
+    gp(o)[(size_t)i * T.N + x] = s < 0 && r ? P.p - r : r;
+}
+
 // Multiplication by the monomial X^m on evaluation-form limbs (FIDESlib
 // Ciphertext::multMonomial, Ciphertext.cpp:1709-1760, multiplies by the NTT of
 // X^m): slot j of limb i holds a(psi^e_j) with e_j = 2 brev(j) + 1, so it is
@@ -963,6 +974,12 @@ hipError_t launch_dot_bsgs(const DevTables& T, const DotJobs& L, int max_nl, int
 hipError_t launch_ext_rot(const DevTables& T, const ExtRotJobs& L, int max_nl, hipStream_t s) {
     if (L.n <= 0 || max_nl <= 0) return hipSuccess;
     hipLaunchKernelGGL(k_ext_rot, dim3(T.N / EW_BLOCK, max_nl + T.K, L.n), dim3(EW_BLOCK), 0, s, T, L);
+    return hipGetLastError();
+}
+
+hipError_t launch_residues(const DevTables& T, const int64_t* v, uint64_t* o, int nl, int limbs, hipStream_t s) {
+    if (limbs <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_residues, dim3(T.N / EW_BLOCK, limbs), dim3(EW_BLOCK), 0, s, T, v, o, nl);
     return hipGetLastError();
 }
 

@@ -158,6 +158,18 @@ void pt_load(Context& c, Plaintext& pt, const uint64_t* limbs, int num_res, doub
     pt.slots = slots;
 }
 
+// The buffer and metadata of a plaintext whose limbs a kernel writes.
+void pt_set(Context& c, Plaintext& pt, int num_res, bool ext, double noise, int noise_level, int slots) {
+    if (num_res < 1 || num_res > c.L + 1) throw Error(E_LEVEL, "num_res out of range");
+    const size_t words = (size_t)(num_res + (ext ? c.K : 0)) * c.N;
+    if (pt.data.bytes < words * 8) pt.data = DevBuf(&c.pool, (size_t)(c.L + 1 + c.K) * c.N);
+    pt.level = num_res - 1;
+    pt.ext = ext;
+    pt.noise = noise;
+    pt.noise_level = noise_level;
+    pt.slots = slots;
+}
+
 void pt_load_ext(Context& c, Plaintext& pt, const uint64_t* limbs, int num_res, double noise, int noise_level,
                  int slots, bool device_src) {
     if (num_res < 1 || num_res > c.L + 1) throw Error(E_LEVEL, "num_res out of range");
