@@ -285,10 +285,11 @@ static void run_plan_fused(Context& c, const BatchPlan& P) {
         ckb(launch_tensor_rows(T, dev_list<TensorJobs>(P.tensor, P.n_mult), P.max_nl, s), "batch tensor and rows");
     if (P.intt_rot.njobs)
         ckb(launch_ntt_inv(T, ntt_list(P.intt_rot), P.intt_rot.limbs, s, NTT_PASS1), "batch intt rows");
-    ckb(launch_ntt_inv(T, ntt_list(P.intt_up), P.intt_up.limbs, s, NTT_PASS2), "batch intt columns");
+    const bool cols = !fused_inv_cols(T);  // the conversions do not run their sources' columns
+    if (cols) ckb(launch_ntt_inv(T, ntt_list(P.intt_up), P.intt_up.limbs, s, NTT_PASS2), "batch intt columns");
     ckb(launch_modup_cols(T, dev_list<ModUpJobs>(P.modup, P.n), P.max_nd, P.max_nl, s), "batch modup and columns");
     ckb(launch_rows_ksk(T, dev_list<KskJobs>(P.ksk, P.n), P.max_npos, s), "batch rows and ksk");
-    ckb(launch_ntt_inv(T, ntt_list(P.intt_sp), P.intt_sp.limbs, s, NTT_PASS2), "batch intt sp columns");
+    if (cols) ckb(launch_ntt_inv(T, ntt_list(P.intt_sp), P.intt_sp.limbs, s, NTT_PASS2), "batch intt sp columns");
     if (P.n_conv_rescale)
         ckb(launch_moddown_cols(T, dev_list<ModDownJobs>(P.conv_rescale, P.n_conv_rescale), P.max_nl, true, s),
             "batch moddown+rescale and columns");
@@ -572,7 +573,8 @@ static void run_hoist_plan(Context& c, const HoistPlan& P) {
         modup_half(c, P.level, P.c1, P.t, P.ext);
         if (P.nk > 1) modup_rows(c, P.level, P.ext);
         ckb(launch_rows_ksk(T, dev_list<KskJobs>(P.ksk, P.nk), P.npos, s, P.nk > 1), "hoist rows and ksk");
-        ckb(launch_ntt_inv(T, ntt_list(P.intt_sp), P.intt_sp.limbs, s, NTT_PASS2), "hoist intt sp columns");
+        if (!fused_inv_cols(T))
+            ckb(launch_ntt_inv(T, ntt_list(P.intt_sp), P.intt_sp.limbs, s, NTT_PASS2), "hoist intt sp columns");
         ckb(launch_moddown_cols(T, dev_list<ModDownJobs>(P.moddown, 2 * P.nk), nl, false, s), "hoist moddown columns");
         ckb(launch_ntt_fwd(T, ntt_list(P.ntt_md), P.ntt_md.limbs, LOAD_PLAIN, STORE_MODDOWN_AUTO, s, NTT_PASS2),
             "hoist moddown automorph rows");

@@ -208,7 +208,7 @@ static void modup_cols(Context& c, int level, const uint64_t* t, uint64_t* ext) 
 
 // ModUp of x up to what the fused inner product takes.
 void modup_half(Context& c, int level, const uint64_t* x, uint64_t* t, uint64_t* ext) {
-    modup_intt(c, level, x, t);
+    modup_intt(c, level, x, t, fused_inv_cols(c.T) ? NTT_PASS1 : NTT_BOTH);
     modup_cols(c, level, t, ext);
 }
 
@@ -271,7 +271,7 @@ static void fused_ksk_moddown(Context& c, int level, const uint64_t* ext, const 
         f.autok = autok;
         fw.push_back(f);
     }
-    run_ntt(c, iv, true, LOAD_PLAIN, STORE_PLAIN, NTT_PASS2);
+    if (!fused_inv_cols(c.T)) run_ntt(c, iv, true, LOAD_PLAIN, STORE_PLAIN, NTT_PASS2);
     ck(launch_moddown_cols(c.T, mj, nl, rescale, c.stream), "moddown conversion and columns");
     run_ntt(c, fw, false, LOAD_PLAIN, rescale ? STORE_MODDOWN_RESCALE : autok ? STORE_MODDOWN_AUTO : STORE_MODDOWN,
             NTT_PASS2);
@@ -422,7 +422,7 @@ static void mult_core(Context& c, const Ciphertext* a, const Ciphertext* b, Ciph
         tj.n = 1;
         if (fused_ok(c.T)) {
             ck(launch_tensor_rows(c.T, tj, nl, c.stream), "tensor and rows");
-            modup_intt(c, level, s.d2.ptr, s.t.ptr, NTT_PASS2);
+            if (!fused_inv_cols(c.T)) modup_intt(c, level, s.d2.ptr, s.t.ptr, NTT_PASS2);
             modup_cols(c, level, s.t.ptr, s.ext.ptr);
             fused_ksk_moddown(c, level, s.ext.ptr, s.d2.ptr, key, s, o0, o0, o1, o1, do_rescale);
             return;

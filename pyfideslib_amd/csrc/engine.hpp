@@ -367,9 +367,13 @@ hipError_t launch_moddown_conv_mode(const DevTables& T, const ModDownJobs& jobs,
 // Whether these parameters take it: rings of 2^12 .. 2^16, at most 4 digits of
 // at most 10 primes, at most 10 special primes, sums within one reduction.
 bool fused_ok(const DevTables& T);
+// Whether the conversion kernels take their sources after the first pass of the
+// inverse transform only (small rings), and run the second themselves.
+bool fused_inv_cols(const DevTables& T);
 // Tensor product, and the first pass of the inverse transform of its third part.
 hipError_t launch_tensor_rows(const DevTables& T, const TensorJobs& jobs, int max_nl, hipStream_t stream);
 // ModUp conversion and the first pass of the forward transform of its outputs.
+// Sources: coefficient form, or see fused_inv_cols.
 // max_nl: limbs of the list's top level.
 hipError_t launch_modup_cols(const DevTables& T, const ModUpJobs& jobs, int max_nd, int max_nl, hipStream_t stream);
 // Second pass of the digits' transforms and the key-switch inner product

@@ -72,7 +72,7 @@ __global__ void __launch_bounds__(FRows<LOGN>::NTR) k_tensor_rows(DevTables T, T
 template <int LOGN, int A>
 __global__ void __launch_bounds__(512, 4) k_modup_cols(DevTables T, ModUpJobs L, ConvGrid g) {
     using G = ConvCols<LOGN>;
-    __shared__ ConvLds<LOGN> S;
+    __shared__ ConvLds<LOGN, A> S;
     const uint32_t item = xcd_item(g.chunk);
     if (item >= g.items) return;
     const uint32_t u = item / G::TPL, u2 = g.tg.div(u), z = g.nd.div(u2);
@@ -93,7 +93,18 @@ __global__ void __launch_bounds__(512, 4) k_modup_cols(DevTables T, ModUpJobs L,
     const int n_tgt = __builtin_amdgcn_readfirstlane(G::n_tgt(tid));
     // the digit's limbs; rows beyond its size are zero
     Half2 x[G::CPT][A];
-    {
+    if constexpr (conv_inv<LOGN>()) {
+        conv_sources(
+            T, S, size, col0, [&](int i) { return J.t + (size_t)(start + i) * G::N; },
+            [&](int i) { return start + i; },
+            [&](int i) { return T.iscale_modup + ((size_t)(nl - 1) * (T.L + 1) + start + i) * 2; });
+#pragma unroll
+        for (int i = 0; i < A; ++i)
+#pragma unroll
+            for (int c = 0; c < G::CPT; ++c)
+                x[c][i] = split30(i < size ? S.s.tile[i][G::c_col(tid) + c][lds_off(G::c_row(tid))] : 0);
+        __syncthreads();  // the targets take over the LDS
+    } else {
         uint64_t v[A][G::CPT];
 #pragma unroll
         for (int i = 0; i < A; ++i) {
@@ -131,7 +142,7 @@ __global__ void __launch_bounds__(512, 4) k_modup_cols(DevTables T, ModUpJobs L,
             for (int c = 0; c < G::CPT; ++c) {
                 uint64_t lo, hi;
                 conv_acc<A>(x[c], row, lo, hi);
-                S.tile[buf][i][G::c_col(tid) + c][lds_off(G::c_row(tid))] = conv_word(T, pid, P, lo, hi);
+                S.t.tile[buf][i][G::c_col(tid) + c][lds_off(G::c_row(tid))] = conv_word(T, pid, P, lo, hi);
             }
         }
         tw.put(S, buf, s_tgt, s_row);
@@ -256,6 +267,8 @@ bool fused_ok(const DevTables& T) {
     return T.logN >= FUSED_LOGN_MIN && T.logN <= FUSED_LOGN_MAX && T.dnum <= FUSED_DIGITS &&
            T.alpha <= FUSED_CONV_MAX && T.K <= FUSED_CONV_MAX && T.modup_one_reduce && T.moddown_one_reduce;
 }
+
+bool fused_inv_cols(const DevTables& T) { return fused_ok(T) && T.logN <= CONV_INV_LOGN; }
 
 template <class F>
 static hipError_t by_logn(int logN, F&& f) {

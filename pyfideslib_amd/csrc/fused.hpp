@@ -8,6 +8,7 @@ namespace fides {
 constexpr int FUSED_LOGN_MIN = 12, FUSED_LOGN_MAX = 16;
 constexpr int FUSED_CONV_MAX = 10;  // source limbs of a conversion
 constexpr int FUSED_DIGITS = 4;
+constexpr int CONV_INV_LOGN = 14;
 
 // Unsigned division by a launch constant d of values up to most: one multiply
 // where it is exact (most d < 2^32), else the division itself.
@@ -53,24 +54,88 @@ struct ConvCols {
     static __device__ __forceinline__ uint32_t n_col(uint32_t tid) { return tid / TPC % CC; }
     static __device__ __forceinline__ uint32_t n_t(uint32_t tid) { return tid % TPC; }
 };
+// Rings up to 2^CONV_INV_LOGN are bound by launches: there the conversion
+// kernels also run the column pass of their sources' inverse transform (once
+// per target group, which costs arithmetic that the idle CUs have to spare).
 template <int LOGN>
+constexpr bool conv_inv() { return LOGN <= CONV_INV_LOGN; }
+template <int LOGN, int SOURCES>
 struct ConvLds {
     using G = ConvCols<LOGN>;
-    uint64_t tile[2][G::TB][G::CC][G::SC];
-    ShoupConst tw[2][G::TB][G::N1];
+    struct Targets {
+        uint64_t tile[2][G::TB][G::CC][G::SC];
+        ShoupConst tw[2][G::TB][G::N1];
+    };
+    struct Sources {
+        uint64_t tile[SOURCES][G::CC][G::SC];
+        ShoupConst tw[SOURCES][G::N1];
+    };
+    struct None {};
+    union {
+        Targets t;
+        std::conditional_t<conv_inv<LOGN>(), Sources, None> s;  // before the first target
+    };
 };
 
+// The column pass of the inverse transform of n source limbs (limb(i): what the
+// row pass left, pid(i), scale(i): the limb's last-stage pair) on the block's
+// columns; coefficient (row, column) of limb i ends at S.s.tile[i][column][row].
+template <int LOGN, int SOURCES, class LIMB, class PID, class SCALE>
+__device__ __forceinline__ void conv_sources(const DevTables& T, ConvLds<LOGN, SOURCES>& S, int n, uint32_t col0,
+                                             const LIMB& limb, const PID& pid_of, const SCALE& scale) {
+    using G = ConvCols<LOGN>;
+    constexpr int LOL = inv_last_lo<2, G::K1>(), NBI = G::K1 - LOL, PAIRS = G::COEF / 2;
+    for (int w = threadIdx.x; w < n * PAIRS; w += G::NT) {
+        const int i = __builtin_amdgcn_readfirstlane(w / PAIRS);  // PAIRS is a multiple of the wave
+        const uint32_t e = (w % PAIRS) * 2, row = e / G::CC, cc = e % G::CC;
+        const u64x2 v = ld2(limb(i) + row * G::N2 + col0 + cc);
+        S.s.tile[i][cc][lds_off(row)] = v.x;
+        S.s.tile[i][cc + 1][lds_off(row)] = v.y;
+    }
+    for (int w = threadIdx.x; w < n * G::N1; w += G::NT) {
+        const int i = __builtin_amdgcn_readfirstlane(w / G::N1), r = w % G::N1;
+        const size_t at = (size_t)pid_of(i) * G::N + r;
+        if (is_fp(T, pid_of(i)))
+            reinterpret_cast<double*>(S.s.tw[i])[r] = T.twd_inv[at];
+        else
+            S.s.tw[i][r] = T.tw_inv[at];
+    }
+    __syncthreads();
+    const uint32_t t = G::n_t(threadIdx.x);
+    for (int ci = threadIdx.x / G::TPC; ci < n * G::CC; ci += G::NT / G::TPC) {
+        const int i = __builtin_amdgcn_readfirstlane(ci / G::CC);  // a wave's columns are of one limb
+        const uint32_t cc = ci % G::CC;
+        const int pid = pid_of(i);
+        const PrimeInfo P = cld(T.primes + pid);
+        const ShoupConst* sc = scale(i);
+        const ShoupConst s = cld(sc), ws = cld(sc + 1);
+        with_arith(T, pid, P, [&](const auto& ar) {
+            using A = std::decay_t<decltype(ar)>;
+            using V = typename A::V;
+            const auto* twl = reinterpret_cast<const typename A::W*>(S.s.tw[i]);
+            V* sub = reinterpret_cast<V*>(S.s.tile[i][cc]);
+            V v[4];
+            lds_get<2, 0, first_nb<2, G::K1>()>(sub, t, v);  // the words as the row pass packed them
+            auto twf = [&](int, int b, uint32_t e) { return twl[(1u << (G::K1 - 1 - b)) + (e >> (b + 1))]; };
+            inv_run<2, G::K1, 0, true, true>(ar, sub, v, t, twf, s, ws);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) S.s.tile[i][cc][lds_off(elem<2, LOL, NBI>(t, j))] = ar.canon_inv(v[j]);
+        });
+    }
+    __syncthreads();
+}
+
 // The column pass of a wave's target (prime pid) on the buffer's tile.
-template <int LOGN>
-__device__ __forceinline__ void conv_columns(const DevTables& T, int pid, ConvLds<LOGN>& S, int buf, int i) {
+template <int LOGN, int SOURCES>
+__device__ __forceinline__ void conv_columns(const DevTables& T, int pid, ConvLds<LOGN, SOURCES>& S, int buf, int i) {
     using G = ConvCols<LOGN>;
     const uint32_t t = G::n_t(threadIdx.x), cc = G::n_col(threadIdx.x);
     const PrimeInfo P = cld(T.primes + pid);
     with_arith(T, pid, P, [&](const auto& ar) {
         using A = std::decay_t<decltype(ar)>;
         using V = typename A::V;
-        const auto* twl = reinterpret_cast<const typename A::W*>(S.tw[buf][i]);
-        V* sub = reinterpret_cast<V*>(S.tile[buf][i][cc]);
+        const auto* twl = reinterpret_cast<const typename A::W*>(S.t.tw[buf][i]);
+        V* sub = reinterpret_cast<V*>(S.t.tile[buf][i][cc]);
         V v[4];
         lds_get<2, G::LO1, 2>(sub, t, v);
         auto twf = [&](int, int b, uint32_t e) { return twl[(1u << (G::K1 - 1 - b)) + (e >> (b + 1))]; };
@@ -90,24 +155,25 @@ struct ConvTw {
         else
             w = T.tw_fwd[(size_t)pid * T.N + r];
     }
-    template <int LOGN>
-    __device__ __forceinline__ void put(ConvLds<LOGN>& S, int buf, int i, int r) const {
+    template <int LOGN, int SOURCES>
+    __device__ __forceinline__ void put(ConvLds<LOGN, SOURCES>& S, int buf, int i, int r) const {
         if (fp)
-            reinterpret_cast<uint64_t*>(S.tw[buf][i])[r] = w.w;
+            reinterpret_cast<uint64_t*>(S.t.tw[buf][i])[r] = w.w;
         else
-            S.tw[buf][i][r] = w;
+            S.t.tw[buf][i][r] = w;
     }
 };
 // The tile's rows to limb `out`: 2048 words of TB targets, 4 a thread.
-template <int LOGN, class F>
-__device__ __forceinline__ void conv_store(const ConvLds<LOGN>& S, int buf, uint32_t col0, const F& limb) {
+template <int LOGN, int SOURCES, class F>
+__device__ __forceinline__ void conv_store(const ConvLds<LOGN, SOURCES>& S, int buf, uint32_t col0, const F& limb) {
     using G = ConvCols<LOGN>;
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
         const uint32_t w = (threadIdx.x + q * G::NT) * 2;
         const uint32_t i = w / G::COEF, row = w / G::CC % G::N1, cc = w % G::CC;
         uint64_t* o = limb((int)i);
-        if (o) st2(o + row * G::N2 + col0 + cc, S.tile[buf][i][cc][lds_off(row)], S.tile[buf][i][cc + 1][lds_off(row)]);
+        if (o) st2(o + row * G::N2 + col0 + cc, S.t.tile[buf][i][cc][lds_off(row)],
+                   S.t.tile[buf][i][cc + 1][lds_off(row)]);
     }
 }
 // A wave-uniform conversion sum in the arithmetic of its prime, as tile word.

@@ -8,7 +8,7 @@ namespace fides {
 template <int LOGN, int KK, bool RESCALE>
 __global__ void __launch_bounds__(512, 4) k_moddown_cols(DevTables T, ModDownJobs L, ConvGrid g) {
     using G = ConvCols<LOGN>;
-    __shared__ ConvLds<LOGN> S;
+    __shared__ ConvLds<LOGN, KK + (RESCALE ? 1 : 0)> S;
     const uint32_t item = xcd_item(g.chunk);
     if (item >= g.items) return;
     const uint32_t u = item / G::TPL, z = g.tg.div(u);
@@ -26,7 +26,24 @@ __global__ void __launch_bounds__(512, 4) k_moddown_cols(DevTables T, ModDownJob
     const int n_tgt = __builtin_amdgcn_readfirstlane(G::n_tgt(tid));
     Half2 x[G::CPT][KK];
     uint64_t top[G::CPT];
-    {
+    if constexpr (conv_inv<LOGN>()) {
+        // the special limbs, and the limb that a rescale drops
+        conv_sources(
+            T, S, KK + (RESCALE ? 1 : 0), col0, [&](int i) { return i < KK ? J.t + (size_t)i * G::N : J.top_acc; },
+            [&](int i) { return i < KK ? T.L + 1 + i : l; },
+            [&](int i) { return i < KK ? T.iscale_moddown + (size_t)i * 2 : T.iscale_plain + (size_t)l * 2; });
+#pragma unroll
+        for (int i = 0; i < KK + (RESCALE ? 1 : 0); ++i)
+#pragma unroll
+            for (int c = 0; c < G::CPT; ++c) {
+                const uint64_t w = S.s.tile[i][G::c_col(tid) + c][lds_off(G::c_row(tid))];
+                if (i < KK)
+                    x[c][i < KK ? i : 0] = split30(w);
+                else
+                    top[c] = w;
+            }
+        __syncthreads();  // the targets take over the LDS
+    } else {
         uint64_t v[KK][G::CPT];
 #pragma unroll
         for (int i = 0; i < KK; ++i) {
@@ -93,7 +110,7 @@ __global__ void __launch_bounds__(512, 4) k_moddown_cols(DevTables T, ModDownJob
                 } else {
                     word = conv_word(T, pid, P, lo, hi);
                 }
-                S.tile[buf][i][G::c_col(tid) + c][lds_off(G::c_row(tid))] = word;
+                S.t.tile[buf][i][G::c_col(tid) + c][lds_off(G::c_row(tid))] = word;
             }
         }
         tw.put(S, buf, s_tgt, s_row);

@@ -173,7 +173,7 @@ void ext_keyswitch(Context& c, int level, const std::vector<KsReq>& reqs, std::v
             iv.push_back(j);
             mu.push_back(ModUpJob{t + i * nl * N, ext + i * nd * npos * N, level});
         }
-        run_ntt_jobs(c, iv, true);
+        run_ntt_jobs(c, iv, true, LOAD_PLAIN, STORE_PLAIN, fused_inv_cols(c.T) ? NTT_PASS1 : NTT_BOTH);
         ck(launch_modup_cols(c.T, job_list<ModUpJobs>(c, keep, mu), nd, nl, c.stream), "ext modup and columns");
     } else {
         for (size_t i = 0; i < xs.size(); ++i) modup_to(c, level, xs[i], t, ext + i * nd * npos * N);
@@ -250,7 +250,7 @@ void ext_moddown(Context& c, int level, const std::vector<std::pair<const uint64
         f.nq = nl;
         fwd.push_back(f);
     }
-    run_ntt_jobs(c, isp, true);
+    run_ntt_jobs(c, isp, true, LOAD_PLAIN, STORE_PLAIN, fused_inv_cols(c.T) ? NTT_PASS1 : NTT_BOTH);
     if (fused_ok(c.T)) {
         ck(launch_moddown_cols(c.T, job_list<ModDownJobs>(c, keep, md), nl, false, c.stream), "ext moddown and columns");
         run_ntt_jobs(c, fwd, false, LOAD_PLAIN, STORE_MODDOWN, NTT_PASS2);
