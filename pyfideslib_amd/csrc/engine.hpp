@@ -184,7 +184,11 @@ using ModUpJobs = JobList<ModUpJob, MODUP_INLINE>;
 // transform, and for a ModDown that follows runs the first pass of the inverse
 // on what goes down: special limb k to down_x + (1 + k) N, and with add_a set
 // (a rescale folded in) acc P^-1 + add of limb l to down_x.  Limbs taken down
-// are not written to acc.
+// are not written to acc.  With rot_a set the product stays in P*Q and leaves
+// rotated instead (acc is not written): rot_b = sigma(acc_b + c0') + base_b, rot_a =
+// sigma(acc_a) + base_a on every limb, c0' as in ExtRotJob; no output may alias
+// add0 or own, a base may be its output.  rot_down: the first pass of the inverse
+// transform of rot_a's special limbs, for the ModDown that follows.
 struct KskJob {
     const uint64_t* ext;  // [nd][l+1+K][N]
     const uint64_t* own;  // [l+1][N] evaluation-form source (own-digit positions)
@@ -198,6 +202,14 @@ struct KskJob {
     uint64_t* down_b;
     const uint64_t* add_a;  // [l+1][N] addends, or nullptr
     const uint64_t* add_b;
+    uint64_t* rot_a;        // [l+1+K][N], or nullptr
+    uint64_t* rot_b;
+    const uint64_t* base_a;
+    const uint64_t* base_b;
+    const uint64_t* add0;   // a Q-basis c0 (scale_p: times P on the Q limbs) or a P*Q one
+    uint64_t* rot_down;     // [K][N], or nullptr
+    uint32_t autok;         // k^-1 mod 2N of sigma_k
+    int scale_p;
 };
 constexpr int KSK_INLINE = 2;
 using KskJobs = JobList<KskJob, KSK_INLINE>;
@@ -378,8 +390,9 @@ hipError_t launch_tensor_rows(const DevTables& T, const TensorJobs& jobs, int ma
 hipError_t launch_modup_cols(const DevTables& T, const ModUpJobs& jobs, int max_nd, int max_nl, hipStream_t stream);
 // Second pass of the digits' transforms and the key-switch inner product
 // (several jobs: sorted by key).  eval: the digits' second pass has been run.
+// rot: every job leaves rotated (KskJob::rot_a).
 hipError_t launch_rows_ksk(const DevTables& T, const KskJobs& jobs, int max_npos, hipStream_t stream,
-                           bool eval = false);
+                           bool eval = false, bool rot = false);
 // ModDown conversion (+ rescale) and the first pass of its outputs' transform.
 hipError_t launch_moddown_cols(const DevTables& T, const ModDownJobs& jobs, int max_nl, bool rescale,
                                hipStream_t stream);

@@ -172,7 +172,7 @@ struct KskGrid {
     int q_primes;  // primes below q_primes are the Q primes of the list's top level
 };
 
-template <int LOGN, bool EVAL>
+template <int LOGN, bool EVAL, bool ROT>
 __global__ void __launch_bounds__(FRows<LOGN>::NTR, 4) k_rows_ksk(DevTables T, KskJobs L, KskGrid g) {
     using G = FRows<LOGN>;
     constexpr int TPL = G::N1 / G::RR;
@@ -228,6 +228,54 @@ __global__ void __launch_bounds__(FRows<LOGN>::NTR, 4) k_rows_ksk(DevTables T, K
             ar.mac(sa[0], v[0], a.x), ar.mac(sa[1], v[1], a.y), ar.mac(sa[2], v[2], ah.x), ar.mac(sa[3], v[3], ah.y);
             ar.mac(sb[0], v[0], b.x), ar.mac(sb[1], v[1], b.y), ar.mac(sb[2], v[2], bh.x), ar.mac(sb[3], v[3], bh.y);
         };
+        // sigma(sum + c0') + base: sigma sends a row to one row (its columns are scattered
+        // in LDS, the index map is STORE_MODDOWN_AUTO's), so what goes out is whole rows
+        // and the kernel that gathered (23 us a giant step of 25 + 8 limbs) is not run
+        auto rotate = [&](typename A::Sum* sums, uint64_t* out, const uint64_t* base, const uint64_t* add0,
+                          uint64_t* rdown) {
+            uint64_t u[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) u[k] = ar.canon_in(ar.sum(sums[k], P));
+            if (add0 && (!J.scale_p || !special)) {
+                const u64x2 f0 = ld2(add0 + limb + x0), f1 = ld2(add0 + limb + x0 + 2);
+                uint64_t f[4] = {f0.x, f0.y, f1.x, f1.y};
+                if (J.scale_p) {
+                    const ShoupConst pm = cld(T.pmodq + pid);
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) f[k] = mul_shoup(f[k], pm.w, pm.wp, P.p);
+                }
+#pragma unroll
+                for (int k = 0; k < 4; ++k) u[k] = addmod(u[k], f[k], P.p);
+            }
+            const uint32_t cx = (uint32_t)(((2ull * brev_bits(r, G::K1) + 1) * J.autok) & (2ull * G::N - 1));
+            const uint32_t rdst = brev_bits((cx & (2u * G::N1 - 1)) >> 1, G::K1), coff = cx >> (G::K1 + 1);
+            uint64_t* words = reinterpret_cast<uint64_t*>(sub);
+            lds_sync<G::WAVE>();
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                words[lds_off(brev_bits((brev_bits(G::mem(t, k), G::K2) * J.autok + coff) & (G::N2 - 1), G::K2))] = u[k];
+            lds_sync<G::WAVE>();
+#pragma unroll
+            for (int k = 0; k < 4; ++k) u[k] = words[lds_off(G::mem(t, k))];
+            const uint32_t y0 = rdst * G::N2 + G::mem(t, 0);
+            if (base) {
+                const u64x2 f0 = ld2(base + limb + y0), f1 = ld2(base + limb + y0 + 2);
+                u[0] = addmod(u[0], f0.x, P.p), u[1] = addmod(u[1], f0.y, P.p);
+                u[2] = addmod(u[2], f1.x, P.p), u[3] = addmod(u[3], f1.y, P.p);
+            }
+            st2(out + limb + y0, u[0], u[1]);
+            st2(out + limb + y0 + 2, u[2], u[3]);
+            if (rdown && special) {
+                V a[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) a[k] = ar.from(u[k]);
+                lds_sync<G::WAVE>();  // the words are read
+                inv_row<G>(ar, sub, a, t, G::N1 + rdst, A::inv(T) + (size_t)pid * G::N);
+                gu64* o = gp(rdown) + (size_t)(pos - nl) * G::N;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) o[rdst * G::N2 + elem<2, G::LOL, G::NBI>(t, k)] = A::pack(a[k]);
+            }
+        };
         auto finish = [&](typename A::Sum* sums, uint64_t* acc, uint64_t* down, const uint64_t* add) {
             V a[4];
 #pragma unroll
@@ -257,8 +305,13 @@ __global__ void __launch_bounds__(FRows<LOGN>::NTR, 4) k_rows_ksk(DevTables T, K
             digit(d, v);
             mac(sa, sb, d, v);
         }
-        finish(sa, J.acc_a, J.down_a, J.add_a);
-        finish(sb, J.acc_b, J.down_b, J.add_b);
+        if constexpr (ROT) {
+            rotate(sa, J.rot_a, J.base_a, nullptr, J.rot_down);
+            rotate(sb, J.rot_b, J.base_b, J.add0, nullptr);
+        } else {
+            finish(sa, J.acc_a, J.down_a, J.add_a);
+            finish(sb, J.acc_b, J.down_b, J.add_b);
+        }
     });
 }
 
@@ -330,7 +383,7 @@ hipError_t launch_modup_cols(const DevTables& T, const ModUpJobs& L, int max_nd,
     return by_logn(T.logN, [&](auto ln) { modup_cols_a<decltype(ln)::value>(T, L, max_nd, targets, s); });
 }
 
-hipError_t launch_rows_ksk(const DevTables& T, const KskJobs& L, int max_npos, hipStream_t s, bool eval) {
+hipError_t launch_rows_ksk(const DevTables& T, const KskJobs& L, int max_npos, hipStream_t s, bool eval, bool rot) {
     if (L.n <= 0 || max_npos <= 0) return hipSuccess;
     if (!fused_ok(T)) return hipErrorInvalidValue;
     return by_logn(T.logN, [&](auto ln) {
@@ -340,10 +393,15 @@ hipError_t launch_rows_ksk(const DevTables& T, const KskJobs& L, int max_npos, h
         const size_t items = (size_t)L.n * max_npos * TPL;
         const XcdGrid x = xcd_grid(items, TPL * L.n);
         const KskGrid g{(uint32_t)items, x.chunk, FastDiv(L.n, items), max_npos - T.K};
-        if (eval)
-            hipLaunchKernelGGL((k_rows_ksk<LN, true>), x.grid, dim3(G::NTR), 0, s, T, L, g);
+        const dim3 b(G::NTR);
+        if (eval && rot)
+            hipLaunchKernelGGL((k_rows_ksk<LN, true, true>), x.grid, b, 0, s, T, L, g);
+        else if (eval)
+            hipLaunchKernelGGL((k_rows_ksk<LN, true, false>), x.grid, b, 0, s, T, L, g);
+        else if (rot)
+            hipLaunchKernelGGL((k_rows_ksk<LN, false, true>), x.grid, b, 0, s, T, L, g);
         else
-            hipLaunchKernelGGL((k_rows_ksk<LN, false>), x.grid, dim3(G::NTR), 0, s, T, L, g);
+            hipLaunchKernelGGL((k_rows_ksk<LN, false, false>), x.grid, b, 0, s, T, L, g);
     });
 }
 
