@@ -427,6 +427,25 @@ void Context::build_tables(const std::vector<uint64_t>& roots) {
     const size_t o_isd = place(is_moddown.size() * sizeof(ShoupConst));
     const size_t o_mum = place(modup_mat.size() * 8);
     const size_t o_mdm = place(moddown_mat.size() * 8);
+    // the same entries as ConvFp for targets on the FP64 units
+    const auto conv_fp_table = [&](const std::vector<uint64_t>& mat, int row) {
+        std::vector<ConvFp> out(mat.size(), ConvFp{0, 0, 0, 0});
+        const auto split = [](uint64_t m, uint64_t p, int32_t& lo, int32_t& hi) {
+            const int64_t b = m > p / 2 ? (int64_t)m - (int64_t)p : (int64_t)m;
+            hi = (int32_t)((b + ((int64_t)1 << 28)) >> 29);
+            lo = (int32_t)(b - (int64_t)hi * ((int64_t)1 << 29));
+        };
+        for (size_t e = 0; e < mat.size(); ++e) {
+            const int t = (int)(e / row % np);
+            if (!primes[t].fp) continue;
+            split(mat[e], q[t], out[e].lo, out[e].hi);
+            split(h_mulmod(mat[e], ((uint64_t)1 << 30) % q[t], q[t]), q[t], out[e].lo30, out[e].hi30);
+        }
+        return out;
+    };
+    const std::vector<ConvFp> modup_fp = conv_fp_table(modup_mat, AP), moddown_fp = conv_fp_table(moddown_mat, KP);
+    const size_t o_muf = place(modup_fp.size() * sizeof(ConvFp));
+    const size_t o_mdf = place(moddown_fp.size() * sizeof(ConvFp));
     const size_t o_pinv = place(pinv.size() * sizeof(ShoupConst));
     const size_t o_pmq = place(pmodq.size() * sizeof(ShoupConst));
     const size_t o_qli = place(qlinv.size() * sizeof(ShoupConst));
@@ -444,6 +463,8 @@ void Context::build_tables(const std::vector<uint64_t>& roots) {
     put(o_isd, is_moddown.data(), is_moddown.size() * sizeof(ShoupConst));
     put(o_mum, modup_mat.data(), modup_mat.size() * 8);
     put(o_mdm, moddown_mat.data(), moddown_mat.size() * 8);
+    put(o_muf, modup_fp.data(), modup_fp.size() * sizeof(ConvFp));
+    put(o_mdf, moddown_fp.data(), moddown_fp.size() * sizeof(ConvFp));
     put(o_pinv, pinv.data(), pinv.size() * sizeof(ShoupConst));
     put(o_pmq, pmodq.data(), pmodq.size() * sizeof(ShoupConst));
     put(o_qli, qlinv.data(), qlinv.size() * sizeof(ShoupConst));
@@ -467,6 +488,8 @@ void Context::build_tables(const std::vector<uint64_t>& roots) {
     T.iscale_moddown = (const ShoupConst*)(b + o_isd);
     T.modup_mat = (const uint64_t*)(b + o_mum);
     T.moddown_mat = (const uint64_t*)(b + o_mdm);
+    T.modup_fp = (const ConvFp*)(b + o_muf);
+    T.moddown_fp = (const ConvFp*)(b + o_mdf);
     T.pinv = (const ShoupConst*)(b + o_pinv);
     T.pmodq = (const ShoupConst*)(b + o_pmq);
     T.qlinv = (const ShoupConst*)(b + o_qli);

@@ -32,6 +32,13 @@ struct Half2 {
     uint32_t lo, hi;  // x = hi * 2^30 + lo
 };
 __device__ __forceinline__ Half2 split30(uint64_t x) { return Half2{(uint32_t)(x & 0x3fffffffu), (uint32_t)(x >> 30)}; }
+// The halves of a value that stays in registers through a kernel: as words of
+// their own, or the compiler keeps the 64-bit values that they were cut from.
+__device__ __forceinline__ Half2 split30_held(uint64_t x) {
+    Half2 h = split30(x);
+    asm("" : "+v"(h.lo), "+v"(h.hi));
+    return h;
+}
 __device__ __forceinline__ void mac_split(Acc4& a, Half2 x, Half2 y) {
     a.s00 = (uint64_t)x.lo * y.lo + a.s00;
     a.s01 = (uint64_t)x.lo * y.hi + a.s01;
@@ -57,5 +64,33 @@ template <int A>
 struct MatRow {
     uint64_t v[A];
 };
+
+// sum x_i m_i mod p as a double of at most (1/2 + 2^-16) p, exact, for p < 2^50, A <= 10
+// and x_i < 2^60.  The halves of x_i take constants of their own, so that two
+// signed sums are enough, U of lo and V of hi parts: |U| <= 20 2^58, |V| <= 20 2^50.
+// V 2^29 + U is regrouped as D 2^32 + l, D an integer below 2^53 and l one word,
+// and is at most 10 2^30 p, so its rounded quotient is off by little and what is
+// left after it a small integer.  11 operations follow the sums, where four
+// unsigned sums and a 128-bit reduction took 45.
+template <int A>
+struct MatRowFp {
+    ConvFp v[A];
+};
+template <int A>
+__device__ __forceinline__ double conv_fp(const Half2* x, const MatRowFp<A>& row, const PrimeInfo& P) {
+    int64_t u = 0, v = 0;
+#pragma unroll
+    for (int i = 0; i < A; ++i) {
+        const int64_t xl = (int32_t)x[i].lo, xh = (int32_t)x[i].hi;
+        u = xl * row.v[i].lo + u;
+        v = xl * row.v[i].hi + v;
+        u = xh * row.v[i].lo30 + u;
+        v = xh * row.v[i].hi30 + v;
+    }
+    u = (int64_t)((uint64_t)(uint32_t)v * 0x20000000u + (uint64_t)u);
+    const double h = __builtin_fma((double)(int32_t)(v >> 32), 0x1p29, (double)(int32_t)(u >> 32)) * 0x1p32;
+    const double l = (double)(uint32_t)u;
+    return __builtin_fma(-__builtin_rint((h + l) * P.pinv), P.pd, h) + l;
+}
 
 }  // namespace fides

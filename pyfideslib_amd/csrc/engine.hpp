@@ -15,6 +15,12 @@
 
 namespace fides {
 
+// A conversion constant m of a target below 2^50, with x = xl + 2^30 xh: balanced
+// residues m = hi 2^29 + lo of m and m30 = hi30 2^29 + lo30 of 2^30 m.
+struct ConvFp {
+    int32_t lo, hi, lo30, hi30;
+};
+
 // Device constant tables (pointers into one device allocation), passed to
 // every kernel by value.
 struct DevTables {
@@ -30,6 +36,8 @@ struct DevTables {
     const ShoupConst* iscale_moddown;  // [K][2]   N^-1 * PHatInvModp
     const uint64_t* modup_mat;         // [dnum][alpha size-1][np target][conv_bound(alpha) i]  PartQlHatModp
     const uint64_t* moddown_mat;       // [np target][conv_bound(K) k]  PHatModq
+    const ConvFp* modup_fp;            // the same entries for targets on the FP64 units
+    const ConvFp* moddown_fp;
     const ShoupConst* pinv;            // [np]     P^-1 mod q_i
     const ShoupConst* pmodq;           // [np]     P mod q_i (0 for the special primes)
     const ShoupConst* qlinv;           // [L+1 l][L+1 i] q_l^-1 mod q_i

@@ -102,7 +102,7 @@ __global__ void __launch_bounds__(512, 4) k_modup_cols(DevTables T, ModUpJobs L,
         for (int i = 0; i < A; ++i)
 #pragma unroll
             for (int c = 0; c < G::CPT; ++c)
-                x[c][i] = split30(i < size ? S.s.tile[i][G::c_col(tid) + c][lds_off(G::c_row(tid))] : 0);
+                x[c][i] = split30_held(i < size ? S.s.tile[i][G::c_col(tid) + c][lds_off(G::c_row(tid))] : 0);
         __syncthreads();  // the targets take over the LDS
     } else {
         uint64_t v[A][G::CPT];
@@ -119,9 +119,9 @@ __global__ void __launch_bounds__(512, 4) k_modup_cols(DevTables T, ModUpJobs L,
 #pragma unroll
         for (int i = 0; i < A; ++i)
 #pragma unroll
-            for (int c = 0; c < G::CPT; ++c) x[c][i] = split30(i < size ? v[i][c] : 0);
+            for (int c = 0; c < G::CPT; ++c) x[c][i] = split30_held(i < size ? v[i][c] : 0);
     }
-    const uint64_t* M = T.modup_mat + (size_t)(d * T.alpha + size - 1) * T.np * A;
+    const size_t m_at = (size_t)(d * T.alpha + size - 1) * T.np * A;
     uint64_t* out = J.ext + (size_t)d * (nl + T.K) * G::N;
     auto pos_of = [&](int m) { const int k = m * TG + tg; return k < start ? k : k + size; };
     auto pid_of = [&](int k) { return pos_pid(pos_of(k), nl, 0, T.L + 1); };
@@ -137,13 +137,8 @@ __global__ void __launch_bounds__(512, 4) k_modup_cols(DevTables T, ModUpJobs L,
             if (k + i >= k1) continue;
             const int pid = pid_of(k + i);
             const PrimeInfo P = cld(T.primes + pid);
-            const MatRow<A> row = cld(reinterpret_cast<const MatRow<A>*>(M + (size_t)pid * A));
-#pragma unroll
-            for (int c = 0; c < G::CPT; ++c) {
-                uint64_t lo, hi;
-                conv_acc<A>(x[c], row, lo, hi);
-                S.t.tile[buf][i][G::c_col(tid) + c][lds_off(G::c_row(tid))] = conv_word(T, pid, P, lo, hi);
-            }
+            conv_tile<A>(T, pid, P, x, T.modup_mat + m_at, T.modup_fp + m_at, &S.t.tile[buf][i][G::c_col(tid)],
+                         lds_off(G::c_row(tid)));
         }
         tw.put(S, buf, s_tgt, s_row);
         if (k + G::TB < k1) tw.load(T, s_pid(k + G::TB), s_row);

@@ -38,7 +38,7 @@ __global__ void __launch_bounds__(512, 4) k_moddown_cols(DevTables T, ModDownJob
             for (int c = 0; c < G::CPT; ++c) {
                 const uint64_t w = S.s.tile[i][G::c_col(tid) + c][lds_off(G::c_row(tid))];
                 if (i < KK)
-                    x[c][i < KK ? i : 0] = split30(w);
+                    x[c][i < KK ? i : 0] = split30_held(w);
                 else
                     top[c] = w;
             }
@@ -62,20 +62,23 @@ __global__ void __launch_bounds__(512, 4) k_moddown_cols(DevTables T, ModDownJob
 #pragma unroll
         for (int i = 0; i < KK; ++i)
 #pragma unroll
-            for (int c = 0; c < G::CPT; ++c) x[c][i] = split30(v[i][c]);
+            for (int c = 0; c < G::CPT; ++c) x[c][i] = split30_held(v[i][c]);
     }
-    const uint64_t* M = T.moddown_mat;
+    // the dropped limb less its converted part, centered on a rescale; as a double
+    // where its prime is on the FP64 units, and else in [0, q_l)
     uint64_t half = 0;
+    const bool l_fp = is_fp(T, l);
     if constexpr (RESCALE) {
         const PrimeInfo Pl = cld(T.primes + l);
         const ShoupConst pl = cld(T.pinv + l);
-        const MatRow<KK> row = cld(reinterpret_cast<const MatRow<KK>*>(M + (size_t)l * KK));
+        const MatRow<KK> row = cld(reinterpret_cast<const MatRow<KK>*>(T.moddown_mat + (size_t)l * KK));
         half = Pl.p >> 1;
 #pragma unroll
         for (int c = 0; c < G::CPT; ++c) {
             uint64_t lo, hi;
             conv_acc<KK>(x[c], row, lo, hi);
             top[c] = submod(top[c], mul_shoup(reduce128(lo, hi, Pl), pl.w, pl.wp, Pl.p), Pl.p);
+            if (l_fp) top[c] = FpArith::pack(fp_from(top[c]) - (top[c] > half ? Pl.pd : 0.0));
         }
     }
     int buf = 0;
@@ -89,28 +92,42 @@ __global__ void __launch_bounds__(512, 4) k_moddown_cols(DevTables T, ModDownJob
             const int i = c_tgt + q, pid = (k + i) * TG + tg;
             if (k + i >= k1) continue;
             const PrimeInfo P = cld(T.primes + pid);
-            const MatRow<KK> row = cld(reinterpret_cast<const MatRow<KK>*>(M + (size_t)pid * KK));
+            uint64_t(*tile)[G::SC] = &S.t.tile[buf][i][G::c_col(tid)];
+            const uint32_t at = lds_off(G::c_row(tid));
+            if constexpr (RESCALE) {
+                const ShoupConst pi = cld(T.pinv + pid);
+                // centered lift of the dropped limb into q_i
+                auto lift = [&](uint64_t t) {
+                    uint64_t sw = reduce64(t, P);
+                    if (t > half) sw = submod(sw, cld(T.qlmodq + (size_t)l * (T.L + 1) + pid), P.p);
+                    return sw;
+                };
+                if (is_fp(T, pid)) {
+                    const FpArith ar(P);
+                    const MatRowFp<KK> row = cld(reinterpret_cast<const MatRowFp<KK>*>(T.moddown_fp + (size_t)pid * KK));
 #pragma unroll
-            for (int c = 0; c < G::CPT; ++c) {
-                uint64_t lo, hi;
-                conv_acc<KK>(x[c], row, lo, hi);
-                uint64_t word;
-                if constexpr (RESCALE) {
-                    const ShoupConst pi = cld(T.pinv + pid);
-                    uint64_t sw = reduce64(top[c], P);  // centered lift of top into q_i
-                    if (top[c] > half) sw = submod(sw, cld(T.qlmodq + (size_t)l * (T.L + 1) + pid), P.p);
-                    const uint64_t y = reduce128_lazy(lo, hi, P);
-                    if (is_fp(T, pid)) {
-                        const FpArith ar(P);
-                        word = FpArith::pack(ar.scale_add(ar.from_lazy(y), pi, sw));
-                    } else {
-                        const IntArith ar(P);
-                        word = ar.scale_add(ar.from_lazy(y), pi, sw);
+                    for (int c = 0; c < G::CPT; ++c) {
+                        const double s = l_fp ? ar.term_fwd(FpArith::unpack(top[c])) : fp_from(lift(top[c]));
+                        tile[c][at] = FpArith::pack(ar.scale_add(conv_fp<KK>(x[c], row, P), pi, s));
                     }
                 } else {
-                    word = conv_word(T, pid, P, lo, hi);
+                    const IntArith ar(P);
+                    const MatRow<KK> row = cld(reinterpret_cast<const MatRow<KK>*>(T.moddown_mat + (size_t)pid * KK));
+                    const double ql = cld(T.primes + l).pd;
+#pragma unroll
+                    for (int c = 0; c < G::CPT; ++c) {
+                        uint64_t lo, hi;
+                        conv_acc<KK>(x[c], row, lo, hi);
+                        uint64_t t = top[c];
+                        if (l_fp) {
+                            const double td = FpArith::unpack(t);
+                            t = fp_to(td < 0 ? td + ql : td);
+                        }
+                        tile[c][at] = ar.scale_add(ar.from_lazy(reduce128_lazy(lo, hi, P)), pi, lift(t));
+                    }
                 }
-                S.t.tile[buf][i][G::c_col(tid) + c][lds_off(G::c_row(tid))] = word;
+            } else {
+                conv_tile<KK>(T, pid, P, x, T.moddown_mat, T.moddown_fp, tile, at);
             }
         }
         tw.put(S, buf, s_tgt, s_row);

@@ -149,8 +149,8 @@ struct FpArith {
         return fp_reduce(fp_mul(e, fp_from(c.w), p, pinv) + fp_from(f), p, pinv);
     }
     // at most (1/2 + 9/8 + 1) p, a first phase's bound
-    __device__ __forceinline__ V scale_add(V y, const ShoupConst& c, uint64_t s) const {
-        return fp_mul(y, fp_from(c.w), p, pinv) + fp_from(s);
+    __device__ __forceinline__ V scale_add(V y, const ShoupConst& c, double s) const {
+        return fp_mul(y, fp_from(c.w), p, pinv) + s;
     }
     // uncentered constants: fp_mul of a value B returns at most 1/2 + 3B/8; no sum below exceeds 7.1
     __device__ __forceinline__ uint64_t sub_mul(uint64_t e, V v, const ShoupConst& c) const {
