@@ -337,7 +337,7 @@ hipError_t launch_tensor_rows(const DevTables& T, const TensorJobs& L, int max_n
         using G = FRows<decltype(ln)::value>;
         constexpr int TPL = G::N1 / G::RR;
         const size_t items = (size_t)L.n * max_nl * TPL;
-        const XcdGrid x = xcd_grid(items, TPL);
+        const XcdGrid x = xcd_chunks(items, XCD_TILES);
         const RowsGrid g{(uint32_t)items, x.chunk, FastDiv(max_nl, items)};
         hipLaunchKernelGGL((k_tensor_rows<decltype(ln)::value>), x.grid, dim3(G::NTR), 0, s, T, L, g);
     });
@@ -348,7 +348,7 @@ static void modup_cols(const DevTables& T, const ModUpJobs& L, int max_nd, int t
     using G = ConvCols<LOGN>;
     const int tg = fused_groups((size_t)G::TPL * max_nd * L.n, targets, G::TB);
     const size_t items = (size_t)L.n * max_nd * tg * G::TPL;
-    const XcdGrid x = xcd_grid(items, G::TPL);
+    const XcdGrid x = conv_grid(items, G::TPL);
     const ConvGrid g{(uint32_t)items, x.chunk, FastDiv(tg, items), FastDiv(max_nd, items)};
     hipLaunchKernelGGL((k_modup_cols<LOGN, A>), x.grid, dim3(G::NT), 0, s, T, L, g);
 }
@@ -386,7 +386,7 @@ hipError_t launch_rows_ksk(const DevTables& T, const KskJobs& L, int max_npos, h
         using G = FRows<LN>;
         constexpr int TPL = G::N1 / G::RR;
         const size_t items = (size_t)L.n * max_npos * TPL;
-        const XcdGrid x = xcd_grid(items, TPL * L.n);
+        const XcdGrid x = xcd_chunks(items, XCD_TILES);
         const KskGrid g{(uint32_t)items, x.chunk, FastDiv(L.n, items), max_npos - T.K};
         const dim3 b(G::NTR);
         if (eval && rot)

@@ -177,12 +177,16 @@ __device__ __forceinline__ void conv_store(const ConvLds<LOGN, SOURCES>& S, int 
     }
 }
 
-// Grid of a conversion kernel: items (job, [digit,] target group, tile), a
-// chunk of half a limb's tiles to an XCD at a time.
+// Grid of a conversion kernel: items (job, [digit,] target group, tile).
 struct ConvGrid {
     uint32_t items, chunk;
     FastDiv tg, nd;
 };
+// Past 32 limbs of tiles half a limb to an XCD (24 products at 25 limbs: 410 us for the
+// ModUp against 438 with XCD_TILES).
+inline XcdGrid conv_grid(size_t items, int per) {
+    return items <= (size_t)32 * per ? xcd_chunks(items, XCD_TILES) : xcd_grid(items, per);
+}
 // Target groups, of whole rounds of tb targets: about 1024 blocks in all, two
 // rounds of what is resident (512 or 1600 took 5 to 10% longer at N = 2^16, level 24).
 inline int fused_groups(size_t base_blocks, int targets, int tb) {

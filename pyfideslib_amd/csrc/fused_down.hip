@@ -146,7 +146,7 @@ static void moddown_cols(const DevTables& T, const ModDownJobs& L, int targets, 
     using G = ConvCols<LOGN>;
     const int tg = fused_groups((size_t)G::TPL * L.n, targets, G::TB);
     const size_t items = (size_t)L.n * tg * G::TPL;
-    const XcdGrid x = xcd_grid(items, G::TPL);
+    const XcdGrid x = conv_grid(items, G::TPL);
     const ConvGrid g{(uint32_t)items, x.chunk, FastDiv(tg, items), FastDiv(1, items)};
     if (rescale)
         hipLaunchKernelGGL((k_moddown_cols<LOGN, KK, true>), x.grid, dim3(G::NT), 0, s, T, L, g);

@@ -516,13 +516,24 @@ struct XcdGrid {
     uint32_t chunk;
     dim3 grid;  // a whole number of rounds of chunks: items beyond the real ones return
 };
-// items tiles, per of them to a limb
-inline XcdGrid xcd_grid(size_t items, int per) {
+inline XcdGrid xcd_chunks(size_t items, size_t c) {
     const size_t each = (items + 7) / 8;
-    size_t c = items <= (size_t)32 * per ? each : (size_t)(per > 1 ? per / 2 : 1);
+    c = c < each ? c : each;
     c = c ? c : 1;
     return XcdGrid{(uint32_t)c, dim3((unsigned)((items + 8 * c - 1) / (8 * c) * (8 * c)))};
 }
+// items tiles, per of them to a limb
+inline XcdGrid xcd_grid(size_t items, int per) {
+    return xcd_chunks(items, items <= (size_t)32 * per ? items : (size_t)(per > 1 ? per / 2 : 1));
+}
+// Kernels with arithmetic of their own between the passes (the inner product,
+// the tensor, small conversions): what is slow about a 64-bit limb, and the end of
+// the launch, have to be spread over the XCDs more than the passes' tiles have
+// to stay on one; 2 to 12 tiles take the same time.  At N = 2^16, against xcd_grid:
+// inner product of 25 + 8 limbs 53.9 -> 50.0 us, of 6 + 8 19.6 -> 15.6, for 9 keys
+// at 18 + 8 197 -> 165; tensor 26.1 -> 24.7; conversions 41.6 -> 40.3 and
+// 30.8 -> 28.4.  The transforms are the other way round (25 limbs inverse: 21.3 -> 22.5).
+constexpr int XCD_TILES = 8;
 
 // The job and position of flattened limb a: a device list is walked through
 // its limb map; an inline list has `most` limbs per job.  False: nothing to do.
