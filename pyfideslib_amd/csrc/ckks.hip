@@ -468,9 +468,28 @@ void eval_square(Context& c, const Ciphertext& a, Ciphertext& out, bool do_resca
 
 // Rescale with caller-provided scratch: top = the coefficient-form top limbs
 // of both parts (2 limbs), mid = the forward NTT's intermediate (2 l limbs).
-static void rescale_with(Context& c, Ciphertext& a, uint64_t* top, uint64_t* mid) {
+static void rescale_with(Context& c, Ciphertext& a, uint64_t* top, uint64_t* mid, const uint64_t* x0 = nullptr,
+                         const uint64_t* x1 = nullptr, const uint64_t* w = nullptr) {
     const int l = a.level;
     const size_t N = c.N;
+    if (rescale_ok(c.T)) {
+        RescaleJobs rj = inline_list<RescaleJobs>();
+        rj.inl[0] = RescaleJob{w ? x0 : a.c0(), w, top, mid, l, 0};
+        rj.inl[1] = RescaleJob{w ? x1 : a.c1(), w, top + N, mid + l * N, l, 0};
+        rj.n = 2;
+        ck(launch_rescale_cols(c.T, rj, l, c.stream), "rescale columns");
+        NttJob f0 = ntt_job(nullptr, mid, a.c0(), l, l, 0);
+        NttJob f1 = ntt_job(nullptr, mid + l * N, a.c1(), l, l, 0);
+        f0.level = f1.level = l;
+        f0.aux = x0;
+        f1.aux = x1;
+        f0.add = f1.add = w;
+        run_ntt(c, {f0, f1}, false, LOAD_PLAIN, w ? STORE_MUL_RESCALE : STORE_RESCALE, NTT_PASS2);
+        a.level = l - 1;
+        a.noise /= c.mod_reduce_factor[l];
+        a.noise_level -= 1;
+        return;
+    }
     NttJob i0 = ntt_job(a.c0() + l * N, top, top, 1, 1, l);
     NttJob i1 = ntt_job(a.c1() + l * N, top + N, top + N, 1, 1, l);
     run_ntt(c, {i0, i1}, true);
@@ -487,6 +506,12 @@ void rescale(Context& c, Ciphertext& a) {
     if (a.level < 1) throw Error(E_LEVEL, "cannot rescale at level 0");
     DevBuf top(&c.pool, 2 * (size_t)c.N), mid(&c.pool, 2 * (size_t)a.level * c.N);
     rescale_with(c, a, top.ptr, mid.ptr);
+}
+
+// out's metadata is the product's, its limbs are not yet: out = (x0, x1) w rescaled.
+void mul_rescale(Context& c, const uint64_t* x0, const uint64_t* x1, const uint64_t* w, Ciphertext& out) {
+    DevBuf top(&c.pool, 2 * (size_t)c.N), mid(&c.pool, 2 * (size_t)out.level * c.N);
+    rescale_with(c, out, top.ptr, mid.ptr, x0, x1, w);
 }
 
 static void ew(Context& c, const Ciphertext& a, const Ciphertext& b, Ciphertext& out, int op) {

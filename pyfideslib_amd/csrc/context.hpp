@@ -255,6 +255,7 @@ void load_key(Context& c, KeySwitchingKey& k, const uint64_t* a, const uint64_t*
 void eval_mult(Context& c, const Ciphertext& a, const Ciphertext& b, Ciphertext& out, bool rescale);
 void eval_square(Context& c, const Ciphertext& a, Ciphertext& out, bool rescale);
 void rescale(Context& c, Ciphertext& a);
+void mul_rescale(Context& c, const uint64_t* x0, const uint64_t* x1, const uint64_t* w, Ciphertext& out);
 void eval_add(Context& c, const Ciphertext& a, const Ciphertext& b, Ciphertext& out);
 void eval_sub(Context& c, const Ciphertext& a, const Ciphertext& b, Ciphertext& out);
 void eval_rotate(Context& c, const Ciphertext& a, int index, Ciphertext& out);

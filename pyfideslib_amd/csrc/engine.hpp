@@ -146,7 +146,8 @@ enum NttStore {
     STORE_MODDOWN = 1,
     STORE_RESCALE = 2,
     STORE_MODDOWN_RESCALE = 3,
-    STORE_MODDOWN_AUTO = 4  // STORE_MODDOWN, then the automorphism of NttJob::autok
+    STORE_MODDOWN_AUTO = 4,  // STORE_MODDOWN, then the automorphism of NttJob::autok
+    STORE_MUL_RESCALE = 5    // STORE_RESCALE of the product aux * add (dst may be either)
 };
 enum IScale { ISCALE_PLAIN = 0, ISCALE_MODUP = 1, ISCALE_MODDOWN = 2 };
 
@@ -166,6 +167,19 @@ struct NttJob {
     uint32_t autok;       // STORE_MODDOWN_AUTO: k^-1 mod 2N of the automorphism X -> X^k
 };
 constexpr int NTT_INLINE = 8;
+
+// The limb that a rescale of one polynomial drops (of a, or of a w) and the
+// first pass of its lifts' transform.
+struct RescaleJob {
+    const uint64_t* a;  // [l+1][N]
+    const uint64_t* w;  // factor, or nullptr
+    uint64_t* top;      // [N] scratch
+    uint64_t* y;        // [l][N]
+    int level;          // l
+    int pad;
+};
+constexpr int RESCALE_INLINE = 2;
+using RescaleJobs = JobList<RescaleJob, RESCALE_INLINE>;
 using NttJobs = JobList<NttJob, NTT_INLINE>;
 
 struct TensorJob {
@@ -401,6 +415,9 @@ hipError_t launch_modup_cols(const DevTables& T, const ModUpJobs& jobs, int max_
 // rot: every job leaves rotated (KskJob::rot_a).
 hipError_t launch_rows_ksk(const DevTables& T, const KskJobs& jobs, int max_npos, hipStream_t stream,
                            bool eval = false, bool rot = false);
+// A rescale up to the second pass of its transform, in two launches (rescale_ok).
+bool rescale_ok(const DevTables& T);
+hipError_t launch_rescale_cols(const DevTables& T, const RescaleJobs& jobs, int max_level, hipStream_t stream);
 // ModDown conversion (+ rescale) and the first pass of its outputs' transform.
 hipError_t launch_moddown_cols(const DevTables& T, const ModDownJobs& jobs, int max_nl, bool rescale,
                                hipStream_t stream);

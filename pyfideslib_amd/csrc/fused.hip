@@ -12,9 +12,6 @@
 namespace fides {
 
 // ------------------------------------------------ tensor + inverse rows ----
-template <int LOGN>
-using FRows = RowGeom<(LOGN + 1) / 2, LOGN / 2, 2, (LOGN >= 15 ? 256 : 64) / ((1 << (LOGN / 2)) / 4)>;
-
 struct RowsGrid {
     uint32_t items, chunk;
     FastDiv npos;
@@ -317,19 +314,6 @@ bool fused_ok(const DevTables& T) {
 }
 
 bool fused_inv_cols(const DevTables& T) { return fused_ok(T) && T.logN <= CONV_INV_LOGN; }
-
-template <class F>
-static hipError_t by_logn(int logN, F&& f) {
-    switch (logN) {
-        case 12: f(std::integral_constant<int, 12>{}); break;
-        case 13: f(std::integral_constant<int, 13>{}); break;
-        case 14: f(std::integral_constant<int, 14>{}); break;
-        case 15: f(std::integral_constant<int, 15>{}); break;
-        case 16: f(std::integral_constant<int, 16>{}); break;
-        default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
-}
 
 hipError_t launch_tensor_rows(const DevTables& T, const TensorJobs& L, int max_nl, hipStream_t s) {
     if (L.n <= 0 || max_nl <= 0) return hipSuccess;

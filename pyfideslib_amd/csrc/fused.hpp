@@ -10,6 +10,23 @@ constexpr int FUSED_CONV_MAX = 10;  // source limbs of a conversion
 constexpr int FUSED_DIGITS = 4;
 constexpr int CONV_INV_LOGN = 14;
 
+// Rows of the second pass: as many per block as fill one wave or four.
+template <int LOGN>
+using FRows = RowGeom<(LOGN + 1) / 2, LOGN / 2, 2, (LOGN >= 15 ? 256 : 64) / ((1 << (LOGN / 2)) / 4)>;
+
+template <class F>
+static hipError_t by_logn(int logN, F&& f) {
+    switch (logN) {
+        case 12: f(std::integral_constant<int, 12>{}); break;
+        case 13: f(std::integral_constant<int, 13>{}); break;
+        case 14: f(std::integral_constant<int, 14>{}); break;
+        case 15: f(std::integral_constant<int, 15>{}); break;
+        case 16: f(std::integral_constant<int, 16>{}); break;
+        default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
 // Unsigned division by a launch constant d of values up to most: one multiply
 // where it is exact (most d < 2^32), else the division itself.
 struct FastDiv {
@@ -59,7 +76,7 @@ struct ConvCols {
 // per target group, which costs arithmetic that the idle CUs have to spare).
 template <int LOGN>
 constexpr bool conv_inv() { return LOGN <= CONV_INV_LOGN; }
-template <int LOGN, int SOURCES>
+template <int LOGN, int SOURCES, bool INV = conv_inv<LOGN>()>
 struct ConvLds {
     using G = ConvCols<LOGN>;
     struct Targets {
@@ -73,15 +90,15 @@ struct ConvLds {
     struct None {};
     union {
         Targets t;
-        std::conditional_t<conv_inv<LOGN>(), Sources, None> s;  // before the first target
+        std::conditional_t<INV, Sources, None> s;  // before the first target
     };
 };
 
 // The column pass of the inverse transform of n source limbs (limb(i): what the
 // row pass left, pid(i), scale(i): the limb's last-stage pair) on the block's
 // columns; coefficient (row, column) of limb i ends at S.s.tile[i][column][row].
-template <int LOGN, int SOURCES, class LIMB, class PID, class SCALE>
-__device__ __forceinline__ void conv_sources(const DevTables& T, ConvLds<LOGN, SOURCES>& S, int n, uint32_t col0,
+template <int LOGN, int SOURCES, bool INV, class LIMB, class PID, class SCALE>
+__device__ __forceinline__ void conv_sources(const DevTables& T, ConvLds<LOGN, SOURCES, INV>& S, int n, uint32_t col0,
                                              const LIMB& limb, const PID& pid_of, const SCALE& scale) {
     using G = ConvCols<LOGN>;
     constexpr int LOL = inv_last_lo<2, G::K1>(), NBI = G::K1 - LOL, PAIRS = G::COEF / 2;
@@ -126,8 +143,8 @@ __device__ __forceinline__ void conv_sources(const DevTables& T, ConvLds<LOGN, S
 }
 
 // The column pass of a wave's target (prime pid) on the buffer's tile.
-template <int LOGN, int SOURCES>
-__device__ __forceinline__ void conv_columns(const DevTables& T, int pid, ConvLds<LOGN, SOURCES>& S, int buf, int i) {
+template <int LOGN, int SOURCES, bool INV>
+__device__ __forceinline__ void conv_columns(const DevTables& T, int pid, ConvLds<LOGN, SOURCES, INV>& S, int buf, int i) {
     using G = ConvCols<LOGN>;
     const uint32_t t = G::n_t(threadIdx.x), cc = G::n_col(threadIdx.x);
     const PrimeInfo P = cld(T.primes + pid);
@@ -155,8 +172,8 @@ struct ConvTw {
         else
             w = T.tw_fwd[(size_t)pid * T.N + r];
     }
-    template <int LOGN, int SOURCES>
-    __device__ __forceinline__ void put(ConvLds<LOGN, SOURCES>& S, int buf, int i, int r) const {
+    template <int LOGN, int SOURCES, bool INV>
+    __device__ __forceinline__ void put(ConvLds<LOGN, SOURCES, INV>& S, int buf, int i, int r) const {
         if (fp)
             reinterpret_cast<uint64_t*>(S.t.tw[buf][i])[r] = w.w;
         else
@@ -164,8 +181,8 @@ struct ConvTw {
     }
 };
 // The tile's rows to limb `out`: 2048 words of TB targets, 4 a thread.
-template <int LOGN, int SOURCES, class F>
-__device__ __forceinline__ void conv_store(const ConvLds<LOGN, SOURCES>& S, int buf, uint32_t col0, const F& limb) {
+template <int LOGN, int SOURCES, bool INV, class F>
+__device__ __forceinline__ void conv_store(const ConvLds<LOGN, SOURCES, INV>& S, int buf, uint32_t col0, const F& limb) {
     using G = ConvCols<LOGN>;
 #pragma unroll
     for (int q = 0; q < 2; ++q) {

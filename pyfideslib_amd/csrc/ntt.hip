@@ -30,6 +30,8 @@
 //                 centered into q_i (OpenFHE SwitchModulus) -- rescale.
 //   STORE_MODDOWN (forward, pass 2): y = (acc - v) P^-1 (+ addend) -- ModDown.
 //   STORE_RESCALE (forward, pass 2): y = (x - v) q_l^-1 -- rescale.
+//   STORE_MUL_RESCALE (forward, pass 2): y = (x w - v) q_l^-1 -- rescale of a
+//                 product with a plaintext, which is not written out before.
 //   STORE_MODDOWN_RESCALE (forward, pass 2): y = (acc P^-1 + add - v) q_l^-1 --
 //                 ModDown and rescale merged (k_moddown_conv explains the form).
 //   STORE_MODDOWN_AUTO (forward, pass 2): STORE_MODDOWN, then the automorphism
@@ -327,6 +329,8 @@ static void fwd_rows(const DevTables& T, const NttJobs& L, int limbs, int store,
         hipLaunchKernelGGL((k_ntt_fwd_rows<LOGN, W, STORE_MODDOWN_AUTO>), g, b, 0, s, T, L, n);
     else if (store == STORE_MODDOWN_RESCALE)
         hipLaunchKernelGGL((k_ntt_fwd_rows<LOGN, W, STORE_MODDOWN_RESCALE>), g, b, 0, s, T, L, n);
+    else if (store == STORE_MUL_RESCALE)
+        hipLaunchKernelGGL((k_ntt_fwd_rows<LOGN, W, STORE_MUL_RESCALE>), g, b, 0, s, T, L, n);
     else if (store == STORE_RESCALE)
         hipLaunchKernelGGL((k_ntt_fwd_rows<LOGN, W, STORE_RESCALE>), g, b, 0, s, T, L, n);
     else

@@ -96,6 +96,10 @@ struct IntArith {
     __device__ __forceinline__ uint64_t sub_mul_add(uint64_t e, V v, const ShoupConst& c, uint64_t f) const {
         return addmod(sub_mul(e, v, c), f, p);
     }
+    __device__ __forceinline__ uint64_t prod_sub_mul(uint64_t e, uint64_t f, V v, const ShoupConst& d,
+                                                     const PrimeInfo& P) const {
+        return sub_mul(mul(e, f, P), v, d);
+    }
     __device__ __forceinline__ uint64_t mul_add_sub_mul(uint64_t e, const ShoupConst& c, uint64_t f, V v,
                                                         const ShoupConst& d) const {
         return mul_shoup(mul_shoup_lazy(e, c.w, c.wp, p) + f + 8 * p - csub(v, 8 * p), d.w, d.wp, p);
@@ -158,6 +162,10 @@ struct FpArith {
     }
     __device__ __forceinline__ uint64_t sub_mul_add(uint64_t e, V v, const ShoupConst& c, uint64_t f) const {
         return fp_canon(fp_mul(fp_from(e) - v, fp_from(c.w), p, pinv) + fp_from(f), p, pinv);
+    }
+    __device__ __forceinline__ uint64_t prod_sub_mul(uint64_t e, uint64_t f, V v, const ShoupConst& d,
+                                                     const PrimeInfo&) const {
+        return fp_canon(fp_mul(fp_mul(fp_from(e), fp_from(f), p, pinv) - v, fp_from(d.w), p, pinv), p, pinv);
     }
     __device__ __forceinline__ uint64_t mul_add_sub_mul(uint64_t e, const ShoupConst& c, uint64_t f, V v,
                                                         const ShoupConst& d) const {
@@ -433,6 +441,10 @@ struct Epilogue {
             const gu64* dst = gp(J.dst) + limb;
 #pragma unroll
             for (int j = 0; j < G::R; ++j) e0[j] = dst[row + G::mem(t, j)];
+        } else if constexpr (STORE == STORE_MUL_RESCALE) {
+            const gu64 *a = gp(J.aux) + limb, *w = gp(J.add) + limb;
+#pragma unroll
+            for (int j = 0; j < G::R; ++j) e0[j] = a[row + G::mem(t, j)], e1[j] = w[row + G::mem(t, j)];
         }
     }
     // row r of the transform; sub: the row's LDS
@@ -474,6 +486,11 @@ struct Epilogue {
             const ShoupConst qi = cld(T.qlinv + (size_t)J.level * (T.L + 1) + pid);
 #pragma unroll
             for (int j = 0; j < G::R; ++j) dst[row + G::mem(t, j)] = ar.mul_add_sub_mul(e0[j], pinv, e1[j], v[j], qi);
+        } else if constexpr (STORE == STORE_MUL_RESCALE) {
+            const ShoupConst qi = cld(T.qlinv + (size_t)J.level * (T.L + 1) + pid);
+            const PrimeInfo P = cld(T.primes + pid);
+#pragma unroll
+            for (int j = 0; j < G::R; ++j) dst[row + G::mem(t, j)] = ar.prod_sub_mul(e0[j], e1[j], v[j], qi, P);
         } else {  // STORE_RESCALE
             const ShoupConst qi = cld(T.qlinv + (size_t)J.level * (T.L + 1) + pid);
 #pragma unroll

@@ -199,18 +199,26 @@ void eval_mult_plain(Context& c, const Ciphertext& a_in, const Plaintext& pt, Ci
     if (do_rescale && c.scaling_technique == FIXEDMANUAL && a.level < 1)
         throw Error(E_LEVEL, "cannot rescale at level 0");
     const int nl = a.level + 1;
-    EwJobs L = ew_list();
-    L.inl[0] = EwJob{a.c0(), pt.c0(), out.c0(), nl};
-    L.inl[1] = EwJob{a.c1(), pt.c0(), out.c1(), nl};
-    L.n = 2;
-    ck(launch_elementwise(c.T, L, nl, EW_MUL, c.stream), "mult plain");
+    const bool resc = do_rescale && c.scaling_technique == FIXEDMANUAL;
+    const bool fused = resc && rescale_ok(c.T);
+    if (!fused) {
+        EwJobs L = ew_list();
+        L.inl[0] = EwJob{a.c0(), pt.c0(), out.c0(), nl};
+        L.inl[1] = EwJob{a.c1(), pt.c0(), out.c1(), nl};
+        L.n = 2;
+        ck(launch_elementwise(c.T, L, nl, EW_MUL, c.stream), "mult plain");
+    }
+    const uint64_t *x0 = a.c0(), *x1 = a.c1();
     const double noise = a.noise * pt.noise;
     const int nlev = a.noise_level + pt.noise_level, slots = std::max(a.slots, pt.slots);
     out.level = a.level;
     out.noise = noise;
     out.noise_level = nlev;
     out.slots = slots;
-    if (do_rescale && c.scaling_technique == FIXEDMANUAL) rescale(c, out);
+    if (fused)
+        mul_rescale(c, x0, x1, pt.c0(), out);
+    else if (resc)
+        rescale(c, out);
 }
 
 // out = a + pt (c0 only; Ciphertext::addPt).
