@@ -29,7 +29,9 @@
 // is one batched key switch over the whole batch.
 // The operation order is this file's own, so results are checked against the
 // FP64 value of the series, not residue by residue against the reference.
+#include <algorithm>
 #include <cmath>
+#include <map>
 
 #include "context.hpp"
 
@@ -43,6 +45,12 @@ using Scales = std::vector<double>;
 
 std::vector<const Ciphertext*> cptrs(const CtVec& v) {
     std::vector<const Ciphertext*> o;
+    for (const auto& p : v) o.push_back(p.get());
+    return o;
+}
+
+std::vector<Ciphertext*> ptrs(const CtVec& v) {
+    std::vector<Ciphertext*> o;
     for (const auto& p : v) o.push_back(p.get());
     return o;
 }
@@ -79,19 +87,18 @@ struct Cheb {
     // 2 a b - s (s steered onto the product's scale) or 2 a b - k
     CtVec two_ab_minus(const CtVec& a, const CtVec& b, const CtVec* s, double k) {
         CtVec p = mult(cptrs(a), cptrs(b));
-        for (int i = 0; i < B; ++i) {
-            eval_add(c, *p[i], *p[i], *p[i]);
-            if (s) {
-                const Ciphertext& si = *(*s)[i];
-                if (si.level <= p[i]->level) throw Error(E_STATE, "Chebyshev: subtrahend has no level to spare");
-                CtPtr u = ct_create(c);
-                mult_const_to_scale(c, si, p[i]->level + 1, 1.0, p[i]->noise, *u);
-                rescale(c, *u);
-                eval_sub(c, *p[i], *u, *p[i]);
-            } else {
-                add_const_at_scale(c, *p[i], -k, *p[i]);
-            }
+        if (!s) {
+            double_add_const(c, ptrs(p), -k);
+            return p;
         }
+        CtVec u = fresh();
+        for (int i = 0; i < B; ++i) {
+            const Ciphertext& si = *(*s)[i];
+            if (si.level <= p[i]->level) throw Error(E_STATE, "Chebyshev: subtrahend has no level to spare");
+            mult_const_to_scale(c, si, p[i]->level + 1, 1.0, p[i]->noise, *u[i]);
+        }
+        rescale_batch(c, ptrs(u));
+        double_sub_batch(c, ptrs(p), cptrs(u));
         return p;
     }
     static void trim(std::vector<double>& cf) {
@@ -127,6 +134,7 @@ struct Cheb {
     }
     // sum_(j<n) cf[j] T_j at scales S (n <= m + 1; T_m taken from the baby steps)
     CtVec base(const std::vector<double>& cf, const Scales& S) {
+        if (next < leaves.size() && leaves[next].S == S && leaves[next].cf == cf) return std::move(leaves[next++].sum);
         const int lo = base_level(cf) + 1;
         CtVec acc = fresh();
         for (int b = 0; b < B; ++b) {
@@ -143,10 +151,91 @@ struct Cheb {
                 mult_const_to_scale(c, *xs[0], lo, vs[0], S[b], *acc[b]);
             else  // constant: T_1 * 0 + c_0, as the reference's degree-0 case
                 mult_const_to_scale(c, *T[1][b], lo, 0.0, S[b], *acc[b]);
-            rescale(c, *acc[b]);
-            if (!cf.empty() && cf[0] != 0.0) add_const_at_scale(c, *acc[b], cf[0], *acc[b]);
         }
+        rescale_batch(c, ptrs(acc));
+        if (!cf.empty()) add_const_batch(c, ptrs(acc), cf[0]);
         return acc;
+    }
+    // The sums that rec() asks base() for, in its order, with the scales it will
+    // ask for: every operation's effect on level and scale is known beforehand.
+    struct Leaf {
+        std::vector<double> cf;
+        Scales S;
+        CtVec sum;
+    };
+    std::vector<Leaf> leaves;
+    size_t next = 0;
+    Scales plan(std::vector<double> cf, int t, const Scales& S) {
+        trim(cf);
+        Scales out(B);
+        if ((int)cf.size() <= m + 1 || t < 0) {
+            const double mrf = c.mod_reduce_factor[base_level(cf) + 1];
+            for (int b = 0; b < B; ++b) {
+                out[b] = S[b] * mrf;
+                out[b] /= mrf;
+            }
+            leaves.push_back(Leaf{std::move(cf), S, {}});
+            return out;
+        }
+        const int M = m << t;
+        if ((int)cf.size() <= M) return plan(cf, t - 1, S);
+        std::vector<double> q, r;
+        divide(cf, M, q, r);
+        const int lvl = std::min(rec_level(q, t - 1), G[t][0]->level);
+        const double mrf = c.mod_reduce_factor[lvl];
+        Scales sq(B);
+        for (int b = 0; b < B; ++b) sq[b] = S[b] * mrf / G[t][b]->noise;
+        const Scales Q = plan(q, t - 1, sq);
+        for (int b = 0; b < B; ++b) {
+            out[b] = Q[b] * G[t][b]->noise;
+            out[b] /= mrf;
+        }
+        plan(r, t - 1, out);
+        return out;
+    }
+    // All of them together, those at one level in one pass over the T_j, where
+    // there are enough to gain and few enough to hold at once: at N = 2^16 the 8 of
+    // a series of degree 58 over two ciphertexts took 955 us one by one.
+    static constexpr size_t LEAVES = 16;
+    void fill(const std::vector<double>& cf, int t, const Scales& S) {
+        plan(cf, t, S);
+        if (leaves.size() < 2 || leaves.size() > LEAVES) {
+            leaves.clear();
+            return;
+        }
+        std::map<int, std::vector<Leaf*>> levels;
+        for (Leaf& l : leaves) {
+            l.sum = fresh();
+            levels[base_level(l.cf) + 1].push_back(&l);
+        }
+        std::vector<Ciphertext*> all;
+        for (const auto& [lo, ls] : levels) {
+            size_t terms = 2;  // T_1 at least, also where all are constants
+            for (const Leaf* l : ls) terms = std::max(terms, l->cf.size());
+            for (int b = 0; b < B; ++b) {
+                std::vector<const Ciphertext*> xs;
+                std::vector<size_t> js;
+                for (size_t j = 1; j < terms; ++j)
+                    if (T[j][b]->level >= lo) {
+                        js.push_back(j);
+                        xs.push_back(T[j][b].get());
+                    }
+                std::vector<std::vector<double>> vs;
+                Scales s;
+                std::vector<Ciphertext*> out;
+                for (Leaf* l : ls) {
+                    vs.emplace_back();
+                    for (size_t j : js) vs.back().push_back(j < l->cf.size() ? l->cf[j] : 0.0);
+                    s.push_back(l->S[b]);
+                    out.push_back(l->sum[b].get());
+                    all.push_back(out.back());
+                }
+                lincomb_set_to_scale(c, xs, vs, lo, s, out);
+            }
+        }
+        rescale_batch(c, all);
+        for (Leaf& l : leaves)
+            if (!l.cf.empty()) add_const_batch(c, ptrs(l.sum), l.cf[0]);
     }
     // sum_j cf[j] T_j at scales S, for cf.size() <= m 2^(t+1)
     CtVec rec(std::vector<double> cf, int t, const Scales& S) {
@@ -165,10 +254,8 @@ struct Cheb {
         Scales sp(B);
         for (int b = 0; b < B; ++b) sp[b] = p[b]->noise;
         CtVec R = rec(r, t - 1, sp);
-        for (int b = 0; b < B; ++b) {
-            align(p[b], R[b], c);
-            eval_add(c, *p[b], *R[b], *p[b]);
-        }
+        for (int b = 0; b < B; ++b) align(p[b], R[b], c);
+        add_batch(c, ptrs(p), cptrs(R));
         return p;
     }
 };
@@ -192,7 +279,7 @@ void eval_chebyshev_series_batch(Context& c, const std::vector<const Ciphertext*
     int deg = (int)coeffs.size() - 1;
     while (deg > 0 && coeffs[deg] == 0.0) --deg;
     ManualScaling manual(c);
-    Cheb S{c, B, {}, {}, 1};
+    Cheb S{c, B, {}, {}, 1, {}, 0};
     // y = (2x - (a + b)) / (b - a); no level spent when [a, b] = [-1, 1]
     CtVec y;
     for (int i = 0; i < B; ++i) {
@@ -237,6 +324,7 @@ void eval_chebyshev_series_batch(Context& c, const std::vector<const Ciphertext*
     const int lout = S.rec_level(cf, tmax);
     if (lout < 0) throw Error(E_LEVEL, "not enough levels for the Chebyshev series");
     const double s_out = c.scaling_factor_real.empty() ? S.T[1][0]->noise : c.scaling_factor_real[lout];
+    S.fill(cf, tmax, Scales(B, s_out));
     CtVec res = S.rec(cf, tmax, Scales(B, s_out));
     for (int i = 0; i < B; ++i) {
         if (res[i]->level != lout) throw Error(E_STATE, "Chebyshev: level plan and evaluation disagree");
@@ -267,16 +355,15 @@ void eval_mod_reduction_batch(Context& c, const std::vector<const Ciphertext*>& 
     const double two_pi = 2.0 * 3.14159265358979323846;
     const std::vector<const Ciphertext*> in(outs.begin(), outs.end());
     for (int j = 1; j <= double_angle_its; ++j) {
+        std::vector<Ciphertext*> deep;
         for (Ciphertext* o : outs)
-            if (o->noise_level == 2) rescale(c, *o);
+            if (o->noise_level == 2) deep.push_back(o);
+        rescale_batch(c, deep);
         if (outs.size() == 1)
             eval_square(c, *outs[0], *outs[0], false);
         else
             eval_mult_batch(c, in, in, outs, false);
-        for (Ciphertext* o : outs) {
-            eval_add(c, *o, *o, *o);
-            add_const_at_scale(c, *o, -1.0 / std::pow(two_pi, std::pow(2.0, j - double_angle_its)), *o);
-        }
+        double_add_const(c, outs, -1.0 / std::pow(two_pi, std::pow(2.0, j - double_angle_its)));
     }
     for (Ciphertext* o : outs) eval_mult_int(c, *o, post, *o);
 }

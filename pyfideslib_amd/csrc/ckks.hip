@@ -468,28 +468,9 @@ void eval_square(Context& c, const Ciphertext& a, Ciphertext& out, bool do_resca
 
 // Rescale with caller-provided scratch: top = the coefficient-form top limbs
 // of both parts (2 limbs), mid = the forward NTT's intermediate (2 l limbs).
-static void rescale_with(Context& c, Ciphertext& a, uint64_t* top, uint64_t* mid, const uint64_t* x0 = nullptr,
-                         const uint64_t* x1 = nullptr, const uint64_t* w = nullptr) {
+static void rescale_unfused(Context& c, Ciphertext& a, uint64_t* top, uint64_t* mid) {
     const int l = a.level;
     const size_t N = c.N;
-    if (rescale_ok(c.T)) {
-        RescaleJobs rj = inline_list<RescaleJobs>();
-        rj.inl[0] = RescaleJob{w ? x0 : a.c0(), w, top, mid, l, 0};
-        rj.inl[1] = RescaleJob{w ? x1 : a.c1(), w, top + N, mid + l * N, l, 0};
-        rj.n = 2;
-        ck(launch_rescale_cols(c.T, rj, l, c.stream), "rescale columns");
-        NttJob f0 = ntt_job(nullptr, mid, a.c0(), l, l, 0);
-        NttJob f1 = ntt_job(nullptr, mid + l * N, a.c1(), l, l, 0);
-        f0.level = f1.level = l;
-        f0.aux = x0;
-        f1.aux = x1;
-        f0.add = f1.add = w;
-        run_ntt(c, {f0, f1}, false, LOAD_PLAIN, w ? STORE_MUL_RESCALE : STORE_RESCALE, NTT_PASS2);
-        a.level = l - 1;
-        a.noise /= c.mod_reduce_factor[l];
-        a.noise_level -= 1;
-        return;
-    }
     NttJob i0 = ntt_job(a.c0() + l * N, top, top, 1, 1, l);
     NttJob i1 = ntt_job(a.c1() + l * N, top + N, top + N, 1, 1, l);
     run_ntt(c, {i0, i1}, true);
@@ -497,21 +478,78 @@ static void rescale_with(Context& c, Ciphertext& a, uint64_t* top, uint64_t* mid
     NttJob f1 = ntt_job(top + N, mid + l * N, a.c1(), l, l, 0);
     f0.level = f1.level = l;
     run_ntt(c, {f0, f1}, false, LOAD_SWITCH, STORE_RESCALE);
+}
+
+static void rescaled(Context& c, Ciphertext& a) {
+    const int l = a.level;
     a.level = l - 1;
     a.noise /= c.mod_reduce_factor[l];
     a.noise_level -= 1;
 }
 
+// n ciphertexts (of any levels above 0) rescaled in the launches of one; with w
+// the limbs of (x0, x1) w take the place of the first one's.
+constexpr int RESCALE_BATCH = NTT_INLINE / 2;
+static_assert(RESCALE_INLINE >= 2 * RESCALE_BATCH, "two polynomials a ciphertext");
+static void rescale_fused(Context& c, Ciphertext* const* a, int n, const uint64_t* x0 = nullptr,
+                          const uint64_t* x1 = nullptr, const uint64_t* w = nullptr) {
+    const size_t N = c.N;
+    size_t limbs = 0;
+    int most = 0;
+    for (int i = 0; i < n; ++i) {
+        limbs += 2 * (size_t)a[i]->level;
+        most = std::max(most, a[i]->level);
+    }
+    DevBuf top(&c.pool, 2 * n * N), mid(&c.pool, limbs * N);
+    RescaleJobs rj = inline_list<RescaleJobs>();
+    std::vector<NttJob> f;
+    uint64_t *t = top.ptr, *y = mid.ptr;
+    for (int i = 0; i < n; ++i)
+        for (int part = 0; part < 2; ++part, t += N) {
+            const int l = a[i]->level;
+            uint64_t* o = part ? a[i]->c1() : a[i]->c0();
+            const uint64_t* x = part ? x1 : x0;
+            rj.inl[rj.n++] = RescaleJob{w ? x : o, w, t, y, l, 0};
+            NttJob j = ntt_job(nullptr, y, o, l, l, 0);
+            j.level = l;
+            j.aux = x;
+            j.add = w;
+            f.push_back(j);
+            y += (size_t)l * N;
+        }
+    ck(launch_rescale_cols(c.T, rj, most, c.stream), "rescale columns");
+    run_ntt(c, f, false, LOAD_PLAIN, w ? STORE_MUL_RESCALE : STORE_RESCALE, NTT_PASS2);
+    for (int i = 0; i < n; ++i) rescaled(c, *a[i]);
+}
+
 void rescale(Context& c, Ciphertext& a) {
     if (a.level < 1) throw Error(E_LEVEL, "cannot rescale at level 0");
+    if (rescale_ok(c.T)) {
+        Ciphertext* p = &a;
+        rescale_fused(c, &p, 1);
+        return;
+    }
     DevBuf top(&c.pool, 2 * (size_t)c.N), mid(&c.pool, 2 * (size_t)a.level * c.N);
-    rescale_with(c, a, top.ptr, mid.ptr);
+    rescale_unfused(c, a, top.ptr, mid.ptr);
+    rescaled(c, a);
+}
+
+void rescale_batch(Context& c, const std::vector<Ciphertext*>& a) {
+    for (Ciphertext* x : a)
+        if (x->level < 1) throw Error(E_LEVEL, "cannot rescale at level 0");
+    for (size_t i = 0; i < a.size(); i += RESCALE_BATCH) {
+        const int n = (int)std::min<size_t>(RESCALE_BATCH, a.size() - i);
+        if (rescale_ok(c.T))
+            rescale_fused(c, a.data() + i, n);
+        else
+            for (int k = 0; k < n; ++k) rescale(c, *a[i + k]);
+    }
 }
 
 // out's metadata is the product's, its limbs are not yet: out = (x0, x1) w rescaled.
 void mul_rescale(Context& c, const uint64_t* x0, const uint64_t* x1, const uint64_t* w, Ciphertext& out) {
-    DevBuf top(&c.pool, 2 * (size_t)c.N), mid(&c.pool, 2 * (size_t)out.level * c.N);
-    rescale_with(c, out, top.ptr, mid.ptr, x0, x1, w);
+    Ciphertext* p = &out;
+    rescale_fused(c, &p, 1, x0, x1, w);
 }
 
 static void ew(Context& c, const Ciphertext& a, const Ciphertext& b, Ciphertext& out, int op) {

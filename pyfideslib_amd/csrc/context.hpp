@@ -255,6 +255,7 @@ void load_key(Context& c, KeySwitchingKey& k, const uint64_t* a, const uint64_t*
 void eval_mult(Context& c, const Ciphertext& a, const Ciphertext& b, Ciphertext& out, bool rescale);
 void eval_square(Context& c, const Ciphertext& a, Ciphertext& out, bool rescale);
 void rescale(Context& c, Ciphertext& a);
+void rescale_batch(Context& c, const std::vector<Ciphertext*>& a);
 void mul_rescale(Context& c, const uint64_t* x0, const uint64_t* x1, const uint64_t* w, Ciphertext& out);
 void eval_add(Context& c, const Ciphertext& a, const Ciphertext& b, Ciphertext& out);
 void eval_sub(Context& c, const Ciphertext& a, const Ciphertext& b, Ciphertext& out);
@@ -331,6 +332,13 @@ void mult_const_to_scale(Context& c, const Ciphertext& a, int level, double v, d
 void double_angle_at_scale(Context& c, Ciphertext& out, int iterations);
 void lincomb_to_scale(Context& c, const std::vector<const Ciphertext*>& x, const std::vector<double>& v, int level,
                       double s_after, Ciphertext& out);
+void lincomb_set_to_scale(Context& c, const std::vector<const Ciphertext*>& x,
+                          const std::vector<std::vector<double>>& v, int level, const std::vector<double>& s_after,
+                          const std::vector<Ciphertext*>& outs);
+void double_add_const(Context& c, const std::vector<Ciphertext*>& p, double v);
+void add_const_batch(Context& c, const std::vector<Ciphertext*>& p, double v);
+void double_sub_batch(Context& c, const std::vector<Ciphertext*>& p, const std::vector<const Ciphertext*>& u);
+void add_batch(Context& c, const std::vector<Ciphertext*>& p, const std::vector<const Ciphertext*>& u);
 void eval_chebyshev_series(Context& c, const Ciphertext& x, const std::vector<double>& coeffs, double a, double b,
                            Ciphertext& out);
 void eval_mod_reduction(Context& c, const Ciphertext& x, const std::vector<double>& coeffs, int double_angle_its,

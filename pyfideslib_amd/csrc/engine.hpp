@@ -178,7 +178,7 @@ struct RescaleJob {
     int level;          // l
     int pad;
 };
-constexpr int RESCALE_INLINE = 2;
+constexpr int RESCALE_INLINE = 8;
 using RescaleJobs = JobList<RescaleJob, RESCALE_INLINE>;
 using NttJobs = JobList<NttJob, NTT_INLINE>;
 
@@ -260,7 +260,15 @@ struct EwJob {
 };
 constexpr int EW_INLINE = 4;
 using EwJobs = JobList<EwJob, EW_INLINE>;
-enum EwOp { EW_ADD = 0, EW_SUB = 1, EW_MUL = 2, EW_MUL_SCALAR = 3, EW_ADD_SCALAR = 4 };
+enum EwOp {
+    EW_ADD = 0,
+    EW_SUB = 1,
+    EW_MUL = 2,
+    EW_MUL_SCALAR = 3,
+    EW_ADD_SCALAR = 4,
+    EW_DOUBLE_SUB = 5,        // 2 a - b
+    EW_DOUBLE_ADD_SCALAR = 6  // 2 a + constant, without the constant where b is null
+};
 
 // Per-limb constants of a scalar op (limb i: c[i], with its Shoup companion
 // for EW_MUL_SCALAR), passed by value in the kernel arguments.
@@ -346,6 +354,19 @@ struct LinCombJob {
     int n;
     int nl;
 };
+// g <= LINCOMB_SET sums of the same n terms at one level: out j = sum_t w[i][t][j] x_t
+// on limb i, w centered doubles (as words, in ShoupConst::w) on the FP64 units' limbs.
+// The rows of w hold lincomb_row(g) sums.
+constexpr int LINCOMB_SET = 8;
+inline int lincomb_row(int g) { return g <= 2 ? 2 : g <= 4 ? 4 : LINCOMB_SET; }
+struct LinCombSet {
+    const uint64_t* const* x0;
+    const uint64_t* const* x1;
+    uint64_t* const* o0;
+    uint64_t* const* o1;
+    const ShoupConst* w;
+    int n, nl, g;
+};
 
 // ------------------------------------------------------------- tuning ----
 // Launch configurations picked per (kind, logN, size) from a table measured
@@ -424,6 +445,7 @@ hipError_t launch_moddown_cols(const DevTables& T, const ModDownJobs& jobs, int 
 hipError_t launch_elementwise(const DevTables& T, const EwJobs& jobs, int max_nl, int op, hipStream_t stream);
 hipError_t launch_tensor_sum(const DevTables& T, const TensorSumJob& J, hipStream_t s);
 hipError_t launch_lincomb(const DevTables& T, const LinCombJob& job, hipStream_t stream);
+hipError_t launch_lincomb_set(const DevTables& T, const LinCombSet& set, hipStream_t stream);
 // max_gc: the largest gc of the list (selects the accumulator count)
 hipError_t launch_dot_bsgs(const DevTables& T, const DotJobs& jobs, int max_nl, int max_gc, hipStream_t stream);
 hipError_t launch_ext_rot(const DevTables& T, const ExtRotJobs& jobs, int max_nl, hipStream_t stream);

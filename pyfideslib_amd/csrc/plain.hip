@@ -577,6 +577,139 @@ void lincomb_to_scale(Context& c, const std::vector<const Ciphertext*>& x, const
     out.slots = x[0]->slots;
 }
 
+// The same for several sums of the terms x, outs[j] = sum_t v[j][t] x[t] onto
+// s_after[j], each term read once for up to LINCOMB_SET of them.
+void lincomb_set_to_scale(Context& c, const std::vector<const Ciphertext*>& x,
+                          const std::vector<std::vector<double>>& v, int level, const std::vector<double>& s_after,
+                          const std::vector<Ciphertext*>& outs) {
+    const int n = (int)x.size();
+    if (n < 1 || v.size() != outs.size() || s_after.size() != outs.size())
+        throw Error(E_ARG, "linear combinations need one constant per term and output");
+    if (level < 1) throw Error(E_LEVEL, "no level left to rescale into");
+    for (const Ciphertext* a : x) {
+        require_loaded(*a);
+        if (level > a->level) throw Error(E_LEVEL, "term below the combination's level");
+        if (a->noise_level != x[0]->noise_level) throw Error(E_STATE, "terms at different noise levels");
+    }
+    const int nl = level + 1;
+    const double mrf = c.mod_reduce_factor[level];
+    for (size_t first = 0; first < outs.size(); first += LINCOMB_SET) {
+        const int g = (int)std::min<size_t>(LINCOMB_SET, outs.size() - first), row = lincomb_row(g);
+        // table: x0 | x1 | o0 | o1 pointers | constants [nl][n][row]
+        auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
+        const size_t pb = up((size_t)n * sizeof(uint64_t*)), ob = up((size_t)g * sizeof(uint64_t*));
+        const size_t o_o = 2 * pb, o_w = o_o + 2 * ob, bytes = o_w + (size_t)nl * n * row * sizeof(ShoupConst);
+        std::vector<char> host(bytes, 0);
+        auto put = [&](size_t at, const uint64_t* p) { std::memcpy(host.data() + at, &p, sizeof(p)); };
+        for (int t = 0; t < n; ++t) {
+            put(t * sizeof(uint64_t*), x[t]->c0());
+            put(pb + t * sizeof(uint64_t*), x[t]->c1());
+        }
+        ShoupConst* w = (ShoupConst*)(host.data() + o_w);
+        for (int j = 0; j < g; ++j) {
+            if ((int)v[first + j].size() != n) throw Error(E_ARG, "linear combination needs one constant per term");
+            put(o_o + j * sizeof(uint64_t*), outs[first + j]->c0());
+            put(o_o + ob + j * sizeof(uint64_t*), outs[first + j]->c1());
+            for (int t = 0; t < n; ++t) {
+                if (v[first + j][t] == 0.0) continue;
+                const std::vector<uint64_t> r =
+                    round_residues(c, level, v[first + j][t] * mrf * (s_after[first + j] / x[t]->noise));
+                for (int i = 0; i < nl; ++i) {
+                    ShoupConst& k = w[((size_t)i * n + t) * row + j];
+                    if ((c.T.fpmask[i >> 6] >> (i & 63)) & 1) {
+                        const double d = r[i] > c.q[i] / 2 ? (double)r[i] - (double)c.q[i] : (double)r[i];
+                        std::memcpy(&k.w, &d, sizeof(d));
+                    } else {
+                        k = ShoupConst{r[i], (uint64_t)(((unsigned __int128)r[i] << 64) / c.q[i])};
+                    }
+                }
+            }
+        }
+        DevBuf table(&c.pool, (bytes + 7) / 8);
+        c.upload(table.ptr, host.data(), bytes);
+        char* d = (char*)table.ptr;
+        const LinCombSet J{(const uint64_t* const*)d, (const uint64_t* const*)(d + pb),
+                           (uint64_t* const*)(d + o_o), (uint64_t* const*)(d + o_o + ob),
+                           (const ShoupConst*)(d + o_w), n, nl, g};
+        ck(launch_lincomb_set(c.T, J, c.stream), "linear combinations");
+        for (int j = 0; j < g; ++j) {
+            Ciphertext& o = *outs[first + j];
+            o.level = level;
+            o.noise = s_after[first + j] * mrf;
+            o.noise_level = x[0]->noise_level + 1;
+            o.slots = x[0]->slots;
+        }
+    }
+}
+
+// Runs of a batch that share level and tracked scale, up to a list's inline
+// jobs (per of them to a ciphertext) each: f(first, end).
+template <class F>
+static void like_runs(const std::vector<Ciphertext*>& p, size_t per, F&& f) {
+    for (size_t i = 0; i < p.size();) {
+        size_t e = i + 1;
+        while (e < p.size() && (e - i + 1) * per <= EW_INLINE && p[e]->level == p[i]->level &&
+               p[e]->noise == p[i]->noise)
+            ++e;
+        f(i, e);
+        i = e;
+    }
+}
+
+// p = 2 p + v (v at each one's tracked scale), p = p + v, p = 2 p - u and p = p + u, for
+// batches, in place; metadata as add_const_at_scale and eval_add leave it.
+void double_add_const(Context& c, const std::vector<Ciphertext*>& p, double v) {
+    like_runs(p, 2, [&](size_t i, size_t e) {
+        const int nl = p[i]->level + 1;
+        const LimbConsts k = limb_consts(c, round_residues(c, p[i]->level, v * p[i]->noise), false);
+        EwJobs L = ew_list();
+        for (; i < e; ++i) {
+            require_loaded(*p[i]);
+            L.inl[L.n++] = EwJob{p[i]->c0(), p[i]->c0(), p[i]->c0(), nl};
+            L.inl[L.n++] = EwJob{p[i]->c1(), nullptr, p[i]->c1(), nl};
+        }
+        ck(launch_scalar(c.T, L, nl, EW_DOUBLE_ADD_SCALAR, k, c.stream), "double and add const");
+    });
+}
+void add_const_batch(Context& c, const std::vector<Ciphertext*>& p, double v) {
+    if (v == 0.0) return;
+    like_runs(p, 1, [&](size_t i, size_t e) {
+        const int nl = p[i]->level + 1;
+        const LimbConsts k = limb_consts(c, round_residues(c, p[i]->level, v * p[i]->noise), false);
+        EwJobs L = ew_list();
+        for (; i < e; ++i) {
+            require_loaded(*p[i]);
+            L.inl[L.n++] = EwJob{p[i]->c0(), nullptr, p[i]->c0(), nl};
+        }
+        ck(launch_scalar(c.T, L, nl, EW_ADD_SCALAR, k, c.stream), "add const");
+    });
+}
+static void ew_batch(Context& c, const std::vector<Ciphertext*>& p, const std::vector<const Ciphertext*>& u, int op) {
+    if (p.size() != u.size()) throw Error(E_ARG, "batch size mismatch");
+    for (size_t i = 0; i < p.size();) {
+        EwJobs L = ew_list();
+        int most = 0;
+        for (; i < p.size() && L.n + 2 <= EW_INLINE; ++i) {
+            require_loaded(*p[i]);
+            require_loaded(*u[i]);
+            if (p[i]->noise_level != u[i]->noise_level) throw Error(E_STATE, "operands at different noise degrees");
+            p[i]->level = std::min(p[i]->level, u[i]->level);
+            p[i]->slots = std::max(p[i]->slots, u[i]->slots);
+            const int nl = p[i]->level + 1;
+            most = std::max(most, nl);
+            L.inl[L.n++] = EwJob{p[i]->c0(), u[i]->c0(), p[i]->c0(), nl};
+            L.inl[L.n++] = EwJob{p[i]->c1(), u[i]->c1(), p[i]->c1(), nl};
+        }
+        ck(launch_elementwise(c.T, L, most, op, c.stream), "batched elementwise");
+    }
+}
+void double_sub_batch(Context& c, const std::vector<Ciphertext*>& p, const std::vector<const Ciphertext*>& u) {
+    ew_batch(c, p, u, EW_DOUBLE_SUB);
+}
+void add_batch(Context& c, const std::vector<Ciphertext*>& p, const std::vector<const Ciphertext*>& u) {
+    ew_batch(c, p, u, EW_ADD);
+}
+
 // EvalAddMany (api/CryptoContext.cpp:834-880): out = sum of the ciphertexts
 // in ONE launch (each read once; the linear-combination kernel with unit
 // constants), at the lowest input level; metadata of the first input, as
