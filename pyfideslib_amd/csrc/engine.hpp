@@ -147,7 +147,8 @@ enum NttStore {
     STORE_RESCALE = 2,
     STORE_MODDOWN_RESCALE = 3,
     STORE_MODDOWN_AUTO = 4,  // STORE_MODDOWN, then the automorphism of NttJob::autok
-    STORE_MUL_RESCALE = 5    // STORE_RESCALE of the product aux * add (dst may be either)
+    STORE_MUL_RESCALE = 5,   // STORE_RESCALE of the product aux * add (dst may be either)
+    STORE_MODDOWN_INV = 6    // STORE_MODDOWN, and the inverse's first pass of what it stored to mid
 };
 enum IScale { ISCALE_PLAIN = 0, ISCALE_MODUP = 1, ISCALE_MODDOWN = 2 };
 

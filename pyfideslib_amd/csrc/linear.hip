@@ -157,8 +157,11 @@ struct RotOut {
 // One ModUp per distinct source, then every key switch in one KSK launch.
 // rots (fused kernels only): req i's product leaves rotated as rots[i], with
 // downs[i] (or nullptr) as KskJob::rot_down, and its accumulators are not written.
+// inv: the sources after the first pass of their inverse transform, in the requests'
+// order (ext_moddown left them), or nullptr.
 void ext_keyswitch(Context& c, int level, const std::vector<KsReq>& reqs, std::vector<DevBuf>& keep,
-                   const std::vector<const RotOut*>& rots = {}, const std::vector<uint64_t*>& downs = {}) {
+                   const std::vector<const RotOut*>& rots = {}, const std::vector<uint64_t*>& downs = {},
+                   uint64_t* inv = nullptr) {
     if (reqs.empty()) return;
     const int nl = level + 1, nd = c.num_digits(level);
     const size_t N = c.N, npos = (size_t)nl + c.K;
@@ -166,8 +169,8 @@ void ext_keyswitch(Context& c, int level, const std::vector<KsReq>& reqs, std::v
     for (const KsReq& r : reqs)
         if (std::find(xs.begin(), xs.end(), r.x) == xs.end()) xs.push_back(r.x);
     const bool fused = fused_ok(c.T);
-    keep.emplace_back(&c.pool, (fused ? xs.size() : 1) * nl * N);
-    uint64_t* t = keep.back().ptr;
+    if (!inv) keep.emplace_back(&c.pool, (fused ? xs.size() : 1) * nl * N);
+    uint64_t* t = inv ? inv : keep.back().ptr;
     keep.emplace_back(&c.pool, xs.size() * nd * npos * N);
     uint64_t* ext = keep.back().ptr;
     if (fused) {
@@ -184,7 +187,8 @@ void ext_keyswitch(Context& c, int level, const std::vector<KsReq>& reqs, std::v
             iv.push_back(j);
             mu.push_back(ModUpJob{t + i * nl * N, ext + i * nd * npos * N, level});
         }
-        run_ntt_jobs(c, iv, true, LOAD_PLAIN, STORE_PLAIN, fused_inv_cols(c.T) ? NTT_PASS1 : NTT_BOTH);
+        const int passes = (inv ? 0 : NTT_PASS1) | (fused_inv_cols(c.T) ? 0 : NTT_PASS2);
+        if (passes) run_ntt_jobs(c, iv, true, LOAD_PLAIN, STORE_PLAIN, passes);
         ck(launch_modup_cols(c.T, job_list<ModUpJobs>(c, keep, mu), nd, nl, c.stream), "ext modup and columns");
     } else {
         for (size_t i = 0; i < xs.size(); ++i) modup_to(c, level, xs[i], t, ext + i * nd * npos * N);
@@ -250,10 +254,12 @@ void ext_keyswitch(Context& c, int level, const std::vector<KsReq>& reqs, std::v
 
 // ModDown of P*Q polynomials ([nl + K][N]) into Q-basis ones ([nl][N]).
 // rows: the special limbs after the first pass of their inverse transform
-// ([polys][K][N], overwritten), or nullptr.
-void ext_moddown(Context& c, int level, const std::vector<std::pair<const uint64_t*, uint64_t*>>& polys,
-                 std::vector<DevBuf>& keep, uint64_t* rows = nullptr) {
-    if (polys.empty()) return;
+// ([polys][K][N], overwritten), or nullptr.  switched: the outputs are key-switched
+// next, and with the fused kernels their inverse transform is begun; returns
+// where that is (ext_keyswitch's inv), or nullptr.
+uint64_t* ext_moddown(Context& c, int level, const std::vector<std::pair<const uint64_t*, uint64_t*>>& polys,
+                      std::vector<DevBuf>& keep, uint64_t* rows = nullptr, bool switched = false) {
+    if (polys.empty()) return nullptr;
     const int nl = level + 1, K = c.K;
     const size_t N = c.N, n = polys.size();
     if (!rows) keep.emplace_back(&c.pool, n * K * N);
@@ -286,12 +292,13 @@ void ext_moddown(Context& c, int level, const std::vector<std::pair<const uint64
     if (passes) run_ntt_jobs(c, isp, true, LOAD_PLAIN, STORE_PLAIN, passes);
     if (fused_ok(c.T)) {
         ck(launch_moddown_cols(c.T, job_list<ModDownJobs>(c, keep, md), nl, false, c.stream), "ext moddown and columns");
-        run_ntt_jobs(c, fwd, false, LOAD_PLAIN, STORE_MODDOWN, NTT_PASS2);
-        return;
+        run_ntt_jobs(c, fwd, false, LOAD_PLAIN, switched ? STORE_MODDOWN_INV : STORE_MODDOWN, NTT_PASS2);
+        return switched ? y : nullptr;
     }
     ck(launch_moddown_conv(c.T, job_list<ModDownJobs>(c, keep, md), nl, c.stream),
        "ext moddown conv");
     run_ntt_jobs(c, fwd, false, LOAD_PLAIN, STORE_MODDOWN);
+    return nullptr;
 }
 
 void ext_rot_outs(Context& c, int level, const std::vector<RotOut>& outs, std::vector<DevBuf>& keep) {
@@ -318,20 +325,20 @@ void ext_rot_outs(Context& c, int level, const std::vector<RotOut>& outs, std::v
 // and with downs.  No output may alias a source (x, add0) of any request.
 // downs: per request KskJob::rot_down (fused kernels and outputs of one term only).
 void ext_switch_rotate(Context& c, int level, const std::vector<KsReq>& reqs, const std::vector<RotOut>& outs,
-                       std::vector<DevBuf>& keep, const std::vector<uint64_t*>& downs = {}) {
+                       std::vector<DevBuf>& keep, const std::vector<uint64_t*>& downs = {}, uint64_t* inv = nullptr) {
     std::vector<const RotOut*> rots;
     std::vector<RotOut> rest;
     for (const KsReq& r : reqs)
         for (const RotOut& o : outs)
             if (o.terms.size() == 1 && o.terms[0].acc_a == r.acc_a && !o.terms[0].add1) rots.push_back(&o);
     if (!fused_ok(c.T) || rots.size() != reqs.size()) {
-        ext_keyswitch(c, level, reqs, keep);
+        ext_keyswitch(c, level, reqs, keep, {}, {}, inv);
         ext_rot_outs(c, level, outs, keep);
         return;
     }
     for (const RotOut& o : outs)
         if (std::find(rots.begin(), rots.end(), &o) == rots.end()) rest.push_back(o);
-    ext_keyswitch(c, level, reqs, keep, rots, downs);
+    ext_keyswitch(c, level, reqs, keep, rots, downs, inv);
     ext_rot_outs(c, level, rest, keep);
 }
 
@@ -406,7 +413,7 @@ static void lt_ext(Context& c, const std::vector<const Ciphertext*>& as, const s
                                                     c.rot_index((int)(gstep % half)), 0}},
                                         inn(k, j), inn(k, j) + pw, inn(k, j), inn(k, j) + pw});
                 }
-                ext_moddown(c, level, md, keep, rows);
+                uint64_t* inv = ext_moddown(c, level, md, keep, rows, true);
                 // the next giant step takes c1 of these sums down
                 rows = nullptr;
                 std::vector<uint64_t*> downs;
@@ -414,7 +421,7 @@ static void lt_ext(Context& c, const std::vector<const Ciphertext*>& as, const s
                     rows = next_rows;
                     for (int k = 0; k < B; ++k) downs.push_back(rows + (size_t)k * c.K * N);
                 }
-                ext_switch_rotate(c, level, reqs, ro, keep, downs);
+                ext_switch_rotate(c, level, reqs, ro, keep, downs, inv);
             } else {
                 for (int k = 0; k < B; ++k)
                     ro.push_back(RotOut{{ExtRotTerm{nullptr, nullptr, inn(k, j + 1), inn(k, j + 1) + pw, 1u, 0}},
@@ -441,8 +448,8 @@ static void lt_ext(Context& c, const std::vector<const Ciphertext*>& as, const s
                 ro[k].terms.push_back(ExtRotTerm{aa, aa + pw, inn(k, j), nullptr, c.rot_index((int)(r % half)), 0});
             }
         }
-        ext_moddown(c, level, md, keep);
-        ext_switch_rotate(c, level, reqs, ro, keep);
+        uint64_t* inv = ext_moddown(c, level, md, keep, nullptr, true);
+        ext_switch_rotate(c, level, reqs, ro, keep, {}, inv);
     }
 
     // offset rotation (kept in P*Q), then one ModDown of both parts
@@ -462,8 +469,8 @@ static void lt_ext(Context& c, const std::vector<const Ciphertext*>& as, const s
             fin.emplace_back(o, outs[k]->c0());
             fin.emplace_back(o + pw, outs[k]->c1());
         }
-        ext_moddown(c, level, md, keep);
-        ext_switch_rotate(c, level, reqs, ro, keep);
+        uint64_t* inv = ext_moddown(c, level, md, keep, nullptr, true);
+        ext_switch_rotate(c, level, reqs, ro, keep, {}, inv);
     } else {
         for (int k = 0; k < B; ++k) {
             fin.emplace_back(inn(k, 0), outs[k]->c0());

@@ -425,7 +425,8 @@ struct Epilogue {
     uint64_t e0[G::R], e1[G::R];
     // limb: the limb's first word within the polynomial (uniform), row: the row's within the limb
     __device__ __forceinline__ void load(const NttJob& J, size_t limb, uint32_t row, uint32_t t) {
-        if constexpr (STORE == STORE_MODDOWN || STORE == STORE_MODDOWN_RESCALE || STORE == STORE_MODDOWN_AUTO) {
+        if constexpr (STORE == STORE_MODDOWN || STORE == STORE_MODDOWN_RESCALE || STORE == STORE_MODDOWN_AUTO ||
+                      STORE == STORE_MODDOWN_INV) {
             const gu64* aux = gp(J.aux) + limb;
 #pragma unroll
             for (int j = 0; j < G::R; ++j) e0[j] = aux[row + G::mem(t, j)];
@@ -460,6 +461,21 @@ struct Epilogue {
             const ShoupConst pinv = cld(T.pinv + pid);
 #pragma unroll
             for (int j = 0; j < G::R; ++j) dst[row + G::mem(t, j)] = ar.sub_mul_add(e0[j], v[j], pinv, e1[j]);
+        } else if constexpr (STORE == STORE_MODDOWN_INV) {
+            using V = typename A::V;
+            const ShoupConst pinv = cld(T.pinv + pid);
+            V u[G::R];
+#pragma unroll
+            for (int j = 0; j < G::R; ++j) {
+                const uint64_t w = ar.sub_mul_add(e0[j], v[j], pinv, e1[j]);
+                dst[row + G::mem(t, j)] = w;
+                u[j] = ar.from(w);
+            }
+            lds_sync<G::WAVE>();  // the LDS reads before are done
+            inv_row<G>(ar, reinterpret_cast<V*>(sub), u, t, G::N1 + r, A::inv(T) + (size_t)pid * G::N);
+            gu64* mid = gp(J.mid) + (size_t)pos * G::N;
+#pragma unroll
+            for (int j = 0; j < G::R; ++j) mid[row + elem<G::LR, G::LOL, G::NBI>(t, j)] = A::pack(u[j]);
         } else if constexpr (STORE == STORE_MODDOWN_AUTO) {
             // Element jg = r N2 + e sits at exponent 2 brev(jg) + 1 =
             // 2 N1 brev(e) + 2 brev(r) + 1; times k (mod 2N) it lands at
