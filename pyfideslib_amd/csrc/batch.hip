@@ -1,10 +1,11 @@
 // Batched key-switched ops -- HMult + relinearize (+ rescale) pairs and
 // rotations -- over many independent ciphertexts at uneven levels.
 //
-// Every stage of the per-op pipeline (tensor, INTT, ModUp conversion, NTT of
-// the extended digits, KSK inner product, INTT of the special limbs, ModDown
-// conversion, NTT+ModDown(+rescale) epilogue) becomes ONE launch covering all
-// pairs: the grid walks a flattened list of (job, limb) tiles read from a
+// Every stage of the per-op pipeline (tensor with the first inverse pass, its
+// second pass, ModUp conversion with the first forward pass, the second pass
+// with the inner product, the special limbs' inverse column pass, ModDown
+// conversion, the last pass with its epilogue; past the fused sizes the
+// separate transforms and kernels) becomes ONE launch covering all pairs: the grid walks a flattened list of (job, limb) tiles read from a
 // device-resident job table, so ragged levels cost nothing and small levels
 // still fill the 256 CUs.  Job tables and scratch are built once per batch
 // signature and reused (the plan cache), so repeated calls upload nothing;

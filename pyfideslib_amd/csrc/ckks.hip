@@ -1,5 +1,5 @@
-// CKKS evaluation ops: launch sequences over the kernels in ntt.hip and
-// kernels.hip.  Each op mirrors a FIDESlib CKKS::Ciphertext method and keeps
+// CKKS evaluation ops: launch sequences over the kernels in ntt.hip, fused.hip,
+// fused_down.hip and rescale.hip (kernels.hip past their sizes).  Each op mirrors a FIDESlib CKKS::Ciphertext method and keeps
 // OpenFHE's arithmetic order so that every residue is bit-exact:
 //   mult      tensor -> ModUp(d2) -> KSK inner product -> ModDown -> add
 //             (Ciphertext.cpp:409-622, LimbPartitionMGPU.cu:573-1746)

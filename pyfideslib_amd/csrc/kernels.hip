@@ -1,4 +1,5 @@
-// Elementwise, base-conversion, key-switch and automorphism kernels (gfx950).
+// Elementwise, dot-product and automorphism kernels, and the separate
+// base-conversion and key-switch kernels of the sizes past the fused ones (gfx950).
 //
 // All are HBM streams over limb-major polynomials: 256-thread blocks along the
 // coefficient axis, the limb (position) along blockIdx.y and the job along
@@ -734,7 +735,7 @@ __global__ void __launch_bounds__(EW_BLOCK) k_lincomb(DevTables T, LinCombJob J)
 
 // Several sums of the same terms in one pass, one coefficient per thread: bound by
 // memory, so every term is read once for all of them (at N = 2^16 with 18 limbs and 15
-// terms eight sums one by one take 480 us).  Terms in pairs, so that the loads
+// terms eight sums take 480 us one by one, 93 together).  Terms in pairs, so that the loads
 // of both are in flight.  On the FP64 units a product of a term below p and a centered
 // weight is at most 0.7 p (its quotient's error included), eight of them and
 // what is left of the ones before below 6.2 p.
