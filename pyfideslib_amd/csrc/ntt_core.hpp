@@ -12,7 +12,7 @@ __device__ __forceinline__ uint32_t lds_off(uint32_t e) { return e + (e >> 4); }
 // Arithmetic of one limb's transform, picked per block by the limb's prime
 // (wave-uniform): IntArith (any p < 2^60; Harvey-lazy Shoup butterflies on
 // 64-bit words) or FpArith (p < 2^50; exact FP64 butterflies, modarith.hpp's
-// fp_mul).  An FP64 butterfly is 8 to 9 instructions against about 36, and its
+// fp_mul).  An FP64 butterfly is 8 to 9 instructions against about 22, and its
 // twiddles are 8 bytes against 16.
 //
 // Bounds of the FP64 values, in units of p (every step must stay below 8):
@@ -34,30 +34,32 @@ struct IntArith {
     __device__ __forceinline__ V from(uint64_t x) const { return x; }
     static __device__ __forceinline__ V unpack(uint64_t m) { return m; }
     static __device__ __forceinline__ uint64_t pack(V v) { return v; }
-    // every stage adds 2p to the bound; U is brought below 8p where FpArith
-    // reduces, so four stages stay below 16p < 2^64 (any 64-bit b will do)
-    template <bool RED>
+    // every stage adds 4p to the bound (any 64-bit b will do): U is brought below
+    // 8p at the start of every phase of two stages, and below 4p at that of
+    // three (RED 2), so what a phase leaves is below 16p < 2^64
+    static constexpr bool EACH_PHASE = true;
+    template <int RED>
     __device__ __forceinline__ void fwd_bf(V& a, V& b, const W& w) const {
-        const uint64_t U = RED ? csub(a, 8 * p) : a;
-        const uint64_t X = mul_shoup_lazy(b, w.w, w.wp, p);
+        const uint64_t U = RED == 2 ? csub(csub(a, 8 * p), 4 * p) : RED == 1 ? csub(a, 8 * p) : a;
+        const uint64_t X = mul_shoup_lazy4(b, w.w, w.wp, p);
         a = U + X;
-        b = U - X + 2 * p;
+        b = U - X + 4 * p;
     }
-    // inputs in [0, 2p), outputs in [0, 2p)
+    // inputs in [0, 4p), outputs in [0, 4p)
     template <bool RED>
     __device__ __forceinline__ void inv_bf(V& a, V& b, const W& w) const {
-        const uint64_t U = a, X = U + b;
-        a = X >= 2 * p ? X - 2 * p : X;
-        b = mul_shoup_lazy(U - b + 2 * p, w.w, w.wp, p);
+        const uint64_t U = a;
+        a = csub(U + b, 4 * p);
+        b = mul_shoup_lazy4(U - b + 4 * p, w.w, w.wp, p);
     }
     __device__ __forceinline__ void inv_last(V& a, V& b, const ShoupConst& s, const ShoupConst& ws) const {
         const uint64_t U = a, X = b;
-        a = mul_shoup_lazy(U + X, s.w, s.wp, p);
-        b = mul_shoup_lazy(U - X + 2 * p, ws.w, ws.wp, p);
+        a = mul_shoup_lazy4(U + X, s.w, s.wp, p);
+        b = mul_shoup_lazy4(U - X + 4 * p, ws.w, ws.wp, p);
     }
-    // the residue of a forward output in [0, 16p), of an inverse one in [0, 2p)
+    // the residue of a forward output in [0, 16p), of an inverse one in [0, 4p)
     __device__ __forceinline__ uint64_t canon_fwd(V x) const { return csub(term_fwd(x), p); }
-    __device__ __forceinline__ uint64_t canon_inv(V x) const { return csub(x, p); }
+    __device__ __forceinline__ uint64_t canon_inv(V x) const { return csub(csub(x, 2 * p), p); }
     // a b, a b + c d as residues; a value below 3p from reduce128_lazy
     __device__ __forceinline__ uint64_t mul(uint64_t a, uint64_t b, const PrimeInfo& P) const { return mulmod(a, b, P); }
     __device__ __forceinline__ uint64_t mul2(uint64_t a, uint64_t b, uint64_t c, uint64_t d,
@@ -116,7 +118,8 @@ struct FpArith {
     // between the two passes a limb holds the doubles themselves
     static __device__ __forceinline__ V unpack(uint64_t m) { return __longlong_as_double((long long)m); }
     static __device__ __forceinline__ uint64_t pack(V v) { return (uint64_t)__double_as_longlong(v); }
-    template <bool RED>
+    static constexpr bool EACH_PHASE = false;
+    template <int RED>
     __device__ __forceinline__ void fwd_bf(V& a, V& b, W w) const {
         const double U = RED ? fp_reduce(a, p, pinv) : a;
         const double X = fp_mul(b, w, p, pinv);
@@ -232,8 +235,8 @@ template <int LR, int K>
 constexpr int inv_last_lo() { return LR * ((K - 1) / LR); }
 
 // ---- forward (Cooley-Tukey), bits processed from the top down ----
-// RED: the first stage of the phase reduces its U (FpArith's bound).
-template <int LR, int K, int LO, int NB, bool RED, class A, class TW>
+// RED: the first stage of the phase reduces its U (the arithmetic's bound).
+template <int LR, int K, int LO, int NB, int RED, class A, class TW>
 __device__ __forceinline__ void fwd_bfly(const A& ar, typename A::V* v, uint32_t t, const TW& tw) {
     constexpr int R = 1 << LR;
 #pragma unroll
@@ -242,10 +245,10 @@ __device__ __forceinline__ void fwd_bfly(const A& ar, typename A::V* v, uint32_t
         for (int j = 0; j < R; ++j) {
             if (j & (1 << bb)) continue;
             const auto w = tw(slot<LR>(K - LO - NB, NB - 1 - bb, j, bb), LO + bb, elem<LR, LO, NB>(t, j));
-            if (RED && bb == NB - 1)
-                ar.template fwd_bf<true>(v[j], v[j | (1 << bb)], w);
+            if (bb == NB - 1)
+                ar.template fwd_bf<RED>(v[j], v[j | (1 << bb)], w);
             else
-                ar.template fwd_bf<false>(v[j], v[j | (1 << bb)], w);
+                ar.template fwd_bf<0>(v[j], v[j | (1 << bb)], w);
         }
     }
 }
@@ -278,7 +281,10 @@ __device__ __forceinline__ void fwd_run(const A& ar, typename A::V* sub, typenam
                                         const HOOK& hook = HOOK{}) {
     constexpr int NB = HI < LR ? HI : LR;
     constexpr int LO = HI - NB;
-    constexpr bool RED = ((K - HI) % 4 == 0 || LR == 3) && !(FRESH && HI == K);
+    constexpr int RED = FRESH && HI == K   ? 0
+                        : A::EACH_PHASE    ? (LR == 3 ? 2 : 1)
+                        : (K - HI) % 4 == 0 || LR == 3 ? 1
+                                                       : 0;
     hook(std::integral_constant<int, HI>{});
     fwd_bfly<LR, K, LO, NB, RED>(ar, v, t, tw);
     if constexpr (LO > 0) {
