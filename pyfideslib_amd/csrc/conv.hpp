@@ -65,11 +65,12 @@ struct MatRow {
     uint64_t v[A];
 };
 
-// sum x_i m_i mod p as a double of at most (1/2 + 2^-16) p, exact, for p < 2^50, A <= 10
+// sum x_i m_i mod p as a double of at most (1/2 + 2^-15) p, exact, for p < 2^50, A <= 12
 // and x_i < 2^60.  The halves of x_i take constants of their own, so that two
-// signed sums are enough, U of lo and V of hi parts: |U| <= 20 2^58, |V| <= 20 2^50.
+// signed sums are enough, U of lo and V of hi parts: |U| < 24 2^58, |V| <= 24 2^50, and
+// U with the low word of V on top stays below 2^63.
 // V 2^29 + U is regrouped as D 2^32 + l, D an integer below 2^53 and l one word,
-// and is at most 10 2^30 p, so its rounded quotient is off by little and what is
+// and is at most 12 2^30 p, so its rounded quotient is off by little and what is
 // left after it a small integer.  11 operations follow the sums, where four
 // unsigned sums and a 128-bit reduction took 45.
 template <int A>

@@ -349,7 +349,8 @@ static void modup_cols_a(const DevTables& T, const ModUpJobs& L, int max_nd, int
         case 7: modup_cols<LOGN, 7>(T, L, max_nd, targets, s); break;
         case 8: modup_cols<LOGN, 8>(T, L, max_nd, targets, s); break;
         case 9: modup_cols<LOGN, 9>(T, L, max_nd, targets, s); break;
-        default: modup_cols<LOGN, 10>(T, L, max_nd, targets, s); break;
+        case 10: modup_cols<LOGN, 10>(T, L, max_nd, targets, s); break;
+        default: modup_cols<LOGN, 12>(T, L, max_nd, targets, s); break;
     }
 }
 

@@ -6,7 +6,10 @@
 namespace fides {
 
 constexpr int FUSED_LOGN_MIN = 12, FUSED_LOGN_MAX = 16;
-constexpr int FUSED_CONV_MAX = 10;  // source limbs of a conversion
+// Source limbs of a conversion (11 as 12, conv_bound).  At 12 the ModDown with a rescale
+// spills 38 registers and is still ahead of the separate kernels (8 products, N = 2^15, 14
+// limbs of 59 bits, 11 special primes: 365 -> 353 us); past it sources would not fit.
+constexpr int FUSED_CONV_MAX = 12;
 constexpr int FUSED_DIGITS = 4;
 constexpr int CONV_INV_LOGN = 14;
 

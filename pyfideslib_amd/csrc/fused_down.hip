@@ -24,30 +24,30 @@ __global__ void __launch_bounds__(512, 4) k_moddown_cols(DevTables T, ModDownJob
     const uint32_t c_at = G::c_row(tid) * G::N2 + col0 + G::c_col(tid);
     const int c_tgt = __builtin_amdgcn_readfirstlane(G::c_tgt(tid));
     const int n_tgt = __builtin_amdgcn_readfirstlane(G::n_tgt(tid));
+    const int K = KK > 10 ? T.K : KK;  // past 10 the matrix rows are padded with zeros
     Half2 x[G::CPT][KK];
     uint64_t top[G::CPT];
     if constexpr (conv_inv<LOGN>()) {
         // the special limbs, and the limb that a rescale drops
         conv_sources(
-            T, S, KK + (RESCALE ? 1 : 0), col0, [&](int i) { return i < KK ? J.t + (size_t)i * G::N : J.top_acc; },
-            [&](int i) { return i < KK ? T.L + 1 + i : l; },
-            [&](int i) { return i < KK ? T.iscale_moddown + (size_t)i * 2 : T.iscale_plain + (size_t)l * 2; });
+            T, S, K + (RESCALE ? 1 : 0), col0, [&](int i) { return i < K ? J.t + (size_t)i * G::N : J.top_acc; },
+            [&](int i) { return i < K ? T.L + 1 + i : l; },
+            [&](int i) { return i < K ? T.iscale_moddown + (size_t)i * 2 : T.iscale_plain + (size_t)l * 2; });
 #pragma unroll
-        for (int i = 0; i < KK + (RESCALE ? 1 : 0); ++i)
+        for (int i = 0; i < KK; ++i)
 #pragma unroll
-            for (int c = 0; c < G::CPT; ++c) {
-                const uint64_t w = S.s.tile[i][G::c_col(tid) + c][lds_off(G::c_row(tid))];
-                if (i < KK)
-                    x[c][i < KK ? i : 0] = split30_held(w);
-                else
-                    top[c] = w;
-            }
+            for (int c = 0; c < G::CPT; ++c)
+                x[c][i] = split30_held(i < K ? S.s.tile[i][G::c_col(tid) + c][lds_off(G::c_row(tid))] : 0);
+        if constexpr (RESCALE) {
+#pragma unroll
+            for (int c = 0; c < G::CPT; ++c) top[c] = S.s.tile[K][G::c_col(tid) + c][lds_off(G::c_row(tid))];
+        }
         __syncthreads();  // the targets take over the LDS
     } else {
         uint64_t v[KK][G::CPT];
 #pragma unroll
         for (int i = 0; i < KK; ++i) {
-            const uint64_t* src = J.t + (size_t)i * G::N + c_at;
+            const uint64_t* src = J.t + (size_t)(i < K ? i : K - 1) * G::N + c_at;
             if constexpr (G::CPT == 2) {
                 const u64x2 w = ld2(src);
                 v[i][0] = w.x, v[i][1] = w.y;
@@ -62,7 +62,7 @@ __global__ void __launch_bounds__(512, 4) k_moddown_cols(DevTables T, ModDownJob
 #pragma unroll
         for (int i = 0; i < KK; ++i)
 #pragma unroll
-            for (int c = 0; c < G::CPT; ++c) x[c][i] = split30_held(v[i][c]);
+            for (int c = 0; c < G::CPT; ++c) x[c][i] = split30_held(i < K ? v[i][c] : 0);
     }
     // the dropped limb less its converted part, centered on a rescale; as a double
     // where its prime is on the FP64 units, and else in [0, q_l)
@@ -166,7 +166,8 @@ static hipError_t moddown_cols_k(const DevTables& T, const ModDownJobs& L, int t
         case 7: moddown_cols<LOGN, 7>(T, L, targets, rescale, s); break;
         case 8: moddown_cols<LOGN, 8>(T, L, targets, rescale, s); break;
         case 9: moddown_cols<LOGN, 9>(T, L, targets, rescale, s); break;
-        default: moddown_cols<LOGN, 10>(T, L, targets, rescale, s); break;
+        case 10: moddown_cols<LOGN, 10>(T, L, targets, rescale, s); break;
+        default: moddown_cols<LOGN, 12>(T, L, targets, rescale, s); break;
     }
     return hipGetLastError();
 }

@@ -11,7 +11,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("first,bits,special", [(60, 50, 60), (60, 25, 60), (50, 50, 50), (50, 25, 25), (60, 59, 50)])
-@pytest.mark.parametrize("logN,L,dnum,K", [(12, 9, 1, 10), (16, 1, 1, 1), (16, 8, 1, 9)])
+@pytest.mark.parametrize("logN,L,dnum,K", [(12, 9, 1, 10), (16, 1, 1, 1), (16, 8, 1, 9), (12, 12, 1, 13), (13, 11, 1, 12),
+                                           (14, 10, 1, 11), (15, 11, 1, 12), (16, 10, 1, 11)])
 def test_products_and_rotations(logN, L, dnum, K, first, bits, special):
     P = O.make_params(logN, first, bits, L, special, dnum, K=K)
     o, ctx, keys = make_env(P, rotations=(1,))
