@@ -5,8 +5,8 @@
 // tensor product with the row pass of its third part's inverse transform.
 //
 // At N = 2^16 a pass over the 25 to 74 limbs of a key switch is bound by memory
-// and by the latency of a launch's chain, not by arithmetic: what is fused
-// away is the write and read of every limb in between.
+// and by the latency of a launch's chain, the conversions apart, which are bound by
+// instruction issue: what is fused away is the write and read of every limb in between.
 #include "fused.hpp"
 
 namespace fides {

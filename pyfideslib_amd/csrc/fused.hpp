@@ -207,8 +207,9 @@ struct ConvGrid {
 inline XcdGrid conv_grid(size_t items, int per) {
     return items <= (size_t)32 * per ? xcd_chunks(items, XCD_TILES) : xcd_grid(items, per);
 }
-// Target groups, of whole rounds of tb targets: about 1024 blocks in all, two
-// rounds of what is resident (512 or 1600 took 5 to 10% longer at N = 2^16, level 24).
+// Target groups, of whole rounds of tb targets: up to 1024 blocks in all, two
+// rounds of what is resident (ModUp at N = 2^16, level 24: 40.3 us with 768 blocks, 45 with
+// 384, 47 with 1536; ModDown 28.4 with 768, 27.5 with 512, 33 with 256 or 1024).
 // Where whole rounds leave less than half of the CUs with a block, single targets up
 // to 192 blocks: a thread then forms one sum instead of TPT in turn (N = 2^13, 4
 // limbs: ModDown 9.2 -> 8.2 us, ModUp 8.2 -> 7.4; at 128 blocks, N = 2^14, no gain).
