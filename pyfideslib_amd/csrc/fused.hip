@@ -210,6 +210,7 @@ __global__ void __launch_bounds__(FRows<LOGN>::NTR, 4) k_rows_ksk(DevTables T, K
             for (int k = 0; k < 4; ++k) m[k] = e[in0 + elem<2, G::LO1, G::NB1>(t, k)];
 #pragma unroll
             for (int k = 0; k < 4; ++k) v[k] = A::unpack(m[k]);
+            lds_sync<G::WAVE>();  // the row pass before has read its words
             fwd_row<G, false>(ar, sub, v, t, G::N1 + r, tf);
 #pragma unroll
             for (int k = 0; k < 4; ++k) v[k] = ar.term_fwd(v[k]);
@@ -285,6 +286,7 @@ __global__ void __launch_bounds__(FRows<LOGN>::NTR, 4) k_rows_ksk(DevTables T, K
                 a[2] = ar.mul_add(a[2], pinv, f1.x);
                 a[3] = ar.mul_add(a[3], pinv, f1.y);
             }
+            lds_sync<G::WAVE>();  // the row pass before has read its words
             inv_row<G>(ar, sub, a, t, G::N1 + r, A::inv(T) + (size_t)pid * G::N);
             gu64* o = gp(down) + (special ? (size_t)(1 + pos - nl) * G::N : (size_t)0);
 #pragma unroll

@@ -259,6 +259,8 @@ __device__ __forceinline__ void fwd_bfly(const A& ar, typename A::V* v, uint32_t
 // elements of the last phase (bits [0, fwd_last_nb)), which the caller stores
 // straight to global memory.  One barrier per exchange: a thread writes back
 // exactly the elements it read, so reads and writes of one phase never race.
+// That holds within a pass: whoever runs another pass on the same LDS waits first
+// (lds_sync).
 // hook(integral_constant<HI>) runs at the start of each phase (the row pass
 // issues later phases' twiddle loads there).
 template <bool WAVE>
