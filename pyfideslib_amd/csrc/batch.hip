@@ -88,6 +88,15 @@ static int item_level(const KsItem& it) {
     return it.mult ? std::min(it.a->level, it.b->level) : it.a->level;
 }
 
+// Scratch layout per item: [d2 (mult)], t, ext, acc_a, acc_b, then what goes down
+// to Q (fused: per part the limb that a rescale drops and the K special limbs;
+// separate kernels: tk(2K)), y(2nl), [separate kernels: top(4) (rescale)].
+size_t ks_scratch_words(const Context& c, int level, bool mult, bool rescale) {
+    const size_t nl = level + 1, npos = nl + c.K, nd = c.num_digits(level);
+    const size_t down = fused_ok(c.T) ? 2 * (c.K + 1) : 2 * c.K + (rescale ? 4 : 0);
+    return ((mult ? nl : 0) + nl + nd * npos + 2 * npos + down + 2 * nl) * c.N;
+}
+
 static std::shared_ptr<BatchPlan> build_plan(Context& c, const std::vector<KsItem>& items, std::vector<uint64_t> sig) {
     auto P = std::make_shared<BatchPlan>();
     P->sig = std::move(sig);
@@ -95,17 +104,14 @@ static std::shared_ptr<BatchPlan> build_plan(Context& c, const std::vector<KsIte
     const size_t N = c.N;
     const int K = c.K;
     P->fused = fused_ok(c.T);
-    // scratch layout per item: [d2 (mult)], t, ext, acc_a, acc_b, tk(2K + 2), y(2nl), [top(4) (rescale)]
     std::vector<size_t> off(P->n + 1, 0);
     for (int i = 0; i < P->n; ++i) {
         const KsItem& it = items[i];
         const int l = item_level(it);
-        const size_t nl = l + 1, npos = nl + K, nd = c.num_digits(l);
-        const size_t words = (it.mult ? nl : 0) + nl + nd * npos + 2 * npos + 2 * K + 2 + 2 * nl + (it.rescale ? 4 : 0);
-        off[i + 1] = off[i] + words * N;
-        P->max_nl = std::max(P->max_nl, (int)nl);
-        P->max_nd = std::max(P->max_nd, (int)nd);
-        P->max_npos = std::max(P->max_npos, (int)npos);
+        off[i + 1] = off[i] + ks_scratch_words(c, l, it.mult, it.mult && it.rescale);
+        P->max_nl = std::max(P->max_nl, l + 1);
+        P->max_nd = std::max(P->max_nd, c.num_digits(l));
+        P->max_npos = std::max(P->max_npos, l + 1 + K);
     }
     uint64_t* base = c.batch_arena(off[P->n]);
 
@@ -124,8 +130,10 @@ static std::shared_ptr<BatchPlan> build_plan(Context& c, const std::vector<KsIte
         uint64_t* acc_a = ext + (size_t)nd * npos * N;
         uint64_t* acc_b = acc_a + npos * N;
         uint64_t* tk = acc_b + npos * N;
-        uint64_t* y = tk + (2 * K + 2) * N;
+        uint64_t* y = tk + (size_t)2 * (K + P->fused) * N;
         uint64_t* top = y + 2 * nl * N;
+        if (top + (!P->fused && it.mult && it.rescale ? 4 * N : 0) != base + off[i + 1])
+            throw Error(E_STATE, "batch scratch: layout and size disagree");
         Ciphertext& O = *it.out;
         // the key-switch input: c1 d1 (mult, from the tensor) or c1 (rotation)
         const uint64_t* x = it.mult ? d2 : it.a->c1();
@@ -487,8 +495,9 @@ static std::shared_ptr<HoistPlan> build_hoist_plan(Context& c, const Ciphertext&
     for (uint32_t k : ks) nk += (k != 1);
     P->nk = nk;
     P->fused = fused_ok(c.T);
-    // scratch: t, ext, then per key-switched rotation acc_a, acc_b, tk(2K + 2), y(2nl)
-    const size_t per = 2 * npos + 2 * K + 2 + 2 * nl;
+    // scratch: t, ext, then per key-switched rotation acc_a, acc_b, tk(2K; fused: one
+    // limb before each part, KskJob's layout), y(2nl)
+    const size_t per = 2 * npos + 2 * (K + P->fused) + 2 * nl;
     P->scratch = DevBuf(&c.pool, (nl + (size_t)nd * npos + per * nk) * N);
     P->t = P->scratch.ptr;
     P->ext = P->t + nl * N;
@@ -509,8 +518,8 @@ static std::shared_ptr<HoistPlan> build_hoist_plan(Context& c, const Ciphertext&
         uint64_t* s = base + per * r * N;
         uint64_t* acc_a = s;
         uint64_t* acc_b = acc_a + npos * N;
-        uint64_t* tka = acc_b + npos * N + N;  // one limb before each part: KskJob's layout
-        uint64_t* tkb = tka + (size_t)(K + 1) * N;
+        uint64_t* tka = acc_b + (npos + P->fused) * N;
+        uint64_t* tkb = tka + (size_t)(K + P->fused) * N;
         uint64_t* ya = tkb + (size_t)K * N;
         uint64_t* yb = ya + nl * N;
         const uint32_t kinv = c.auto_inverse(ks[i]);

@@ -127,7 +127,8 @@ struct KsScratch {
         ext = DevBuf(&c.pool, (size_t)c.num_digits(level) * npos * N);
         acc_a = DevBuf(&c.pool, npos * N);
         acc_b = DevBuf(&c.pool, npos * N);
-        tk = DevBuf(&c.pool, (size_t)2 * (c.K + 1) * N);  // per part: the limb a rescale drops, K special limbs
+        // per part K special limbs, and on the fused kernels the limb a rescale drops
+        tk = DevBuf(&c.pool, (size_t)2 * (c.K + fused_ok(c.T)) * N);
         y = DevBuf(&c.pool, 2 * nl * N);
         if (mult) {
             d2 = DevBuf(&c.pool, nl * N);

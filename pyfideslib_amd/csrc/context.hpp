@@ -391,6 +391,8 @@ struct KsItem {
     bool rescale;
 };
 void ks_batch(Context& c, const std::vector<KsItem>& items);
+// Words of scratch that one item takes of a batch's arena (what a server admits it for).
+size_t ks_scratch_words(const Context& c, int level, bool mult, bool rescale);
 void eval_rotate_batch(Context& c, const std::vector<const Ciphertext*>& a, const std::vector<int>& idx,
                        const std::vector<Ciphertext*>& out);
 

@@ -112,11 +112,8 @@ class Server {
 
    private:
     size_t ct_bytes() const { return c_.ct_words() * 8; }
-    // Scratch of one key-switched op at `level` in a batch plan (batch.hip layout).
-    size_t ks_bytes(int level, bool mult) const {
-        const size_t nl = level + 1, npos = nl + c_.K, nd = c_.num_digits(level);
-        return ((mult ? nl : 0) + nl + nd * npos + 2 * npos + 2 * c_.K + 2 * nl + 4) * c_.N * 8;
-    }
+    // Scratch of one key-switched op at `level` in a batch plan.
+    size_t ks_bytes(int level, bool mult) const { return ks_scratch_words(c_, level, mult, mult) * 8; }
     size_t footprint(const Job& j) const {
         const int l = j.a->level;
         if (j.kind == JOB_LOGREG) return 6 * ct_bytes() + ks_bytes(l, true);
