@@ -514,10 +514,14 @@ int fides_stage_modup(fides_context* ctx, int32_t level, const uint64_t* x, uint
  * kind: FIDES_TUNE_NTT_FWD / _NTT_INV (size = limbs per launch; cfg = column
  * tile width, log2 values per column thread, row tile height, unused) or
  * FIDES_TUNE_MODUP / _MODDOWN (size = conversions per launch; cfg[0] =
- * target groups; FIDES_TUNE_MODUP cfg[1] = 1 selects the int8 matrix-core
- * conversion, built when the digit has at most 16 limbs).  fides_tune_force pins a kind's configuration for every
- * later launch in the process (cfg NULL releases it; kind < 0 releases all);
- * fides_tune_config reports what a launch of that size would use. */
+ * target groups of the conversion, by itself or fused with its transform's
+ * first pass; FIDES_TUNE_MODUP cfg[1] = 1 selects the int8 matrix-core
+ * conversion, built when the digit has at most 16 limbs and the sums fit one
+ * reduction: key switches of a ring that it is selected for run on the separate
+ * kernels).  fides_tune_force pins a kind's configuration for every later call
+ * in the process (cfg NULL releases it; kind < 0 releases all);
+ * fides_tune_config reports what a launch of that size would use, of a key
+ * switch's conversions at the top level with that many. */
 #define FIDES_TUNE_NTT_FWD 0
 #define FIDES_TUNE_NTT_INV 1
 #define FIDES_TUNE_MODUP 2
@@ -528,6 +532,10 @@ int fides_tune_load(const char* path, int32_t* entries); /* path NULL: fixed rul
 int fides_ntt_limbs(fides_context* ctx, uint64_t* data, int32_t limbs, int32_t inverse);
 int fides_tune_force(int32_t kind, const int32_t* cfg);
 int fides_tune_config(fides_context* ctx, int32_t kind, int32_t size, int32_t* cfg, int32_t* from_table);
+/* Whether this context's key switches run on the fused kernels: rings of 2^12 to
+ * 2^16, few enough digits and conversion sources, and no matrix-core ModUp
+ * configured. */
+int fides_context_fused(fides_context* ctx, int32_t* fused);
 /* fides_stage_modup without any device allocation: its (level+1)*N-word
  * workspace is a static 16 MiB (2^21-word) device array, one per GPU, held
  * until the process ends.  No counterpart in the reference; it is for callers

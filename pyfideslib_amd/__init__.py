@@ -43,7 +43,7 @@ SYMBOLS = [
     "fides_ct_copy", "fides_ct_device_ptrs", "fides_key_load_eval", "fides_key_load_rotation",
     "fides_key_load_automorph", "fides_rotation_automorph_index", "fides_eval_mult", "fides_eval_square",
     "fides_rescale", "fides_eval_add", "fides_eval_sub", "fides_eval_rotate", "fides_eval_rotate_hoisted",
-    "fides_eval_mult_batch", "fides_poly_ntt", "fides_stage_modup", "fides_stage_modup_noalloc", "fides_tune_load", "fides_tune_force", "fides_tune_config", "fides_ntt_limbs", "fides_stage_moddown",
+    "fides_eval_mult_batch", "fides_poly_ntt", "fides_stage_modup", "fides_stage_modup_noalloc", "fides_tune_load", "fides_tune_force", "fides_tune_config", "fides_context_fused", "fides_ntt_limbs", "fides_stage_moddown",
     "fides_stage_keyswitch", "fides_pt_create", "fides_pt_destroy", "fides_pt_load", "fides_eval_mult_plain",
     "fides_eval_add_plain", "fides_eval_mult_scalar", "fides_eval_add_scalar", "fides_drop_to_level",
     "fides_scalar_encoding", "fides_eval_rotate_batch", "fides_server_create", "fides_server_destroy",
@@ -145,6 +145,7 @@ def lib():
         L.fides_tune_load.argtypes = [C.c_char_p, C.POINTER(i32)]
         L.fides_ntt_limbs.argtypes = [vp, vp, i32, i32]
         L.fides_tune_force.argtypes = [i32, C.POINTER(i32)]
+        L.fides_context_fused.argtypes = [vp, C.POINTER(i32)]
         L.fides_tune_config.argtypes = [vp, i32, i32, C.POINTER(i32), C.POINTER(i32)]
         L.fides_stage_moddown.argtypes = [vp, i32, vp, vp]
         L.fides_stage_keyswitch.argtypes = [vp, i32, vp, u32, vp, vp]
@@ -649,6 +650,13 @@ class Context:
         cfg, tab = (C.c_int32 * 4)(), C.c_int32()
         _check(lib().fides_tune_config(self.h, kind, size, cfg, C.byref(tab)))
         return [int(x) for x in cfg], bool(tab.value)
+
+    @property
+    def fused(self) -> bool:
+        """Whether key switches run on the fused kernels (parameters and tuning configuration permitting)."""
+        v = C.c_int32()
+        _check(lib().fides_context_fused(self.h, C.byref(v)))
+        return bool(v.value)
 
     def stage_modup_noalloc(self, level: int, x, ext):
         """ModUp with the library's static device workspace (no allocation)."""

@@ -50,10 +50,11 @@ struct BatchPlan {
     const int* ksk_chunks = nullptr;
     int n_ksk_chunks = 0;
     bool keystat = false;  // at least two jobs per key on average
-    bool fused = false;    // fused.hip's kernels (fused_ok)
+    bool fused = false;    // fused.hip's kernels (Context::fused)
 };
 
-// Key-stationary KSK for single-key batches (FIDES_KSK_KEYSTAT=0 turns it off).
+// Key-stationary KSK for single-key batches on the separate kernels
+// (FIDES_KSK_KEYSTAT=0 turns it off; the fused inner product has no such form).
 bool ksk_keystat_on() {
     static const bool on = [] {
         const char* e = std::getenv("FIDES_KSK_KEYSTAT");
@@ -93,7 +94,7 @@ static int item_level(const KsItem& it) {
 // separate kernels: tk(2K)), y(2nl), [separate kernels: top(4) (rescale)].
 size_t ks_scratch_words(const Context& c, int level, bool mult, bool rescale) {
     const size_t nl = level + 1, npos = nl + c.K, nd = c.num_digits(level);
-    const size_t down = fused_ok(c.T) ? 2 * (c.K + 1) : 2 * c.K + (rescale ? 4 : 0);
+    const size_t down = c.fused ? 2 * (c.K + 1) : 2 * c.K + (rescale ? 4 : 0);
     return ((mult ? nl : 0) + nl + nd * npos + 2 * npos + down + 2 * nl) * c.N;
 }
 
@@ -103,7 +104,7 @@ static std::shared_ptr<BatchPlan> build_plan(Context& c, const std::vector<KsIte
     P->n = (int)items.size();
     const size_t N = c.N;
     const int K = c.K;
-    P->fused = fused_ok(c.T);
+    P->fused = c.fused;
     std::vector<size_t> off(P->n + 1, 0);
     for (int i = 0; i < P->n; ++i) {
         const KsItem& it = items[i];
@@ -354,7 +355,7 @@ static void run_plan(Context& c, const BatchPlan& P) {
 void ks_batch(Context& c, const std::vector<KsItem>& items) {
     const size_t n = items.size();
     if (n == 0) return;
-    std::vector<uint64_t> sig{tune_epoch()};
+    std::vector<uint64_t> sig{tune_epoch(), c.fused};
     for (size_t i = 0; i < n; ++i) {
         const KsItem& it = items[i];
         if (!it.a || !it.out || !it.key || (it.mult && !it.b)) throw Error(E_ARG, "incomplete batch item");
@@ -472,7 +473,7 @@ struct HoistPlan {
     }
     DevBuf scratch, table;
     int level = 0, nk = 0, npos = 0;
-    bool fused = false;  // fused.hip's kernels (fused_ok)
+    bool fused = false;  // fused.hip's kernels (Context::fused)
     const uint64_t *c0 = nullptr, *c1 = nullptr;
     uint64_t *t = nullptr, *ext = nullptr;
     const KskJob* ksk = nullptr;
@@ -494,7 +495,7 @@ static std::shared_ptr<HoistPlan> build_hoist_plan(Context& c, const Ciphertext&
     int nk = 0;
     for (uint32_t k : ks) nk += (k != 1);
     P->nk = nk;
-    P->fused = fused_ok(c.T);
+    P->fused = c.fused;
     // scratch: t, ext, then per key-switched rotation acc_a, acc_b, tk(2K; fused: one
     // limb before each part, KskJob's layout), y(2nl)
     const size_t per = 2 * npos + 2 * (K + P->fused) + 2 * nl;
@@ -606,7 +607,7 @@ static void run_hoist_plan(Context& c, const HoistPlan& P) {
 void rotate_hoisted_batch(Context& c, const Ciphertext& a, const std::vector<uint32_t>& ks,
                           const std::vector<Ciphertext*>& outs) {
     std::vector<uint64_t> sig{(uint64_t)(uintptr_t)a.c0(), (uint64_t)a.level, (uint64_t)(uintptr_t)a.c1(),
-                              tune_epoch()};
+                              tune_epoch(), c.fused};
     for (size_t i = 0; i < ks.size(); ++i) {
         sig.push_back(ks[i]);
         if (ks[i] != 1) {

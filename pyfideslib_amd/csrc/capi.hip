@@ -45,6 +45,7 @@ static int guard_ctx(fides_context* ctx, F&& f) {
         return FIDES_E_ARG;
     }
     std::lock_guard<std::recursive_mutex> lk(ctx->c->api_mu);
+    ctx->c->enter();
     return guard(std::forward<F>(f));
 }
 
@@ -1062,11 +1063,20 @@ int fides_tune_config(fides_context* ctx, int32_t kind, int32_t size, int32_t* c
                 t = ntt_rule_cfg(kind == TUNE_NTT_FWD, c.logN, size);
             } else {
                 const int targets = kind == TUNE_MODUP ? c.L + 1 + c.K - c.alpha : c.L + 1;
-                t = TuneCfg{{conv_rule_tg((c.N / 256) * size, targets), 0, 0, 0}};
+                const int set = conv_set_tg(kind, c.logN, size, targets);
+                t = TuneCfg{{c.fused ? fused_conv_tg(c.T, kind, size)
+                             : set   ? set
+                                     : conv_rule_tg((c.N / 256) * size, targets), 0, 0, 0}};
             }
         }
         for (int i = 0; i < TUNE_NV; ++i) cfg[i] = t.v[i];
         if (from_table) *from_table = tab ? 1 : 0;
+    });
+}
+int fides_context_fused(fides_context* ctx, int32_t* fused) {
+    return guard_ctx(ctx, [&] {
+        if (!fused) throw Error(E_ARG, "null out");
+        *fused = C(ctx).fused;
     });
 }
 int fides_stage_modup_noalloc(fides_context* ctx, int32_t level, const uint64_t* x, uint64_t* ext) {

@@ -167,6 +167,7 @@ static void run_cached(Context& c, const std::vector<uint64_t>& sig_in, Body bod
     }
     std::vector<uint64_t> sig(sig_in);
     sig.push_back(tune_epoch());  // the launch configurations the capture bakes in
+    sig.push_back(c.fused);
     auto it = c.graph_cache.find(sig);
     if (it == c.graph_cache.end()) {
         // capture only signatures seen before: one-off operand sets (a stream
@@ -199,7 +200,7 @@ static void modup_intt(Context& c, int level, const uint64_t* x, uint64_t* t, in
     run_ntt(c, {ji}, true, LOAD_PLAIN, STORE_PLAIN, passes);
 }
 
-// The digits of t converted and transformed up to the second pass (fused_ok).
+// The digits of t converted and transformed up to the second pass (Context::fused).
 static void modup_cols(Context& c, int level, const uint64_t* t, uint64_t* ext) {
     ModUpJobs mj = inline_list<ModUpJobs>();
     mj.inl[0] = ModUpJob{t, ext, level};
@@ -364,7 +365,7 @@ static void ksk_moddown_rescale(Context& c, int level, const uint64_t* ext, cons
 static void key_switch(Context& c, int level, const uint64_t* x, const KeySwitchingKey& key, KsScratch& s,
                        uint64_t* out_b, const uint64_t* add_b, uint64_t* out_a, const uint64_t* add_a,
                        uint32_t autok = 0) {
-    if (fused_ok(c.T)) {
+    if (c.fused) {
         modup_half(c, level, x, s.t.ptr, s.ext.ptr);
         fused_ksk_moddown(c, level, s.ext.ptr, x, key, s, out_b, add_b, out_a, add_a, false, autok);
         return;
@@ -421,7 +422,7 @@ static void mult_core(Context& c, const Ciphertext* a, const Ciphertext* b, Ciph
         TensorJobs tj = inline_list<TensorJobs>();
         tj.inl[0] = TensorJob{a0, a1, b0, b1, o0, o1, s.d2.ptr, nl, 0, s.t.ptr};
         tj.n = 1;
-        if (fused_ok(c.T)) {
+        if (c.fused) {
             ck(launch_tensor_rows(c.T, tj, nl, c.stream), "tensor and rows");
             if (!fused_inv_cols(c.T)) modup_intt(c, level, s.d2.ptr, s.t.ptr, NTT_PASS2);
             modup_cols(c, level, s.t.ptr, s.ext.ptr);

@@ -163,6 +163,7 @@ Context::Context(const Params& p, int dev) {
     build_tables(p.roots);
     noalloc_init(device);
     tune_load_default();
+    enter();
 }
 
 Context::~Context() {
@@ -181,6 +182,13 @@ Context::~Context() {
     eval_key.reset();
     rot_keys.clear();
     if (blob_) (void)hipFree(blob_);
+}
+
+void Context::enter() {
+    const uint64_t e = tune_epoch();
+    if (e == tune_seen_) return;
+    tune_seen_ = e;
+    fused = fused_ok(T) && !(T.modup_mfma_ms > 0 && tune_matrix_cores(logN));
 }
 
 void Context::sync() { hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize"); }

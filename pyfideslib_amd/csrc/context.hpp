@@ -145,6 +145,12 @@ class Context {
     std::vector<double> scaling_factor_real_big;
     hipStream_t stream = nullptr;
     DevTables T{};
+    // Key switches of the present call run on the fused kernels: fused_ok, unless the
+    // tuning configuration puts a ModUp of this ring on the matrix cores (k_modup_mfma,
+    // a separate kernel).  Set as a call enters (under api_mu), so that all of a call
+    // goes one way whatever other threads configure meanwhile.
+    bool fused = false;
+    void enter();
     Pool pool;
     std::unique_ptr<KeySwitchingKey> eval_key;
     std::map<uint32_t, std::unique_ptr<KeySwitchingKey>> rot_keys;  // by automorphism index
@@ -203,6 +209,7 @@ class Context {
     uint64_t* batch_arena(size_t words);
 
    private:
+    uint64_t tune_seen_ = 0;  // the epoch that `fused` was set at
     void* blob_ = nullptr;
     // pinned staging ring for upload(): a slot is reused once the copy from it
     // has run, so the host may queue up to STAGE_SLOTS uploads ahead of the
@@ -391,7 +398,8 @@ struct KsItem {
     bool rescale;
 };
 void ks_batch(Context& c, const std::vector<KsItem>& items);
-// Words of scratch that one item takes of a batch's arena (what a server admits it for).
+// Words of scratch that one item takes of a batch's arena (what a server admits it
+// for), on the kernels that c.fused names.
 size_t ks_scratch_words(const Context& c, int level, bool mult, bool rescale);
 void eval_rotate_batch(Context& c, const std::vector<const Ciphertext*>& a, const std::vector<int>& idx,
                        const std::vector<Ciphertext*>& out);
@@ -413,7 +421,7 @@ void rotate_hoisted_batch(Context& c, const Ciphertext& a, const std::vector<uin
 // NTT jobs, NTT_INLINE per launch (ckks.hip).
 void run_ntt_jobs(Context& c, std::vector<NttJob> jobs, bool inverse, int load = LOAD_PLAIN, int store = STORE_PLAIN,
                   int passes = NTT_BOTH);
-// ModUp of x up to what launch_rows_ksk takes (fused_ok).
+// ModUp of x up to what launch_rows_ksk takes (Context::fused).
 void modup_half(Context& c, int level, const uint64_t* x, uint64_t* t, uint64_t* ext);
 // The rest of its transforms, for several keys: ext in evaluation form.
 void modup_rows(Context& c, int level, uint64_t* ext);

@@ -383,11 +383,17 @@ struct TuneCfg {
 };
 // A forced configuration (tune_force), else the table's entry: true if found.
 bool tune_get(int kind, int logN, int size, TuneCfg& out);
+bool tune_matrix_cores(int logN);               // some ModUp of this ring is configured onto the matrix cores
 void tune_force(int kind, const TuneCfg* cfg);  // nullptr clears the kind; kind < 0 clears all
 int tune_load(const char* path);                // entries read, -1 when the file cannot be read
 void tune_load_default();                       // FIDES_TUNE_FILE, else the table next to the library
 uint64_t tune_epoch();                          // changes whenever a lookup result may change
 // The fixed rules (used when no entry applies), for reports.
+// Target groups that a forced configuration, the table or FIDES_CONV_TG sets for
+// `convs` conversions per launch, at most max_targets; 0: the launcher's rule.
+int conv_set_tg(int kind, int logN, int convs, int max_targets);
+// The fused conversions' groups (fused_ok), of the top level that many conversions come from.
+int fused_conv_tg(const DevTables& T, int kind, int convs);
 TuneCfg ntt_rule_cfg(bool forward, int logN, int limbs);
 int conv_rule_tg(int base_blocks, int max_targets);
 

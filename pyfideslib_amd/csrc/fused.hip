@@ -332,7 +332,7 @@ hipError_t launch_tensor_rows(const DevTables& T, const TensorJobs& L, int max_n
 template <int LOGN, int A>
 static void modup_cols(const DevTables& T, const ModUpJobs& L, int max_nd, int targets, hipStream_t s) {
     using G = ConvCols<LOGN>;
-    const int tg = fused_groups((size_t)G::TPL * max_nd * L.n, targets, G::TB);
+    const int tg = conv_launch_groups(TUNE_MODUP, LOGN, max_nd * L.n, (size_t)G::TPL * max_nd * L.n, targets, G::TB);
     const size_t items = (size_t)L.n * max_nd * tg * G::TPL;
     const XcdGrid x = conv_grid(items, G::TPL);
     const ConvGrid g{(uint32_t)items, x.chunk, FastDiv(tg, items), FastDiv(max_nd, items)};
@@ -356,13 +356,26 @@ static void modup_cols_a(const DevTables& T, const ModUpJobs& L, int max_nd, int
     }
 }
 
+// The most targets a digit of any level up to the list's top has: all
+// positions but a full digit's (or all but the top level's, within one digit).
+static int modup_targets(const DevTables& T, int max_nl) { return T.K + (max_nl > T.alpha ? max_nl - 1 : 0); }
+
 hipError_t launch_modup_cols(const DevTables& T, const ModUpJobs& L, int max_nd, int max_nl, hipStream_t s) {
     if (L.n <= 0 || max_nd <= 0) return hipSuccess;
     if (!fused_ok(T)) return hipErrorInvalidValue;
-    // the most targets a digit of any level up to the list's top has: all
-    // positions but a full digit's (or all but the top level's, within one digit)
-    const int targets = T.K + (max_nl > T.alpha ? max_nl - 1 : 0);
+    const int targets = modup_targets(T, max_nl);
     return by_logn(T.logN, [&](auto ln) { modup_cols_a<decltype(ln)::value>(T, L, max_nd, targets, s); });
+}
+
+int fused_conv_tg(const DevTables& T, int kind, int convs) {
+    const int nl = kind == TUNE_MODUP && convs < T.dnum ? convs * T.alpha : T.L + 1;
+    const int targets = kind == TUNE_MODUP ? modup_targets(T, nl) : nl;
+    int tg = 0;
+    (void)by_logn(T.logN, [&](auto ln) {
+        using G = ConvCols<decltype(ln)::value>;
+        tg = conv_launch_groups(kind, T.logN, convs, (size_t)G::TPL * convs, targets, G::TB);
+    });
+    return tg;
 }
 
 hipError_t launch_rows_ksk(const DevTables& T, const KskJobs& L, int max_npos, hipStream_t s, bool eval, bool rot) {

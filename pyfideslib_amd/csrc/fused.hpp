@@ -226,6 +226,12 @@ inline int fused_groups(size_t base_blocks, int targets, int tb) {
     return (int)((rounds + each - 1) / each);
 }
 
+// The groups of a launch of `convs` conversions.
+inline int conv_launch_groups(int kind, int logN, int convs, size_t base_blocks, int targets, int tb) {
+    const int tg = conv_set_tg(kind, logN, convs, targets);
+    return tg ? tg : fused_groups(base_blocks, targets, tb);
+}
+
 // The exact sum over the A sources of x_i m_i (m: one matrix row, scalar
 // loads), before its reduction.
 template <int A>

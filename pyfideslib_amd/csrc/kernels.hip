@@ -849,28 +849,28 @@ hipError_t launch_tensor(const DevTables& T, const TensorJobs& L, int max_nl, hi
     return hipGetLastError();
 }
 
-// Target groups per coefficient range: enough blocks to fill the GPU
-// (FIDES_CONV_TG forces a count).
-int conv_rule_tg(int base_blocks, int max_targets) {
-    static const int forced = [] {
+// Target groups that the table (or a forced configuration), or else FIDES_CONV_TG,
+// sets for `convs` conversions per launch; 0 where neither does.
+int conv_set_tg(int kind, int logN, int convs, int max_targets) {
+    static const int env = [] {
         const char* e = std::getenv("FIDES_CONV_TG");
         return e ? std::atoi(e) : 0;
     }();
-    if (forced > 0) return forced < max_targets ? forced : (max_targets > 0 ? max_targets : 1);
+    TuneCfg c;
+    const int tg = tune_get(kind, logN, convs, c) ? c.v[0] : env;
+    return tg <= 0 ? 0 : tg < max_targets ? tg : (max_targets > 0 ? max_targets : 1);
+}
+
+// Target groups per coefficient range: enough blocks to fill the GPU.
+int conv_rule_tg(int base_blocks, int max_targets) {
     int tg = (CV_MIN_BLOCKS + base_blocks - 1) / base_blocks;
     tg = tg < 1 ? 1 : (tg > 4 ? 4 : tg);
     return tg > max_targets ? (max_targets > 0 ? max_targets : 1) : tg;
 }
 
-// The measured table's target groups for `convs` conversions per launch
-// (pyfideslib_amd/tune.py), else the rule above; at most max_targets.
 static int conv_groups(int kind, int logN, int convs, int base_blocks, int max_targets) {
-    TuneCfg c;
-    if (tune_get(kind, logN, convs, c)) {
-        const int tg = c.v[0];
-        return tg < max_targets ? tg : (max_targets > 0 ? max_targets : 1);
-    }
-    return conv_rule_tg(base_blocks, max_targets);
+    const int tg = conv_set_tg(kind, logN, convs, max_targets);
+    return tg ? tg : conv_rule_tg(base_blocks, max_targets);
 }
 
 template <int A>

@@ -168,7 +168,7 @@ void ext_keyswitch(Context& c, int level, const std::vector<KsReq>& reqs, std::v
     std::vector<const uint64_t*> xs;
     for (const KsReq& r : reqs)
         if (std::find(xs.begin(), xs.end(), r.x) == xs.end()) xs.push_back(r.x);
-    const bool fused = fused_ok(c.T);
+    const bool fused = c.fused;
     if (!inv) keep.emplace_back(&c.pool, (fused ? xs.size() : 1) * nl * N);
     uint64_t* t = inv ? inv : keep.back().ptr;
     keep.emplace_back(&c.pool, xs.size() * nd * npos * N);
@@ -288,9 +288,9 @@ uint64_t* ext_moddown(Context& c, int level, const std::vector<std::pair<const u
         f.nq = nl;
         fwd.push_back(f);
     }
-    const int passes = (rows ? 0 : NTT_PASS1) | (fused_inv_cols(c.T) ? 0 : NTT_PASS2);
+    const int passes = (rows ? 0 : NTT_PASS1) | (c.fused && fused_inv_cols(c.T) ? 0 : NTT_PASS2);
     if (passes) run_ntt_jobs(c, isp, true, LOAD_PLAIN, STORE_PLAIN, passes);
-    if (fused_ok(c.T)) {
+    if (c.fused) {
         ck(launch_moddown_cols(c.T, job_list<ModDownJobs>(c, keep, md), nl, false, c.stream), "ext moddown and columns");
         run_ntt_jobs(c, fwd, false, LOAD_PLAIN, switched ? STORE_MODDOWN_INV : STORE_MODDOWN, NTT_PASS2);
         return switched ? y : nullptr;
@@ -331,7 +331,7 @@ void ext_switch_rotate(Context& c, int level, const std::vector<KsReq>& reqs, co
     for (const KsReq& r : reqs)
         for (const RotOut& o : outs)
             if (o.terms.size() == 1 && o.terms[0].acc_a == r.acc_a && !o.terms[0].add1) rots.push_back(&o);
-    if (!fused_ok(c.T) || rots.size() != reqs.size()) {
+    if (!c.fused || rots.size() != reqs.size()) {
         ext_keyswitch(c, level, reqs, keep, {}, {}, inv);
         ext_rot_outs(c, level, outs, keep);
         return;
@@ -399,7 +399,7 @@ static void lt_ext(Context& c, const std::vector<const Ciphertext*>& as, const s
     const int64_t gstep = (int64_t)bstep * stride;
     if (!batched_giant) {
         uint64_t* rows = nullptr;  // special limbs of the running sums' c1, row pass done
-        uint64_t* next_rows = g > 2 && fused_ok(c.T) ? alloc((size_t)B * c.K * N) : nullptr;
+        uint64_t* next_rows = g > 2 && c.fused ? alloc((size_t)B * c.K * N) : nullptr;
         for (int j = g - 2; j >= 0; --j) {
             std::vector<RotOut> ro;
             if (gstep % half != 0) {
@@ -417,7 +417,7 @@ static void lt_ext(Context& c, const std::vector<const Ciphertext*>& as, const s
                 // the next giant step takes c1 of these sums down
                 rows = nullptr;
                 std::vector<uint64_t*> downs;
-                if (j > 0 && fused_ok(c.T)) {
+                if (j > 0 && c.fused) {
                     rows = next_rows;
                     for (int k = 0; k < B; ++k) downs.push_back(rows + (size_t)k * c.K * N);
                 }

@@ -73,6 +73,14 @@ bool tune_get(int kind, int logN, int size, TuneCfg& out) {
     return false;
 }
 
+bool tune_matrix_cores(int logN) {
+    std::lock_guard<std::mutex> lk(g_mu);
+    if (g_forced[TUNE_MODUP]) return g_force[TUNE_MODUP].v[1] == 1;
+    for (const Entry& e : g_table)
+        if (e.kind == TUNE_MODUP && e.logN == logN && e.cfg.v[1] == 1) return true;
+    return false;
+}
+
 void tune_force(int kind, const TuneCfg* cfg) {
     std::lock_guard<std::mutex> lk(g_mu);
     g_epoch.fetch_add(1, std::memory_order_relaxed);

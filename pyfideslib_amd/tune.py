@@ -7,11 +7,10 @@ context's stream:
     shapes of single ops and of batched stages; fides_ntt_limbs) over every
     column tile width (4, 8, 16), values per column thread (4, 8), row tile
     height (4, 8, 16);
-  * the ModUp conversion's target groups at 1, 2 and 3 digit conversions per
-    launch (fides_stage_modup at levels with that many digits), and the int8
-    matrix-core form of the same conversion against them, and the ModDown
-    conversion's at the two conversions of a key switch (fides_stage_keyswitch
-    at the top level);
+  * the conversions' target groups through whole key switches
+    (fides_stage_keyswitch): the ModUp's at 1, 2 and 3 digit conversions per
+    launch (levels with that many digits), with the int8 matrix-core form
+    against them, and the ModDown's at its two conversions (top level);
 
 keeps the fastest configuration of each size (the fixed rule's unless the
 fastest beats it by more than --margin, so timing noise picks nothing), and
@@ -19,7 +18,8 @@ writes the table the
 library loads (``tune_gfx950.txt`` next to libfides_amd.so, or
 FIDES_TUNE_FILE).  Each size's entry covers the limb counts up to halfway to
 the next measured size (geometric midpoint); the largest covers every larger
-launch.  The report compares every pick with the fixed rules the library
+launch.  A conversion's entry is written only where it beats the rule, which
+also knows the level; an entry holds at every level.  The report compares every pick with the fixed rules the library
 falls back to.
 
     python -m pyfideslib_amd.tune [--logn 16 13] [--out FILE] [--reps 20]
@@ -130,51 +130,39 @@ def tune_conv(F, ctx, raw, reps: int, margin: float, log):
                                                for _ in range(dnum)])) for _ in range(2))
     ctx.load_eval_key(key)
     rows = []
+
+    def pick(kind, name, size, level, cands):
+        """Times key switches at `level` under each configuration (target groups, matrix cores)."""
+        x = ctx.device_array((level + 1, N), np.stack([rng.integers(0, mods[i], N, dtype=np.uint64)
+                                                        for i in range(level + 1)]))
+        kb, ka = ctx.device_array((level + 1, N)), ctx.device_array((level + 1, N))
+        F.tune_force(kind, None)
+        rule = (ctx.tune_config(kind, size)[0][0], 0)
+        res = {}
+        for cfg in sorted(set(cands) | {rule}):
+            try:
+                F.tune_force(kind, list(cfg))
+            except F.FidesError:
+                continue
+            res[cfg] = _time(ctx, lambda: ctx.stage_keyswitch(level, x, kb, ka), reps)
+        F.tune_force(kind, None)
+        best = min(res, key=res.get)
+        if res[best] * (1 + margin) >= res[rule]:
+            best = rule
+        mf = f", matrix cores {res[(1, 1)]:8.2f} us" if (1, 1) in res else ""
+        log(f"  {name:7s} {size} conversions (level {level}): best {best} {res[best]:8.2f} us, "
+            f"rules tg {rule[0]} {res[rule]:8.2f} us{mf}")
+        if best != rule:
+            rows.append((kind, size, list(best), res[best], rule, res[rule]))
+
+    groups = {1, 2, 3, 4, 6, 8, 12, 16}
     # ModUp: one job, nd digit conversions at the highest level with nd digits
     for nd in range(1, dnum + 1):
         level = min(L, nd * alpha - 1)
-        if -(-(level + 1) // alpha) != nd:
-            continue
-        x = ctx.device_array((level + 1, N), np.stack([rng.integers(0, mods[i], N, dtype=np.uint64)
-                                                        for i in range(level + 1)]))
-        ext = ctx.device_array((nd, level + 1 + K, N))
-        targets = L + 1 + K - alpha
-        F.tune_force(F.TUNE_MODUP, None)
-        rule, _ = ctx.tune_config(F.TUNE_MODUP, nd)
-        # (target groups, 0) on the VALU, and (1, 1) the int8 matrix-core conversion
-        res = {}
-        for cfg in [(tg, 0) for tg in sorted({1, 2, 3, 4, 6, 8, 12, 16} & set(range(1, targets + 1)))] + [(1, 1)]:
-            try:
-                F.tune_force(F.TUNE_MODUP, list(cfg))
-            except F.FidesError:
-                continue
-            res[cfg] = _time(ctx, lambda: ctx.stage_modup(level, x, ext), reps)
-        F.tune_force(F.TUNE_MODUP, None)
-        best = min(res, key=res.get)
-        rk = (rule[0], 0)
-        t_rule = res.get(rk, float("nan"))
-        if rk in res and res[best] * (1 + margin) >= t_rule:
-            best = rk
-        mf = res.get((1, 1), float("nan"))
-        log(f"  modup  {nd} conversions (level {level}): best {best} {res[best]:8.2f} us, "
-            f"rules tg {rule[0]} {t_rule:8.2f} us, matrix cores {mf:8.2f} us")
-        rows.append((F.TUNE_MODUP, nd, list(best), res[best], rule, t_rule))
+        if -(-(level + 1) // alpha) == nd:
+            pick(F.TUNE_MODUP, "modup", nd, level, [(tg, 0) for tg in groups if tg <= L + 1 + K - alpha] + [(1, 1)])
     # ModDown: the two conversions of a key switch at the top level
-    x = ctx.device_array((L + 1, N), np.stack([rng.integers(0, mods[i], N, dtype=np.uint64) for i in range(L + 1)]))
-    kb, ka = ctx.device_array((L + 1, N)), ctx.device_array((L + 1, N))
-    F.tune_force(F.TUNE_MODDOWN, None)
-    rule, _ = ctx.tune_config(F.TUNE_MODDOWN, 2)
-    res = {}
-    for tg in sorted({1, 2, 3, 4, 6, 8, 12, 16} & set(range(1, L + 2))):
-        F.tune_force(F.TUNE_MODDOWN, [tg])
-        res[tg] = _time(ctx, lambda: ctx.stage_keyswitch(L, x, kb, ka), reps)
-    F.tune_force(F.TUNE_MODDOWN, None)
-    best = min(res, key=res.get)
-    if rule[0] in res and res[best] * (1 + margin) >= res[rule[0]]:
-        best = rule[0]
-    log(f"  moddown 2 conversions (level {L}): best tg {best} {res[best]:8.2f} us, "
-        f"rules tg {rule[0]} {res.get(rule[0], float('nan')):8.2f} us")
-    rows.append((F.TUNE_MODDOWN, 2, [best, 0], res[best], rule, res.get(rule[0], float("nan"))))
+    pick(F.TUNE_MODDOWN, "moddown", 2, L, [(tg, 0) for tg in groups if tg <= L + 1])
     return rows
 
 
@@ -212,10 +200,8 @@ def main(argv=None):
             conv_sizes.setdefault(kind, []).append((size, best, t, tr))
         for kind, lst in conv_sizes.items():
             lst.sort()
-            for i, (size, best, t, tr) in enumerate(lst):
-                lo = 1 if i == 0 else lst[i - 1][0] + 1
-                hi = size if i + 1 < len(lst) else size
-                lines.append(f"{names[kind]} {logN} {lo} {hi} {best[0]} {best[1]} 0 0   # {size} conversions: "
+            for size, best, t, tr in lst:
+                lines.append(f"{names[kind]} {logN} {size} {size} {best[0]} {best[1]} 0 0   # {size} conversions: "
                              f"{t:.2f} / {tr:.2f}")
         ctx.close()
     with open(args.out, "w") as f:
