@@ -134,7 +134,10 @@ struct Cheb {
     }
     // sum_(j<n) cf[j] T_j at scales S (n <= m + 1; T_m taken from the baby steps)
     CtVec base(const std::vector<double>& cf, const Scales& S) {
-        if (next < leaves.size() && leaves[next].S == S && leaves[next].cf == cf) return std::move(leaves[next++].sum);
+        if (next < leaves.size() && leaves[next].S == S && leaves[next].cf == cf) {
+            if (leaves[next].sum.empty()) fill(next, std::min(leaves.size(), next + HELD / B));
+            return std::move(leaves[next++].sum);
+        }
         const int lo = base_level(cf) + 1;
         CtVec acc = fresh();
         for (int b = 0; b < B; ++b) {
@@ -193,21 +196,23 @@ struct Cheb {
         plan(r, t - 1, out);
         return out;
     }
-    // All of them together, those at one level in one pass over the T_j, where
-    // there are enough to gain and few enough to hold at once (they are at most as
-    // many as the T_j): at N = 2^16 those of a degree-119 series over two ciphertexts
-    // took 955 us one by one and take 264 together.
-    static constexpr size_t LEAVES = 16;
-    void fill(const std::vector<double>& cf, int t, const Scales& S) {
+    // Several of them together, those at one level in one pass over the T_j, where
+    // there are enough to gain: at N = 2^16 those of a degree-119 series over two
+    // ciphertexts took 955 us one by one and take 264 together.  At most HELD
+    // ciphertexts of sums at once, whatever the batch, and past half of HELD in the
+    // batch one by one: 40 bootstraps together, which held 640 more, took 5798
+    // ciphertexts' memory against 5638 now and with sums one by one (N = 2^10).
+    static constexpr size_t LEAVES = 16, HELD = 256;
+    void plan_sums(const std::vector<double>& cf, int t, const Scales& S) {
+        if (HELD / B < 2) return;
         plan(cf, t, S);
-        if (leaves.size() < 2 || leaves.size() > LEAVES) {
-            leaves.clear();
-            return;
-        }
+        if (leaves.size() < 2 || leaves.size() > LEAVES) leaves.clear();
+    }
+    void fill(size_t from, size_t to) {
         std::map<int, std::vector<Leaf*>> levels;
-        for (Leaf& l : leaves) {
-            l.sum = fresh();
-            levels[base_level(l.cf) + 1].push_back(&l);
+        for (size_t i = from; i < to; ++i) {
+            leaves[i].sum = fresh();
+            levels[base_level(leaves[i].cf) + 1].push_back(&leaves[i]);
         }
         std::vector<Ciphertext*> all;
         for (const auto& [lo, ls] : levels) {
@@ -235,8 +240,8 @@ struct Cheb {
             }
         }
         rescale_batch(c, all);
-        for (Leaf& l : leaves)
-            if (!l.cf.empty()) add_const_batch(c, ptrs(l.sum), l.cf[0]);
+        for (size_t i = from; i < to; ++i)
+            if (!leaves[i].cf.empty()) add_const_batch(c, ptrs(leaves[i].sum), leaves[i].cf[0]);
     }
     // sum_j cf[j] T_j at scales S, for cf.size() <= m 2^(t+1)
     CtVec rec(std::vector<double> cf, int t, const Scales& S) {
@@ -325,7 +330,7 @@ void eval_chebyshev_series_batch(Context& c, const std::vector<const Ciphertext*
     const int lout = S.rec_level(cf, tmax);
     if (lout < 0) throw Error(E_LEVEL, "not enough levels for the Chebyshev series");
     const double s_out = c.scaling_factor_real.empty() ? S.T[1][0]->noise : c.scaling_factor_real[lout];
-    S.fill(cf, tmax, Scales(B, s_out));
+    S.plan_sums(cf, tmax, Scales(B, s_out));
     CtVec res = S.rec(cf, tmax, Scales(B, s_out));
     for (int i = 0; i < B; ++i) {
         if (res[i]->level != lout) throw Error(E_STATE, "Chebyshev: level plan and evaluation disagree");
