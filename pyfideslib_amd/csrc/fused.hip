@@ -332,7 +332,7 @@ hipError_t launch_tensor_rows(const DevTables& T, const TensorJobs& L, int max_n
 template <int LOGN, int A>
 static void modup_cols(const DevTables& T, const ModUpJobs& L, int max_nd, int targets, hipStream_t s) {
     using G = ConvCols<LOGN>;
-    const int tg = conv_launch_groups(TUNE_MODUP, LOGN, max_nd * L.n, (size_t)G::TPL * max_nd * L.n, targets, G::TB);
+    const int tg = conv_launch_groups(TUNE_MODUP, LOGN, max_nd * L.n, (size_t)G::TPL * max_nd * L.n, targets, G::TB, A);
     const size_t items = (size_t)L.n * max_nd * tg * G::TPL;
     const XcdGrid x = conv_grid(items, G::TPL);
     const ConvGrid g{(uint32_t)items, x.chunk, FastDiv(tg, items), FastDiv(max_nd, items)};
@@ -373,7 +373,8 @@ int fused_conv_tg(const DevTables& T, int kind, int convs) {
     int tg = 0;
     (void)by_logn(T.logN, [&](auto ln) {
         using G = ConvCols<decltype(ln)::value>;
-        tg = conv_launch_groups(kind, T.logN, convs, (size_t)G::TPL * convs, targets, G::TB);
+        const int sources = kind == TUNE_MODUP ? conv_bound(T.alpha) : conv_bound(T.K) + 1;  // of a product
+        tg = conv_launch_groups(kind, T.logN, convs, (size_t)G::TPL * convs, targets, G::TB, sources);
     });
     return tg;
 }

@@ -207,19 +207,29 @@ struct ConvGrid {
 inline XcdGrid conv_grid(size_t items, int per) {
     return items <= (size_t)32 * per ? xcd_chunks(items, XCD_TILES) : xcd_grid(items, per);
 }
+// Blocks of a conversion's launch.  Where each group runs the sources' column
+// pass again, groups past one round of what is resident cost more than they
+// give: two blocks a CU, one where the sources' tiles take more than half of its
+// LDS.  Against 1024 blocks, N = 2^13, 59-bit limbs (separate kernels in brackets): 10 special
+// primes, 5 hoisted rotations 96 -> 87 us (87), 8 products 162 -> 143 (156); 11 special primes
+// 105 -> 93 (90) and 192 -> 156 (167).
+constexpr size_t conv_most_blocks(int logN, int sources) {
+    const size_t n1 = (size_t)1 << ((logN + 1) / 2), bytes = sources * (4 * (n1 + n1 / 16 + 1) * 8 + n1 * 16);
+    return logN > CONV_INV_LOGN ? 1024 : bytes > (80 << 10) ? 256 : 512;
+}
 // Target groups, of whole rounds of tb targets: up to 1024 blocks in all, two
 // rounds of what is resident (ModUp at N = 2^16, level 24: 40.3 us with 768 blocks, 45 with
 // 384, 47 with 1536; ModDown 28.4 with 768, 27.5 with 512, 33 with 256 or 1024).
 // Where whole rounds leave less than half of the CUs with a block, single targets up
 // to 192 blocks: a thread then forms one sum instead of TPT in turn (N = 2^13, 4
 // limbs: ModDown 9.2 -> 8.2 us, ModUp 8.2 -> 7.4; at 128 blocks, N = 2^14, no gain).
-inline int fused_groups(size_t base_blocks, int targets, int tb) {
+inline int fused_groups(size_t base_blocks, int targets, int tb, size_t most = 1024) {
     const int rounds = (targets + tb - 1) / tb;
     if (base_blocks && base_blocks * rounds < 128) {
         const int g = (int)(192 / base_blocks);
         return g < 1 ? 1 : g < targets ? g : targets;
     }
-    size_t g = (size_t)1024 / (base_blocks ? base_blocks : 1);
+    size_t g = most / (base_blocks ? base_blocks : 1);
     if (g < 1) g = 1;
     if (g > (size_t)rounds) g = rounds;
     const size_t each = (rounds + g - 1) / g;  // rounds per group, evened out
@@ -227,9 +237,9 @@ inline int fused_groups(size_t base_blocks, int targets, int tb) {
 }
 
 // The groups of a launch of `convs` conversions.
-inline int conv_launch_groups(int kind, int logN, int convs, size_t base_blocks, int targets, int tb) {
+inline int conv_launch_groups(int kind, int logN, int convs, size_t base_blocks, int targets, int tb, int sources) {
     const int tg = conv_set_tg(kind, logN, convs, targets);
-    return tg ? tg : fused_groups(base_blocks, targets, tb);
+    return tg ? tg : fused_groups(base_blocks, targets, tb, conv_most_blocks(logN, sources));
 }
 
 // The exact sum over the A sources of x_i m_i (m: one matrix row, scalar

@@ -144,7 +144,8 @@ __global__ void __launch_bounds__(512, 4) k_moddown_cols(DevTables T, ModDownJob
 template <int LOGN, int KK>
 static void moddown_cols(const DevTables& T, const ModDownJobs& L, int targets, bool rescale, hipStream_t s) {
     using G = ConvCols<LOGN>;
-    const int tg = conv_launch_groups(TUNE_MODDOWN, LOGN, L.n, (size_t)G::TPL * L.n, targets, G::TB);
+    const int tg = conv_launch_groups(TUNE_MODDOWN, LOGN, L.n, (size_t)G::TPL * L.n, targets, G::TB,
+                                      KK + rescale);
     const size_t items = (size_t)L.n * tg * G::TPL;
     const XcdGrid x = conv_grid(items, G::TPL);
     const ConvGrid g{(uint32_t)items, x.chunk, FastDiv(tg, items), FastDiv(1, items)};

@@ -81,3 +81,19 @@ def test_rule_reported_for_a_key_switch():
     finally:
         F.tune_force(-1)
         ctx.close()
+
+
+# special primes: tiles of 10 + 1 sources leave room for two blocks a CU, of 12 + 1 for one
+@pytest.mark.parametrize("K,hoisted,product", [(10, 3, 5), (11, 1, 5)])
+def test_groups_that_repeat_their_sources(K, hoisted, product):
+    """Rings whose conversions run their sources' column pass: no more groups than one round of blocks."""
+    import pyfideslib_amd as F
+
+    P = O.make_params(13, 60, 59, 17, 59, 2, K=K)
+    raw = F.RawParams.from_lists(P.logN, P.L, P.K, P.dnum, P.moduli, P.roots)
+    ctx = F.Context(raw)
+    # 16 tiles a conversion, 18 targets in rounds of 4
+    assert ctx.fused
+    assert ctx.tune_config(F.TUNE_MODDOWN, 10)[0][0] == hoisted  # 5 rotations
+    assert ctx.tune_config(F.TUNE_MODDOWN, 2)[0][0] == product
+    ctx.close()
