@@ -426,8 +426,9 @@ hipError_t launch_moddown_conv(const DevTables& T, const ModDownJobs& jobs, int 
 hipError_t launch_moddown_conv_mode(const DevTables& T, const ModDownJobs& jobs, bool rescale, hipStream_t stream);
 
 // ---- the fused key switch (fused.hip, fused_down.hip) ----
-// Whether these parameters take it: rings of 2^12 .. 2^16, at most 4 digits of
-// at most 10 primes, at most 10 special primes, sums within one reduction.
+// Whether these parameters take it: rings of 2^12 .. 2^16, at most FUSED_DIGITS
+// digits of at most FUSED_CONV_MAX primes, at most fused_down_max special primes, and
+// conversion sums within one reduction (modup_one_reduce, moddown_one_reduce).
 bool fused_ok(const DevTables& T);
 // Whether the conversion kernels take their sources after the first pass of the
 // inverse transform only (small rings), and run the second themselves.

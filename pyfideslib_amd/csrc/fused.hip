@@ -312,7 +312,7 @@ __global__ void __launch_bounds__(FRows<LOGN>::NTR, 4) k_rows_ksk(DevTables T, K
 // ---------------------------------------------------------- launchers ----
 bool fused_ok(const DevTables& T) {
     return T.logN >= FUSED_LOGN_MIN && T.logN <= FUSED_LOGN_MAX && T.dnum <= FUSED_DIGITS &&
-           T.alpha <= FUSED_CONV_MAX && T.K <= FUSED_CONV_MAX && T.modup_one_reduce && T.moddown_one_reduce;
+           T.alpha <= FUSED_CONV_MAX && T.K <= fused_down_max(T.logN) && T.modup_one_reduce && T.moddown_one_reduce;
 }
 
 bool fused_inv_cols(const DevTables& T) { return fused_ok(T) && T.logN <= CONV_INV_LOGN; }

@@ -6,10 +6,17 @@
 namespace fides {
 
 constexpr int FUSED_LOGN_MIN = 12, FUSED_LOGN_MAX = 16;
-// Source limbs of a conversion (11 as 12, conv_bound).  At 12 the ModDown with a rescale
-// spills 38 registers and is still ahead of the separate kernels (8 products, N = 2^15, 14
-// limbs of 59 bits, 11 special primes: 365 -> 353 us); past it sources would not fit.
+// Source limbs of a conversion (11 as 12, conv_bound), where their sums fit one
+// reduction (fused_ok): with 60-bit special primes that holds up to 8, with shorter ones
+// up to 12.  At 12 the ModDown with a rescale spills 38 registers and is still ahead of
+// the separate kernels: 20 limbs and 11 special primes of 59 bits, separate -> fused, N = 2^16
+// a product 182 -> 182 us, a rotation 155 -> 150, at half the limbs 114 -> 111 and 97 -> 94;
+// N = 2^15 116 -> 110, 99 -> 92, 83 -> 78, 72 -> 66.  Past it sources would not fit.
+// At N = 2^14 a ModDown from more than 9 primes repeats their column pass (conv_inv) at a
+// cost that hoisted sets and large batches do not win back: 10 primes, 5 rotations 127 -> 138 us;
+// 11, 32 products 896 -> 974.
 constexpr int FUSED_CONV_MAX = 12;
+constexpr int fused_down_max(int logN) { return logN == 14 ? 9 : FUSED_CONV_MAX; }
 constexpr int FUSED_DIGITS = 4;
 constexpr int CONV_INV_LOGN = 14;
 

@@ -149,10 +149,12 @@ static void moddown_cols(const DevTables& T, const ModDownJobs& L, int targets, 
     const size_t items = (size_t)L.n * tg * G::TPL;
     const XcdGrid x = conv_grid(items, G::TPL);
     const ConvGrid g{(uint32_t)items, x.chunk, FastDiv(tg, items), FastDiv(1, items)};
-    if (rescale)
-        hipLaunchKernelGGL((k_moddown_cols<LOGN, KK, true>), x.grid, dim3(G::NT), 0, s, T, L, g);
-    else
-        hipLaunchKernelGGL((k_moddown_cols<LOGN, KK, false>), x.grid, dim3(G::NT), 0, s, T, L, g);
+    if constexpr (KK <= fused_down_max(LOGN)) {
+        if (rescale)
+            hipLaunchKernelGGL((k_moddown_cols<LOGN, KK, true>), x.grid, dim3(G::NT), 0, s, T, L, g);
+        else
+            hipLaunchKernelGGL((k_moddown_cols<LOGN, KK, false>), x.grid, dim3(G::NT), 0, s, T, L, g);
+    }
 }
 
 template <int LOGN>
