@@ -144,9 +144,9 @@ static std::shared_ptr<BatchPlan> build_plan(Context& c, const std::vector<KsIte
         j.src = x; j.mid = t; j.dst = t; j.npos = nl; j.nq = nl; j.q0 = 0;
         j.level = l; j.scale_sel = ISCALE_MODUP;
         iu.push_back(j);
-        if (!it.mult) ir.push_back(j);
+        if (!it.mult && P->fused) ir.push_back(j);
         mu.push_back(ModUpJob{t, ext, l});
-        for (int d = 0; d < nd; ++d) {
+        for (int d = 0; d < nd && !P->fused; ++d) {  // the fused kernels run these passes themselves
             NttJob e{};
             uint64_t* ed = ext + (size_t)d * npos * N;
             e.src = ed; e.mid = ed; e.dst = ed; e.npos = npos; e.nq = nl; e.q0 = 0;
@@ -212,18 +212,22 @@ static std::shared_ptr<BatchPlan> build_plan(Context& c, const std::vector<KsIte
     }
     P->n_mult = (int)tj.size();
     // KSK jobs grouped by key (each job carries its own pointers, so their
-    // order is free), cut into chunks of one key for the key-stationary form
+    // order is free); for the separate kernels cut into chunks of one key, for the
+    // key-stationary form
     std::stable_sort(kj.begin(), kj.end(), [](const KskJob& x, const KskJob& y) { return x.ka < y.ka; });
-    std::vector<int> chunks{0};
-    int nkeys = 0;
-    for (int j = 0; j < (int)kj.size(); ++j) {
-        const bool new_key = j == 0 || kj[j].ka != kj[j - 1].ka;
-        nkeys += new_key ? 1 : 0;
-        if (j > 0 && (new_key || j - chunks.back() == ksk_keystat_chunk())) chunks.push_back(j);
+    std::vector<int> chunks;
+    if (!P->fused) {
+        chunks.push_back(0);
+        int nkeys = 0;
+        for (int j = 0; j < (int)kj.size(); ++j) {
+            const bool new_key = j == 0 || kj[j].ka != kj[j - 1].ka;
+            nkeys += new_key ? 1 : 0;
+            if (j > 0 && (new_key || j - chunks.back() == ksk_keystat_chunk())) chunks.push_back(j);
+        }
+        chunks.push_back((int)kj.size());
+        P->n_ksk_chunks = (int)chunks.size() - 1;
+        P->keystat = !kj.empty() && 2 * nkeys <= (int)kj.size();
     }
-    chunks.push_back((int)kj.size());
-    P->n_ksk_chunks = (int)chunks.size() - 1;
-    P->keystat = !kj.empty() && 2 * nkeys <= (int)kj.size();
     int tot;
     std::vector<int> m_iu = limbmap_of(iu, tot); P->intt_up.limbs = tot;
     std::vector<int> m_ir = limbmap_of(ir, tot); P->intt_rot.limbs = tot;

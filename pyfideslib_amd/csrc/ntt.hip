@@ -259,10 +259,10 @@ __global__ void k_fp_twiddles(DevTables T, const ShoupConst* tw, double* out) {
 // ---------------------------------------------------------- launchers ----
 
 // Launch configuration of a transform: column tile width, log2 values per
-// column thread, row tile height (the fourth entry of a tuning configuration
-// capped the grid of a looping form and has no effect).
+// column thread, row tile height (the fourth entry of a tuning configuration is
+// read and has no effect).
 struct NttPick {
-    int cc, lrc, rr, pb;
+    int cc, lrc, rr;
 };
 // Fixed rules (measured on MI355X at N=2^16 over 2..25 limbs): column tiles
 // are 16 wide (128-byte row segments; 4-wide tiles lose more to partial lines
@@ -286,7 +286,6 @@ static NttPick rule_pick(int logN, int limbs) {
     p.cc = ov_c > 0 ? width(ov_c) : (tiles16 < 64 ? 4 : 16);
     p.rr = ov_r > 0 ? width(ov_r) : 4;
     p.lrc = ov_l > 0 ? (ov_l == 3 ? 3 : 2) : (limbs >= 40 ? 3 : 2);
-    p.pb = 0;
     return p;
 }
 
@@ -294,13 +293,13 @@ static NttPick rule_pick(int logN, int limbs) {
 // the fixed rules.
 static NttPick ntt_pick(bool forward, int logN, int limbs) {
     TuneCfg c;
-    if (tune_get(forward ? TUNE_NTT_FWD : TUNE_NTT_INV, logN, limbs, c)) return NttPick{c.v[0], c.v[1], c.v[2], c.v[3]};
+    if (tune_get(forward ? TUNE_NTT_FWD : TUNE_NTT_INV, logN, limbs, c)) return NttPick{c.v[0], c.v[1], c.v[2]};
     return rule_pick(logN, limbs);
 }
 
 TuneCfg ntt_rule_cfg(bool, int logN, int limbs) {
     const NttPick p = rule_pick(logN, limbs);
-    return TuneCfg{{p.cc, p.lrc, p.rr, p.pb}};
+    return TuneCfg{{p.cc, p.lrc, p.rr, 0}};
 }
 
 template <int LOGN, int W, int LRC>

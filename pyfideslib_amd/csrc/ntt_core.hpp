@@ -60,7 +60,7 @@ struct IntArith {
     // the residue of a forward output in [0, 16p), of an inverse one in [0, 4p)
     __device__ __forceinline__ uint64_t canon_fwd(V x) const { return csub(term_fwd(x), p); }
     __device__ __forceinline__ uint64_t canon_inv(V x) const { return csub(csub(x, 2 * p), p); }
-    // a b, a b + c d as residues; a value below 3p from reduce128_lazy
+    // a b, a b + c d as residues
     __device__ __forceinline__ uint64_t mul(uint64_t a, uint64_t b, const PrimeInfo& P) const { return mulmod(a, b, P); }
     __device__ __forceinline__ uint64_t mul2(uint64_t a, uint64_t b, uint64_t c, uint64_t d,
                                              const PrimeInfo& P) const {
@@ -69,9 +69,8 @@ struct IntArith {
         mac128(lo, hi, c, d);
         return reduce128(lo, hi, P);
     }
-    __device__ __forceinline__ V from_lazy(uint64_t x) const {
-        return csub(csub(x, 2 * p), p);
-    }
+    // the residue of a value below 3p (reduce128_lazy)
+    __device__ __forceinline__ V from_lazy(uint64_t x) const { return csub(csub(x, 2 * p), p); }
     // a forward output as an inner product's term, in [0, 2p)
     __device__ __forceinline__ V term_fwd(V x) const { return csub(csub(csub(x, 8 * p), 4 * p), 2 * p); }
     // sum of at most 4 products x k with x < 2p, k < p (below 8p^2 < 2^(bits(p) +
@@ -145,7 +144,6 @@ struct FpArith {
     __device__ __forceinline__ uint64_t mul2(uint64_t a, uint64_t b, uint64_t c, uint64_t d, const PrimeInfo&) const {
         return fp_canon(fp_mul(fp_from(a), fp_from(b), p, pinv) + fp_mul(fp_from(c), fp_from(d), p, pinv), p, pinv);
     }
-    __device__ __forceinline__ V from_lazy(uint64_t x) const { return fp_from(x); }  // 3p < 2^52
     __device__ __forceinline__ V term_fwd(V x) const { return fp_reduce(x, p, pinv); }
     // |x| <= p, k < p: each product at most (1/2 + 3/8) p, four of them below 4p
     using Sum = double;
