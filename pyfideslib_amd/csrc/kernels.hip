@@ -1,5 +1,6 @@
 // Elementwise, dot-product and automorphism kernels, and the separate
-// base-conversion and key-switch kernels of the sizes past the fused ones (gfx950).
+// base-conversion and key-switch kernels of the sizes past the fused ones, of the
+// matrix-core ModUp and of the stage entries (gfx950).
 //
 // All are HBM streams over limb-major polynomials: 256-thread blocks along the
 // coefficient axis, the limb (position) along blockIdx.y and the job along

@@ -264,12 +264,14 @@ __global__ void k_fp_twiddles(DevTables T, const ShoupConst* tw, double* out) {
 struct NttPick {
     int cc, lrc, rr;
 };
-// Fixed rules (measured on MI355X at N=2^16 over 2..25 limbs): column tiles
-// are 16 wide (128-byte row segments; 4-wide tiles lose more to partial lines
-// than they gain in parallelism) except for launches of under 64 tiles; row
-// tiles are 4 rows (256 threads), which keeps register-prefetched twiddles at
-// full occupancy; 8 values per column thread (radix-8 phases, one LDS
-// exchange fewer) from 40 limbs up, where it measured 3-15% faster.
+// Fixed rules: column tiles are 16 wide (128-byte row segments) except for
+// launches of under 64 tiles, row tiles 4 rows (256 threads), 8 values per column
+// thread (radix-8 phases, one LDS exchange fewer) from 40 limbs up.  They were
+// measured at N = 2^16 with integer butterflies in every limb.  With the present ones
+// they hold at 1, 2 and 25 limbs, and tiles of 4 or 8 columns are ahead elsewhere: forward
+// (inverse) at 4 limbs 12.8 -> 11.4 us (13.3 -> 11.5), at 8 13.5 -> 12.0 (13.5 -> 12.1), at 74
+// 44.1 -> 41.3 (45.2 -> 42.9).  The table holds that for N = 2^16 and 2^13; the other rings
+// have not been measured again and keep the rules.
 // FIDES_NTT_COLS / FIDES_NTT_ROWS (4, 8 or 16) and FIDES_NTT_LRC (2 or 3)
 // force a value.
 static int env_int(const char* name) {
